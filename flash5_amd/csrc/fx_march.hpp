@@ -8,13 +8,13 @@
 // hy_getRiemannState.F90:356-1327 regrouped by quantity instead of by cell):
 //   stage A  transverse fluxes sigma_x, sigma_y of plane k+1 into 3-plane LDS
 //            rings (they feed the 3-D CTU terms of planes k and k+2) and,
-//            from the same stencils, the limited characteristic slopes
-//            along x and y of plane k+1 into 2-plane rings; sigma_z of
-//            plane k; slopes along z (with the z flattening tilde) of plane
-//            k+1 into 3-plane rings
-//   stage B1 x-, y- and z-face states of plane k: PPM with characteristic
-//            tracing, 2-D CTU transverse corrections, positivity fallback
-//   stage B2 3-D full-CTU corner terms added to those states
+//            from the same stencils, the limited characteristic slopes and
+//            the flattening tildes along x and y of plane k+1 into 2-plane
+//            rings; sigma_z of plane k; slopes along z (with the z
+//            flattening tilde) of plane k+1 into 3-plane rings
+//   stage B  x-, y- and z-face states of plane k: PPM with characteristic
+//            tracing, 2-D CTU transverse corrections, 3-D full-CTU corner
+//            terms, positivity fallback after either
 //   stage C  x-, y- and z-face fluxes (HLLC, HLL or the hybrid switch, and
 //            the aux internal-energy fluxes, hy_getFaceFlux.F90) to the
 //            tile's flux arrays and the
@@ -58,12 +58,15 @@ template <int NDIM, int TX, int TY> struct MarchLds {
   static constexpr int LX = SZ + (Z ? 6 * I::NC : 1);         // slopes along x, ring
   static constexpr int LY = LX + NRL * 6 * I::NLX;            // slopes along y, ring
   static constexpr int LZ = LY + NRL * 6 * I::NLY;            // slopes along z, ring
-  static constexpr int FZ = LZ + (Z ? 3 * 6 * NCOL : 1);      // flattening tilde along z, ring
-  static constexpr int WX = FZ + (Z ? 3 * NCOL : 1);          // x-face states (Wp, Wn)
-  static constexpr int WY = WX + 12 * I::NRY;                 // y-face states
-  static constexpr int WZ = WY + 12 * I::NRX;                 // z-face states of plane k
-  static constexpr int WZP = WZ + (Z ? 12 * NCOL : 1);        // z-face Wp of plane k-1
-  static constexpr int CST = WZP + (Z ? 6 * NCOL : 1);        // the step's ratios, widths (FP32)
+  static constexpr int FX = LZ + (Z ? 3 * 6 * NCOL : 1);      // flattening tilde along x, ring
+  static constexpr int FY = FX + NRL * I::NLX;                // flattening tilde along y, ring
+  static constexpr int FZ = FY + NRL * I::NLY;                // flattening tilde along z, ring
+  static constexpr int WX = FZ + (Z ? 3 * NCOL : 1);          // x state cells' Wp
+  static constexpr int WY = WX + 6 * I::NRY;                  // y state cells' Wp
+  static constexpr int WZ = WY + 6 * I::NRX;                  // z state cells' Wp of the last plane done
+  static constexpr int PY = WZ + (Z ? 6 * NCOL : 1);          // Wn + Wp pressures of the y state cells
+  static constexpr int PZ = PY + I::NRX;                      // and of the z state cells
+  static constexpr int CST = PZ + (Z ? NCOL : 1);             // the step's ratios, widths (FP32)
   static constexpr int total = CST + 12;
 };
 
@@ -106,26 +109,6 @@ __device__ __forceinline__ void write_face_states(const DevParams& P, R* base, l
     base[q * nf + r] = VL[comp_slot(q)];
     base[(6 + q) * nf + r] = VR[comp_slot(q)];
   }
-}
-
-template <int SD, typename R>
-__device__ __forceinline__ bool sigma_cell(const DevParams& P, const gdouble* __restrict__ U, long c,
-                                           R sig[8]) {
-  return sigma_at<SD>(P, U, c, sig, nullptr);
-}
-
-template <int DIR, typename R>
-__device__ __forceinline__ bool slope_cell(const DevParams& P, const gdouble* __restrict__ U, long c,
-                                           R db[8]) {
-  const long s = axis_stride(P, DIR);
-  R Vm[8], Vc[8], Vp[8];
-  load_prim(P, U, c - s, Vm);
-  load_prim(P, U, c, Vc);
-  load_prim(P, U, c + s, Vp);
-  EigT<R> e;
-  if (!eig_make<DIR>(Vc, e)) return false;
-  tvd_slope<DIR>(P, Vm, Vc, Vp, e, db);
-  return true;
 }
 
 template <typename R>
@@ -181,33 +164,6 @@ __device__ __forceinline__ bool nonpositive(const R* Wp, const R* Wn) {
 template <typename R>
 __device__ __forceinline__ bool negative(const R* Wp, const R* Wn) {
   return Wn[P_DENS] < R(0.) || Wp[P_DENS] < R(0.) || Wn[P_PRES] < R(0.) || Wp[P_PRES] < R(0.);
-}
-
-// store/load a face-state pair (Wp, Wn) of 6 components each
-template <typename R>
-__device__ __forceinline__ void put_state(R* base, int n, int idx, const R Wp[8], const R Wn[8]) {
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    base[q * n + idx] = Wp[comp_slot(q)];
-    base[(6 + q) * n + idx] = Wn[comp_slot(q)];
-  }
-}
-
-template <int D>
-__device__ __forceinline__ void write_flux(const DevParams& P, gdouble* Fo, long r, const double F[8]) {
-  const long nf = P.nface[D];
-#pragma unroll
-  for (int q = 0; q < FX_NFLUX; ++q) Fo[q * nf + r] = F[q];
-}
-
-template <typename R>
-__device__ __forceinline__ void get_state(const R* base, int n, int idx, R Wp[8], R Wn[8]) {
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    Wp[comp_slot(q)] = base[q * n + idx];
-    Wn[comp_slot(q)] = base[(6 + q) * n + idx];
-  }
-  Wp[P_GAMC] = Wp[P_GAME] = Wn[P_GAMC] = Wn[P_GAME] = R(0.);
 }
 
 template <typename R>
@@ -283,13 +239,9 @@ __device__ __forceinline__ double tv_ld(const TileView& tv, unsigned ob, unsigne
 // A stage's item number.  With OPAQUE it passes through an empty asm
 // statement, which the compiler cannot see through: the index arithmetic of
 // each stage's items (item kind, column, cell offsets) is then redone per
-// plane instead of being hoisted out of the plane loop and kept live.  That
-// took the FP32 16x8 march from 160 registers (128 with 21 spilled at 4 waves
-// per SIMD) to 104, and 4096 x 16^3 from 5.95 to 4.81 ms (HLLC) and 6.82 to
-// 5.97 ms (exact-solver face states); the FP64 multi-class kernels from 256
-// registers with 51 spilled to 195.  The single-class FP64 march, which LDS
-// holds at 2 waves per SIMD whatever its registers, keeps the hoisted form
-// (1 % faster).
+// plane instead of being hoisted out of the plane loop and kept live.  With
+// the hoisted form the FP32 16x8 march took 160 registers instead of 104 and
+// the FP64 multi-class kernels 256 with 51 spilled instead of 195.
 template <bool OPAQUE>
 __device__ __forceinline__ int item_index(int w) {
   if constexpr (OPAQUE) asm volatile("" : "+v"(w));
@@ -322,37 +274,6 @@ __device__ __forceinline__ bool tv_sigma(const DevParams& P, const TileView& tv,
   return true;
 }
 
-template <int DIR, typename R>
-__device__ __forceinline__ bool tv_slope(const DevParams& P, const TileView& tv, unsigned cb,
-                                         unsigned sb, R db[8]) {
-  R Vm[8], Vc[8], Vp[8];
-  tv_prim(tv, cb - sb, Vm);
-  tv_prim(tv, cb, Vc);
-  tv_prim(tv, cb + sb, Vp);
-  EigT<R> e;
-  if (!eig_make<DIR>(Vc, e)) return false;
-  tvd_slope<DIR>(P, Vm, Vc, Vp, e, db);
-  return true;
-}
-
-// FlatTilde and FlatCoeff along DIR (hy_getRiemannState.F90:365-453)
-template <int DIR, typename R>
-__device__ __forceinline__ R tv_flat_tilde(const TileView& tv, unsigned cb, unsigned sb) {
-  const unsigned pr = tv.ob[P_PRES], vn = tv.ob[P_VELX + DIR];
-  return flat_tilde_vals(R(tv_ld(tv, pr, cb - 2 * sb)), R(tv_ld(tv, pr, cb - sb)),
-                         R(tv_ld(tv, pr, cb + sb)), R(tv_ld(tv, pr, cb + 2 * sb)),
-                         R(tv_ld(tv, vn, cb - sb)), R(tv_ld(tv, vn, cb + sb)));
-}
-template <int DIR, typename R>
-__device__ __forceinline__ R tv_flat_coeff(const TileView& tv, unsigned cb, unsigned sb) {
-  const unsigned pr = tv.ob[P_PRES];
-  const R dp1 = (R(tv_ld(tv, pr, cb + sb)) - R(tv_ld(tv, pr, cb - sb)));
-  const R f0 = tv_flat_tilde<DIR, R>(tv, cb, sb);
-  if (dp1 < R(0.0)) return fmax(f0, tv_flat_tilde<DIR, R>(tv, cb + sb, sb));
-  if (dp1 == R(0.)) return f0;
-  return fmax(f0, tv_flat_tilde<DIR, R>(tv, cb - sb, sb));
-}
-
 // Whether the face between the cells at cbl and cbr takes HLL (HLL, or the
 // hybrid switch with a flagged cell on either side, hy_getFaceFlux.F90:353-367)
 template <int RS>
@@ -382,10 +303,26 @@ __device__ __forceinline__ void write_flux_b(const DevParams& P, gdouble* Fo, un
 // barrier, so a workgroup may call it again for another column tile.  fsb:
 // tile t's face-state scratch (RS_STATES).
 //
-// Work items are laid out over fixed extents so that item numbers split by
-// compile-time divisors: x-face states over a in [-1, TX], x faces over
-// a in [0, TX] (y likewise); the high row (a = TX) is skipped unless the
-// tile sits at the block's high side, where it owns that row.
+// Two barriers per plane.  Between them run
+//   stage B(k)          one state cell per thread (x, y and z state cells in
+//                       wave-aligned roles): PPM, the 2-D and the 3-D CTU
+//                       corrections.  The high-side state Wp goes to LDS for
+//                       the next face up; the low-side state Wn stays in the
+//                       thread's registers.
+//   stage C(k), A(k+1)  the thread's own face (x, y or z) between its
+//                       neighbour's Wp and its own Wn, then the stage-A items
+//                       of the next plane.  C(k) reads only face states and
+//                       A(k+1) writes only sigmas, slopes and tildes that
+//                       B(k) has done with, so no barrier is needed between.
+// Everything a state cell needs (its stencil, its eigen system, its two face
+// states) is formed once in one thread; the waves that have no face start
+// the next plane's stage A meanwhile.  The loads of a stage start right
+// after its barrier, so fewer barriers are fewer times that all waves wait
+// for the cache together.  Against the form with four barriers (face states,
+// CTU and fluxes as stages of their own over LDS arrays of both states,
+// tildes formed by the state cells) the step of 4096 x 16^3 went from 10.17
+// to 8.89 ms (FP64 HLLC), of 2048 x 16^3 from 3.41 to 3.07 ms (mixed) and of
+// 1024 x 16^3 from 3.52 to 3.15 ms (FP64 exact).
 template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE = (sizeof(R) == 4)>
 __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch& L, int t, int ox,
                                            int oy, R* fsb, ExactStats& es,
@@ -401,11 +338,14 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   R* const LX = smem + M::LX;
   R* const LY = smem + M::LY;
   R* const LZ = smem + M::LZ;
+  R* const FX = smem + M::FX;
+  R* const FY = smem + M::FY;
   R* const FZ = smem + M::FZ;
   R* const WX = smem + M::WX;
   R* const WY = smem + M::WY;
   R* const WZ = smem + M::WZ;
-  R* const WZP = smem + M::WZP;
+  R* const PY = smem + M::PY;
+  R* const PZ = smem + M::PZ;
 
   const int tid = threadIdx.x;
   // A tile owns its high x (y) face row only at the block's high side;
@@ -424,11 +364,8 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   // The step's ratios of dt and the cell widths, and the widths, uniform
   // over the tile.  The FP64 march keeps them in registers (the compiler
   // hoists them); the FP32 march reads them from LDS, written once per
-  // column tile by one thread (stage B1 first reads them after stage A's
-  // barrier, and the previous column tile ended on a barrier): 12 fewer live
-  // registers, mixed-mode march 6.29 -> 6.08 ms (HLLC) and 7.85 -> 7.08 ms
-  // (exact-solver face states) on 4096 x 16^3 at 4 waves per SIMD, bit for
-  // bit the same.
+  // column tile by one thread (stage B first reads them after a barrier, and
+  // the previous column tile ended on one): 12 fewer live registers.
   const R rat[12] = {R(dt / dx), R(dt / dy), R(dt / dz),
                      R(0.5 * dt / dx), R(0.5 * dt / dy), R(0.5 * dt / dz),
                      R(dt * dt / (6. * dy * dz)), R(dt * dt / (6. * dz * dx)),
@@ -461,8 +398,11 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   };
   // stage-A items along x (w < NUX) and y (w < NUY) at plane p: one cell's
   // three-cell stencil and eigen system serve its sigma (sig: p is a plane
-  // the sigma ring takes, and the cell lies in R_x / R_y) and its limited
-  // slope (sl: p is interior, and the cell lies in the slope rows)
+  // the sigma ring takes, and the cell lies in R_x / R_y), its limited slope
+  // and its flattening tilde (sl: p is interior, and the cell lies in the
+  // slope rows).  Each tilde is formed here once: formed by the state cells,
+  // a state cell's coefficient took three (its own, and one of each
+  // neighbour's in diverged branches) and five more loads.
   auto x_item = [&](int w, int p, bool sig, bool sl) {
     int a, b;
     if (w < TX) {
@@ -495,6 +435,10 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
       R db[8];
       tvd_slope<0>(P, Vm, Vc, Vp, e, db);
       lds_put6(LX + ringL(p) * 6 * I::NLX, I::NLX, I::lx(a, b), db);
+      if (P.flat)
+        FX[ringL(p) * I::NLX + I::lx(a, b)] =
+            flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * sxb)), Vm[P_PRES], Vp[P_PRES],
+                            R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * sxb)), Vm[P_VELX], Vp[P_VELX]);
     }
   };
   auto y_item = [&](int w, int p, bool sig, bool sl) {
@@ -530,20 +474,78 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
       R db[8];
       tvd_slope<1>(P, Vm, Vc, Vp, e, db);
       lds_put6(LY + ringL(p) * 6 * I::NLY, I::NLY, I::ly(a, b), db);
+      if (P.flat)
+        FY[ringL(p) * I::NLY + I::ly(a, b)] =
+            flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * syb)), Vm[P_PRES], Vp[P_PRES],
+                            R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * syb)), Vm[P_VELY], Vp[P_VELY]);
     }
   };
   // stage-A item: z-slope and z flattening tilde of column w at plane m
   auto zslope_item = [&](int w, int m) {
     const int a = w % TX, b = w / TX;
     const unsigned cb = cell_b(P, ox + a, oy + b, m);
-    R db[8];
-    if (!tv_slope<2>(P, tv, cb, szb, db)) { bad = true; return; }
+    R db[8], Vm[8], Vc[8], Vp[8];
+    tv_prim(tv, cb - szb, Vm);
+    tv_prim(tv, cb, Vc);
+    tv_prim(tv, cb + szb, Vp);
+    EigT<R> e;
+    if (!eig_make<2>(Vc, e)) { bad = true; return; }
+    tvd_slope<2>(P, Vm, Vc, Vp, e, db);
     lds_put6(LZ + ring(m) * 6 * NCOL, NCOL, w, db);
-    FZ[ring(m) * NCOL + w] = tv_flat_tilde<2, R>(tv, cb, szb);
+    if (P.flat)
+      FZ[ring(m) * NCOL + w] =
+          flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * szb)), Vm[P_PRES], Vp[P_PRES],
+                          R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * szb)), Vm[P_VELZ], Vp[P_VELZ]);
+  };
+  // FlatCoeff of the cell whose pressures across are pm, pp, from its own
+  // tilde and its neighbours' (hy_getRiemannState.F90:408-453)
+  auto flat_of = [&](R pm, R pp, R fm, R f0, R fp) -> R {
+    const R dp1 = pp - pm;
+    return dp1 < R(0.0) ? fmax(f0, fp) : (dp1 == R(0.) ? f0 : fmax(f0, fm));
   };
 
   const int kBeg = Z ? klo - 1 : 0;
   const int kEnd = Z ? khi + 1 : 0;
+  // ------------------------------ stage A ------------------------------
+  // For plane k: sigma_x/y of plane k+1 (the ring's next plane), x/y slopes
+  // and tildes of plane k+1 (the slope ring's next plane), sigma_z of plane
+  // k, z slopes of plane k+1.  (2-D: plane 0's sigmas and slopes.)  Segments
+  // in wave-aligned order (x items, y items, sigma_z, z slopes): one item
+  // kind per wavefront.  Each work item is a lambda whose early exits are
+  // returns, not loop continues: the compiler then allocates registers per
+  // item kind.
+  auto stageA = [&](int k) {
+    const int pA = Z ? k + 1 : 0;
+    const bool interiorA = !Z || (k >= klo && k <= khi);
+    const bool wSig = !Z || k + 1 <= kEnd;
+    const bool wL = !Z || (k + 1 >= klo && k + 1 <= khi);
+    const bool uXY = wSig || wL;
+    const int nSz = (Z && interiorA) ? I::NC : 0;
+    const int nZs = Z ? NCOL : 0;
+    constexpr int PUX = wave_up(I::NUX), PUY = wave_up(I::NUY), PZ4 = wave_up(I::NC);
+    const int s1 = uXY ? PUX + PUY : 0, s2 = s1 + (nSz ? PZ4 : 0), sEnd = s2 + nZs;
+    auto itemA = [&](int v) {
+      if (v < s1) {
+        if (v < PUX) {
+          if (v < I::NUX) x_item(v, pA, wSig, wL);
+        } else if (v - PUX < I::NUY) {
+          y_item(v - PUX, pA, wSig, wL);
+        }
+        return;
+      }
+      if (v < s2) {
+        const int r = v - s1;
+        if (r >= I::NC) return;
+        R v8[8];
+        const int a = r % (TX + 2) - 1, b = r / (TX + 2) - 1;
+        if (!tv_sigma<2>(P, tv, cell_b(P, ox + a, oy + b, k), szb, v8)) { bad = true; return; }
+        lds_put6(SZ, I::NC, r, v8);
+        return;
+      }
+      zslope_item(v - s2, k + 1);
+    };
+    for (int v = tid; v < sEnd; v += NT) itemA(item_index<OPAQUE>(v));
+  };
   if (Z) {
     // prologue: sigma_x/y of plane kBeg, z slopes of kBeg-1 and kBeg
     constexpr int Q1 = wave_up(I::NRX), Q2 = Q1 + wave_up(I::NRY), Q3 = Q2 + wave_up(NCOL);
@@ -554,77 +556,50 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
       else zslope_item(w - Q3, kBeg);
     }
   }
+  stageA(kBeg);
+  __syncthreads();
 
-  // fixed item extents of stages B and C (see above)
+  // roles of stages B and C, one state cell and one face per thread: x state
+  // cells (a in [-1, TX], with the face below each), y ones (b in [-1, TY]),
+  // columns (z state cell and face).  The extents are fixed so that item
+  // numbers split by compile-time divisors; the high row (a = TX) is skipped
+  // unless the tile sits at the block's high side, where it owns that row.
   constexpr int NBX = (TX + 2) * TY, NBY = TX * (TY + 2);
-  constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1);
+  constexpr int B1 = wave_up(NBX), B2 = B1 + wave_up(NBY), B3 = B2 + (Z ? NCOL : 0);
+  static_assert(B3 <= NT, "one state cell per thread");
+
+  // Wn of the thread's state cell from stage B to C; in a column, Wp of the
+  // plane below (the left state of the z face) as well, and the sum of the
+  // state pressures for pavg in the x role
+  R Wk[6], Wo[6], psum = R(0.);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) Wk[q] = Wo[q] = R(0.);
 
   for (int k = kBeg; k <= kEnd; ++k) {
     const bool interior = !Z || (k >= klo && k <= khi);
-    // ------------------------------ stage A ------------------------------
-    // Plane k+1's sigma_x/y (the ring's next plane) and x/y slopes (the
-    // slope ring's next plane), plane k's sigma_z, plane k+1's z slopes.
-    // (2-D: plane 0's sigmas and slopes.)
-    {
-      const int pA = Z ? k + 1 : 0;
-      const bool wSig = !Z || k + 1 <= kEnd;
-      const bool wL = !Z || (k + 1 >= klo && k + 1 <= khi);
-      const bool uXY = wSig || wL;
-      const int nSz = (Z && interior) ? I::NC : 0;
-      const int nZs = Z ? NCOL : 0;
-      constexpr int PUX = wave_up(I::NUX), PUY = wave_up(I::NUY), PZ = wave_up(I::NC);
-      // Segments in wave-aligned order (x items, y items, sigma_z, z
-      // slopes): one item kind per wavefront.  Each stage's work item is a
-      // lambda whose early exits are returns, not loop continues: the
-      // compiler then allocates registers per item kind.  With loop-level
-      // continues the FP64 16x8 march spilled 272 B per lane at 256 VGPRs;
-      // as lambdas it needs 251 and spills nothing (FP64 march 11.7 -> 9.3
-      // ms on 4096 x 16^3, FP32 10.4 -> 7.7 ms).  One x item serves a
-      // cell's sigma_x and x slope (one stencil, one eigen system), which
-      // keeps the slopes of two planes in LDS.
-      const int s1 = uXY ? PUX + PUY : 0, s2 = s1 + (nSz ? PZ : 0), sEnd = s2 + nZs;
-      auto itemA = [&](int v) {
-        if (v < s1) {
-          if (v < PUX) {
-            if (v < I::NUX) x_item(v, pA, wSig, wL);
-          } else if (v - PUX < I::NUY) {
-            y_item(v - PUX, pA, wSig, wL);
-          }
-          return;
-        }
-        if (v < s2) {
-          const int r = v - s1;
-          if (r >= I::NC) return;
-          R v8[8];
-          const int a = r % (TX + 2) - 1, b = r / (TX + 2) - 1;
-          if (!tv_sigma<2>(P, tv, cell_b(P, ox + a, oy + b, k), szb, v8)) { bad = true; return; }
-          lds_put6(SZ, I::NC, r, v8);
-          return;
-        }
-        zslope_item(v - s2, k + 1);
-      };
-      for (int v = tid; v < sEnd; v += NT) itemA(item_index<OPAQUE>(v));
-    }
-    __syncthreads();
-
     const R* sxk = SX + ring(k) * 6 * I::NRX;
     const R* syk = SY + ring(k) * 6 * I::NRY;
-    // ------------------------------ stage B1 -----------------------------
+    // ------------------------------ stage B ------------------------------
     {
-      // x-, y- and z-face states in wave-aligned segments
-      constexpr int B1 = wave_up(NBX), B2 = B1 + wave_up(NBY), B3 = B2 + (Z ? NCOL : 0);
-      auto itemB1 = [&](int w) {
-        R Wp[8], Wn[8], Vm[8], Vc[8], Vp[8], dbN[8], db0[8], dbP[8];
-        EigT<R> e0;
+      auto keep = [&](const R Wn[8]) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) Wk[q] = Wn[comp_slot(q)];
+      };
+      auto itemB = [&](int w) {
+        R Wp[8], Wn[8], Vm[8], Vc[8], Vp[8], dbN[8], db0[8], dbP[8], sg[8];
+        R sm[8], sc[8], sp[8], tA[8], tB[8];
+        EigT<R> e0, e1, e2;
         if (w < B1) {
           if (!interior || w >= NBX) return;
           const int a = w % (TX + 2) - 1, b = w / (TX + 2);
           if (a == TX && !ex) return;
+          const bool own = a >= 0 || ox == P.lo[0];  // (counts its reset)
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - sxb, Vm);
           tv_prim(tv, cb, Vc);
           tv_prim(tv, cb + sxb, Vp);
-          const R flat = P.flat ? tv_flat_coeff<0, R>(tv, cb, sxb) : R(0.);
+          const R* fx = FX + ringL(k) * I::NLX + I::lx(a, b);
+          const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], fx[-1], fx[0], fx[1]) : R(0.);
           const R* lxk = LX + ringL(k) * 6 * I::NLX;
           lds_get6(lxk, I::NLX, I::lx(a - 1, b), dbN);
           lds_get6(lxk, I::NLX, I::lx(a, b), db0);
@@ -633,25 +608,42 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * sxb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * sxb)) : R(0.);
           ppm_trace<0>(P, ratio(0), ratio(9), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          R sg[8];
           lds_get6(syk, I::NRY, I::ry(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(4));
           if (Z) {
-            lds_get6(SZ, I::NC, I::cc(a, b), sg);
-            sub_sigma(Wp, Wn, sg, ratio(5));
+            lds_get6(SZ, I::NC, I::cc(a, b), sc);
+            sub_sigma(Wp, Wn, sc, ratio(5));
           }
-          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, a >= 0 || ox == P.lo[0]);
-          put_state(WX, I::NRY, I::ry(a, b), Wp, Wn);
+          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
+          if (Z && P.ctu3d) {
+            // sigma_z over j with the y eigen system, sigma_y over k with z's
+            e1 = e2 = e0;
+            e1.un = Vc[P_VELY];
+            e2.un = Vc[P_VELZ];
+            lds_get6(SZ, I::NC, I::cc(a, b - 1), sm);
+            lds_get6(SZ, I::NC, I::cc(a, b + 1), sp);
+            trans_sigma<1>(P, sm, sc, sp, e1, tA);
+            lds_get6(SY + ring(k - 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sm);
+            lds_get6(SY + ring(k + 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sp);
+            trans_sigma<2>(P, sm, sg, sp, e2, tB);
+            add_ctu(Wp, Wn, tA, tB, ratio(6));
+            if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
+          }
+          lds_put6(WX, I::NRY, I::ry(a, b), Wp);
+          psum = Wn[P_PRES] + Wp[P_PRES];
+          keep(Wn);
         } else if (w < B2) {
           const int w2 = w - B1;
           if (!interior || w2 >= NBY) return;
           const int a = w2 % TX, b = w2 / TX - 1;
           if (b == TY && !ey) return;
+          const bool own = b >= 0 || oy == P.lo[1];
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - syb, Vm);
           tv_prim(tv, cb, Vc);
           tv_prim(tv, cb + syb, Vp);
-          const R flat = P.flat ? tv_flat_coeff<1, R>(tv, cb, syb) : R(0.);
+          const R* fy = FY + ringL(k) * I::NLY + I::ly(a, b);
+          const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], fy[-TX], fy[0], fy[TX]) : R(0.);
           const R* lyk = LY + ringL(k) * 6 * I::NLY;
           lds_get6(lyk, I::NLY, I::ly(a, b - 1), dbN);
           lds_get6(lyk, I::NLY, I::ly(a, b), db0);
@@ -660,29 +652,40 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * syb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * syb)) : R(0.);
           ppm_trace<1>(P, ratio(1), ratio(10), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          R sg[8];
           lds_get6(sxk, I::NRX, I::rx(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(3));
           if (Z) {
-            lds_get6(SZ, I::NC, I::cc(a, b), sg);
-            sub_sigma(Wp, Wn, sg, ratio(5));
+            lds_get6(SZ, I::NC, I::cc(a, b), sc);
+            sub_sigma(Wp, Wn, sc, ratio(5));
           }
-          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, b >= 0 || oy == P.lo[1]);
-          put_state(WY, I::NRX, I::rx(a, b), Wp, Wn);
-        } else {
+          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
+          if (Z && P.ctu3d) {
+            // sigma_x over k with z's eigen system, sigma_z over i with x's
+            e1 = e2 = e0;
+            e1.un = Vc[P_VELZ];
+            e2.un = Vc[P_VELX];
+            lds_get6(SX + ring(k - 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sm);
+            lds_get6(SX + ring(k + 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sp);
+            trans_sigma<2>(P, sm, sg, sp, e1, tA);
+            lds_get6(SZ, I::NC, I::cc(a - 1, b), sm);
+            lds_get6(SZ, I::NC, I::cc(a + 1, b), sp);
+            trans_sigma<0>(P, sm, sc, sp, e2, tB);
+            add_ctu(Wp, Wn, tA, tB, ratio(7));
+            if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
+          }
+          lds_put6(WY, I::NRX, I::rx(a, b), Wp);
+          PY[I::rx(a, b)] = Wn[P_PRES] + Wp[P_PRES];
+          keep(Wn);
+        } else if (Z && w < B3) {
           const int w2 = w - B2;
           const int a = w2 % TX, b = w2 / TX;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - szb, Vm);
           tv_prim(tv, cb, Vc);
           tv_prim(tv, cb + szb, Vp);
-          R flat = R(0.);
-          if (P.flat) {
-            const R dp1 = Vp[P_PRES] - Vm[P_PRES];
-            const R f0 = FZ[ring(k) * NCOL + w2];
-            flat = dp1 < R(0.0) ? fmax(f0, FZ[ring(k + 1) * NCOL + w2])
-                                : (dp1 == R(0.) ? f0 : fmax(f0, FZ[ring(k - 1) * NCOL + w2]));
-          }
+          const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], FZ[ring(k - 1) * NCOL + w2],
+                                          FZ[ring(k) * NCOL + w2], FZ[ring(k + 1) * NCOL + w2])
+                                : R(0.);
           lds_get6(LZ + ring(k - 1) * 6 * NCOL, NCOL, w2, dbN);
           lds_get6(LZ + ring(k) * 6 * NCOL, NCOL, w2, db0);
           lds_get6(LZ + ring(k + 1) * 6 * NCOL, NCOL, w2, dbP);
@@ -690,180 +693,113 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * szb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * szb)) : R(0.);
           ppm_trace<2>(P, ratio(2), ratio(11), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          R sg[8];
-          lds_get6(sxk, I::NRX, I::rx(a, b), sg);
-          sub_sigma(Wp, Wn, sg, ratio(3));
+          lds_get6(sxk, I::NRX, I::rx(a, b), sc);
+          sub_sigma(Wp, Wn, sc, ratio(3));
           lds_get6(syk, I::NRY, I::ry(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(4));
           if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
-          put_state(WZ, NCOL, w2, Wp, Wn);
+          if (P.ctu3d) {
+            // sigma_y over i with x's eigen system, sigma_x over j with y's
+            e1 = e2 = e0;
+            e1.un = Vc[P_VELX];
+            e2.un = Vc[P_VELY];
+            lds_get6(syk, I::NRY, I::ry(a - 1, b), sm);
+            lds_get6(syk, I::NRY, I::ry(a + 1, b), sp);
+            trans_sigma<0>(P, sm, sg, sp, e1, tA);
+            lds_get6(sxk, I::NRX, I::rx(a, b - 1), sm);
+            lds_get6(sxk, I::NRX, I::rx(a, b + 1), sp);
+            trans_sigma<1>(P, sm, sc, sp, e2, tB);
+            add_ctu(Wp, Wn, tA, tB, ratio(8));
+            if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
+          }
+          // the column's Wp stays with its thread: last plane's out, this one's in
+#pragma unroll
+          for (int q = 0; q < 6; ++q) Wo[q] = WZ[q * NCOL + w2];
+          lds_put6(WZ, NCOL, w2, Wp);
+          PZ[w2] = Wn[P_PRES] + Wp[P_PRES];
+          keep(Wn);
         }
       };
-      for (int w = tid; w < B3; w += NT) itemB1(item_index<OPAQUE>(w));
+      itemB(item_index<OPAQUE>(tid));
     }
     __syncthreads();
 
-    // ------------------------------ stage B2 -----------------------------
-    if (Z && P.ctu3d) {
-      constexpr int C1 = wave_up(NBX), C2 = C1 + wave_up(NBY), C3 = C2 + NCOL;
-      auto itemB2 = [&](int w) {
-        R Wp[8], Wn[8], Vc[8], sm[8], sc[8], sp[8], tA[8], tB[8];
-        EigT<R> e1, e2;
-        R fac;
-        R* base;
-        int n, idx;
-        bool own = true;  // the tile owns this state cell (counts its reset)
-        if (w < C1) {
-          // X: sigma_z over j with the y eigen system, sigma_y over k with z's
-          if (!interior || w >= NBX) return;
-          const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-          if (a == TX && !ex) return;
-          own = a >= 0 || ox == P.lo[0];
-          tv_prim(tv, cell_b(P, ox + a, oy + b, k), Vc);
-          if (!(eig_make<1>(Vc, e1) &&
-                eig_make<2>(Vc, e2))) { bad = true; return; }
-          lds_get6(SZ, I::NC, I::cc(a, b - 1), sm);
-          lds_get6(SZ, I::NC, I::cc(a, b), sc);
-          lds_get6(SZ, I::NC, I::cc(a, b + 1), sp);
-          trans_sigma<1>(P, sm, sc, sp, e1, tA);
-          lds_get6(SY + ring(k - 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sm);
-          lds_get6(syk, I::NRY, I::ry(a, b), sc);
-          lds_get6(SY + ring(k + 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sp);
-          trans_sigma<2>(P, sm, sc, sp, e2, tB);
-          fac = ratio(6);
-          base = WX; n = I::NRY; idx = I::ry(a, b);
-        } else if (w < C2) {
-          // Y: sigma_x over k with z's eigen system, sigma_z over i with x's
-          const int w2 = w - C1;
-          if (!interior || w2 >= NBY) return;
-          const int a = w2 % TX, b = w2 / TX - 1;
-          if (b == TY && !ey) return;
-          own = b >= 0 || oy == P.lo[1];
-          tv_prim(tv, cell_b(P, ox + a, oy + b, k), Vc);
-          if (!(eig_make<2>(Vc, e1) &&
-                eig_make<0>(Vc, e2))) { bad = true; return; }
-          lds_get6(SX + ring(k - 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sm);
-          lds_get6(sxk, I::NRX, I::rx(a, b), sc);
-          lds_get6(SX + ring(k + 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sp);
-          trans_sigma<2>(P, sm, sc, sp, e1, tA);
-          lds_get6(SZ, I::NC, I::cc(a - 1, b), sm);
-          lds_get6(SZ, I::NC, I::cc(a, b), sc);
-          lds_get6(SZ, I::NC, I::cc(a + 1, b), sp);
-          trans_sigma<0>(P, sm, sc, sp, e2, tB);
-          fac = ratio(7);
-          base = WY; n = I::NRX; idx = I::rx(a, b);
-        } else {
-          // Z: sigma_y over i with x's eigen system, sigma_x over j with y's
-          const int w2 = w - C2;
-          const int a = w2 % TX, b = w2 / TX;
-          tv_prim(tv, cell_b(P, ox + a, oy + b, k), Vc);
-          if (!(eig_make<0>(Vc, e1) &&
-                eig_make<1>(Vc, e2))) { bad = true; return; }
-          lds_get6(syk, I::NRY, I::ry(a - 1, b), sm);
-          lds_get6(syk, I::NRY, I::ry(a, b), sc);
-          lds_get6(syk, I::NRY, I::ry(a + 1, b), sp);
-          trans_sigma<0>(P, sm, sc, sp, e1, tA);
-          lds_get6(sxk, I::NRX, I::rx(a, b - 1), sm);
-          lds_get6(sxk, I::NRX, I::rx(a, b), sc);
-          lds_get6(sxk, I::NRX, I::rx(a, b + 1), sp);
-          trans_sigma<1>(P, sm, sc, sp, e2, tB);
-          fac = ratio(8);
-          base = WZ; n = NCOL; idx = w2;
-        }
-        get_state(base, n, idx, Wp, Wn);
-        add_ctu(Wp, Wn, tA, tB, fac);
-        if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
-        put_state(base, n, idx, Wp, Wn);
-      };
-      for (int w = tid; w < C3; w += NT) itemB2(item_index<OPAQUE>(w));
-      __syncthreads();
-    }
-
     // ------------------------------ stage C ------------------------------
     {
-      // x faces, y faces, column items (z face, pavg) in wave-aligned segments
-      constexpr int D1 = wave_up(NFX), D2 = D1 + wave_up(NFY), D3 = D2 + NCOL;
-      const bool cols = Z || interior;
+      auto right = [&](R VR[8]) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) VR[comp_slot(q)] = Wk[q];
+      };
+      auto gammas = [&](unsigned cl, unsigned cr, R VL[8], R VR[8]) {
+        VL[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cl));
+        VL[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cl));
+        VR[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cr));
+        VR[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cr));
+      };
       auto itemC = [&](int w) {
         R VL[8], VR[8];
         double F[8];
-        if (w < D1) {
-          if (!interior || w >= NFX) return;
-          const int a = w % (TX + 1), b = w / (TX + 1);
-          if (a == TX && !ex) return;
-          lds_get6(WX, I::NRY, I::ry(a - 1, b), VL);
-          lds_get6(WX + 6 * I::NRY, I::NRY, I::ry(a, b), VR);
+        if (w < B1) {
+          if (!interior || w >= NBX) return;
+          const int a = w % (TX + 2) - 1, b = w / (TX + 2);
+          if (a < 0 || (a == TX && !ex)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
-          VL[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb - sxb));
-          VL[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb - sxb));
-          VR[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb));
-          VR[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb));
+          if (P.aux && a < TX) {
+            // face-averaged pressure (hy_getFaceFlux.F90:507-561 and the
+            // y, z analogues)
+            R pres = R(0.5) * psum;
+            pres = pres * R(0.5) + PY[I::rx(a, b)] * R(0.25);
+            if (Z) pres = div_const<6>(pres * R(4.0) + PZ[b * TX + a]);
+            const unsigned r = (unsigned)(((k - P.lo[2]) * P.nyb + (oy + b - P.lo[1])) * P.nxb + (ox + a - P.lo[0]));
+            st_at(as_global(T.pavg), r * 8u, double(pres));
+          }
+          lds_get6(WX, I::NRY, I::ry(a - 1, b), VL);
+          right(VR);
+          gammas(cb - sxb, cb, VL, VR);
           const unsigned fr = (unsigned)face_index(P, 0, ox + a, oy + b, k);
           if constexpr (is_states(RS)) {
             write_face_states<0>(P, fsb + fstate_dir_offset(P, 0), fr, VL, VR);
-            return;
           } else {
             if (face_flux<0, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - sxb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 0); return; }
             write_flux_b<0>(P, as_global(T.flux[0]), fr * 8u, F);
           }
-        } else if (w < D2) {
-          const int w2 = w - D1;
-          if (!interior || w2 >= NFY) return;
-          const int a = w2 % TX, b = w2 / TX;
-          if (b == TY && !ey) return;
-          lds_get6(WY, I::NRX, I::rx(a, b - 1), VL);
-          lds_get6(WY + 6 * I::NRX, I::NRX, I::rx(a, b), VR);
+        } else if (w < B2) {
+          const int w2 = w - B1;
+          if (!interior || w2 >= NBY) return;
+          const int a = w2 % TX, b = w2 / TX - 1;
+          if (b < 0 || (b == TY && !ey)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
-          VL[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb - syb));
-          VL[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb - syb));
-          VR[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb));
-          VR[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb));
+          lds_get6(WY, I::NRX, I::rx(a, b - 1), VL);
+          right(VR);
+          gammas(cb - syb, cb, VL, VR);
           const unsigned fr = (unsigned)face_index(P, 1, ox + a, oy + b, k);
           if constexpr (is_states(RS)) {
             write_face_states<1>(P, fsb + fstate_dir_offset(P, 1), fr, VL, VR);
-            return;
           } else {
             if (face_flux<1, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - syb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 1); return; }
             write_flux_b<1>(P, as_global(T.flux[1]), fr * 8u, F);
           }
-        } else {
-          // column item: z-face flux at face k, pavg of the cell, carry Wp
-          if (!cols) return;
-          const int w2 = w - D2;
+        } else if (Z && w < B3) {
+          if (k < klo) return;
+          const int w2 = w - B2;
           const int a = w2 % TX, b = w2 / TX;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
-          if (Z && k >= klo) {
-            lds_get6(WZP, NCOL, w2, VL);
-            lds_get6(WZ + 6 * NCOL, NCOL, w2, VR);
-            VL[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb - szb));
-            VL[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb - szb));
-            VR[P_GAMC] = R(tv_ld(tv, tv.ob[P_GAMC], cb));
-            VR[P_GAME] = R(tv_ld(tv, tv.ob[P_GAME], cb));
-            const unsigned fr = (unsigned)face_index(P, 2, ox + a, oy + b, k);
-            if constexpr (is_states(RS)) {
-              write_face_states<2>(P, fsb + fstate_dir_offset(P, 2), fr, VL, VR);
-            } else {
-              if (face_flux<2, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - szb, cb), F, es)) report_error(st, 2, t, ox + a, oy + b, k, 2);
-              else write_flux_b<2>(P, as_global(T.flux[2]), fr * 8u, F);
-            }
-          }
-          if (interior && P.aux) {
-            // face-averaged pressure (hy_getFaceFlux.F90:507-561 and the
-            // y, z analogues)
-            R pres = R(0.5) * (WX[10 * I::NRY + I::ry(a, b)] + WX[4 * I::NRY + I::ry(a, b)]);
-            pres = pres * R(0.5) + (WY[10 * I::NRX + I::rx(a, b)] + WY[4 * I::NRX + I::rx(a, b)]) * R(0.25);
-            if (Z) pres = div_const<6>(pres * R(4.0) + (WZ[10 * NCOL + w2] + WZ[4 * NCOL + w2]));
-            const unsigned r = (unsigned)(((k - P.lo[2]) * P.nyb + (oy + b - P.lo[1])) * P.nxb + (ox + a - P.lo[0]));
-            st_at(as_global(T.pavg), r * 8u, double(pres));
-          }
-          if (Z) {
 #pragma unroll
-            for (int q = 0; q < 6; ++q) WZP[q * NCOL + w2] = WZ[q * NCOL + w2];
+          for (int q = 0; q < 6; ++q) VL[comp_slot(q)] = Wo[q];
+          right(VR);
+          gammas(cb - szb, cb, VL, VR);
+          const unsigned fr = (unsigned)face_index(P, 2, ox + a, oy + b, k);
+          if constexpr (is_states(RS)) {
+            write_face_states<2>(P, fsb + fstate_dir_offset(P, 2), fr, VL, VR);
+          } else {
+            if (face_flux<2, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - szb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 2); return; }
+            write_flux_b<2>(P, as_global(T.flux[2]), fr * 8u, F);
           }
         }
       };
-      for (int w = tid; w < D3; w += NT) itemC(item_index<OPAQUE>(w));
+      itemC(item_index<OPAQUE>(tid));
     }
+    if (k < kEnd) stageA(k + 1);
     __syncthreads();
   }
   if (bad) report_error(st, 1, t, ox, oy, -1, -1);
@@ -872,10 +808,9 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
 // One workgroup per column tile of a batch of equal-shape tiles.  OCC > 0
 // asks the compiler for OCC waves per SIMD (fewer registers, maybe spills);
 // the autotuner decides whether that pays.  The FP64 16x8 tile runs 768
-// threads, 3 waves per SIMD: its LDS allows one workgroup per CU, and with
-// the item numbers opaque the march fits the 168 registers of 3 waves
-// without spilling.  Stage A's 708 items then take one pass instead of two
-// (B1, B2 and C keep 8 busy waves of 12): 8.83 -> 8.41 ms on 4096 x 16^3.
+// threads: its LDS allows one workgroup per CU, stage A has 12 wavefronts of
+// items, and 3 waves per SIMD leave 168 registers (at 512 threads the march
+// took 8.83 instead of 8.41 ms on 4096 x 16^3).
 template <int NDIM, int TX, int TY, int NT, int RS, typename R, int OCC = 0>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 k_march(DevParams P, MarchLaunch L) {
@@ -887,8 +822,7 @@ k_march(DevParams P, MarchLaunch L) {
   ExactStats es{0ULL, 0ULL};
   R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + t * fstate_tile_stride(P) : nullptr;
   __shared__ R smem[MarchLds<NDIM, TX, TY>::total];
-  march_tile<NDIM, TX, TY, NT, RS, R, (sizeof(R) == 4 || NT > 512)>(P, L, t, ox, oy, fsb, es,
-                                                                    smem);
+  march_tile<NDIM, TX, TY, NT, RS, R, true>(P, L, t, ox, oy, fsb, es, smem);
   flush_exact(L.status, es);
 }
 

@@ -14,25 +14,21 @@ namespace fx {
 template <int RS, typename R>
 void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
                     const MarchHost& H) {
+  constexpr int OCC = sizeof(R) == 8 ? 3 : 0;  // waves per SIMD
   if constexpr (sizeof(R) == 4) {  // FP32 3-D: the autotuner may ask for 4 waves per SIMD
     if (P.ndim == 3 && H.tuneOcc == 4) {
       if (TX == 16)
         hipLaunchKernelGGL((k_march<3, 16, 8, 512, RS, R, 4>), grid, dim3(512), 0, H.stream, P, M);
       else
-        hipLaunchKernelGGL((k_march<3, 8, 8, 256, RS, R, 4>), grid, dim3(256), 0, H.stream, P, M);
+        hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, 4>), grid, dim3(384), 0, H.stream, P, M);
       return;
     }
   }
-  if constexpr (sizeof(R) == 8) {  // FP64 3-D 16x8: 768 threads, 3 waves per SIMD
-    if (P.ndim == 3 && TX == 16) {
-      hipLaunchKernelGGL((k_march<3, 16, 8, 768, RS, R, 3>), grid, dim3(768), 0, H.stream, P, M);
-      return;
-    }
-  }
-  if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, 512, RS, R>), grid, dim3(512), 0, H.stream, P, M);
-  else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 256, RS, R>), grid, dim3(256), 0, H.stream, P, M);
-  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, 256, RS, R>), grid, dim3(256), 0, H.stream, P, M);
-  else hipLaunchKernelGGL((k_march<2, 8, 8, 256, RS, R>), grid, dim3(256), 0, H.stream, P, M);
+  constexpr int NT3 = sizeof(R) == 8 ? 768 : 512;  // FP64 3-D 16x8: 768 threads
+  if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, NT3, RS, R, OCC>), grid, dim3(NT3), 0, H.stream, P, M);
+  else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, OCC>), grid, dim3(384), 0, H.stream, P, M);
+  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, 384, RS, R, OCC>), grid, dim3(384), 0, H.stream, P, M);
+  else hipLaunchKernelGGL((k_march<2, 8, 8, 256, RS, R, OCC>), grid, dim3(256), 0, H.stream, P, M);
 }
 
 // Persistent multi-class march: as many workgroups as stay resident (or
@@ -75,6 +71,7 @@ void launch_march_mixw_k(const MarchLaunch& M, const MarchHost& H) {
 
 template <int RS, typename R>
 void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHost& H) {
+  constexpr int OCC = sizeof(R) == 8 ? 3 : 0;  // waves per SIMD
   if (TX == kPerClassTX) {  // 16- and 8-wide column tiles in one launch
     if constexpr (sizeof(R) == 4) {
       if (ndim == 3 && H.tuneOcc == 4) {
@@ -89,13 +86,13 @@ void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHos
       }
     }
     if (ndim == 3) launch_march_mixw_k<3, 512, RS, R>(M, H);
-    else launch_march_mixw_k<2, 256, RS, R>(M, H);
+    else launch_march_mixw_k<2, 384, RS, R, OCC>(M, H);
     return;
   }
   if constexpr (sizeof(R) == 4) {  // FP32 3-D: the autotuner may ask for 4 waves per SIMD
     if (ndim == 3 && H.tuneOcc == 4) {
       if (TX == 16) launch_march_multi_k<3, 16, 8, 512, RS, R, 4>(M, H);
-      else launch_march_multi_k<3, 8, 8, 256, RS, R, 4>(M, H);
+      else launch_march_multi_k<3, 8, 8, 384, RS, R, 4>(M, H);
       return;
     }
   }
@@ -106,9 +103,9 @@ void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHos
     }
   }
   if (ndim == 3 && TX == 16) launch_march_multi_k<3, 16, 8, 512, RS, R>(M, H);
-  else if (ndim == 3) launch_march_multi_k<3, 8, 8, 256, RS, R>(M, H);
-  else if (TX == 16) launch_march_multi_k<2, 16, 8, 256, RS, R>(M, H);
-  else launch_march_multi_k<2, 8, 8, 256, RS, R>(M, H);
+  else if (ndim == 3) launch_march_multi_k<3, 8, 8, 384, RS, R, OCC>(M, H);
+  else if (TX == 16) launch_march_multi_k<2, 16, 8, 384, RS, R, OCC>(M, H);
+  else launch_march_multi_k<2, 8, 8, 256, RS, R, OCC>(M, H);
 }
 
 template void launch_march_r<FX_MARCH_RS, FX_MARCH_R>(const DevParams&, const MarchLaunch&, int,
