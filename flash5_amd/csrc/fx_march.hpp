@@ -66,7 +66,7 @@ template <int NDIM, int TX, int TY> struct MarchLds {
   static constexpr int WZ = WY + 6 * I::NRX;                  // z state cells' Wp of the last plane done
   static constexpr int PY = WZ + (Z ? 6 * NCOL : 1);          // Wn + Wp pressures of the y state cells
   static constexpr int PZ = PY + I::NRX;                      // and of the z state cells
-  static constexpr int CST = PZ + (Z ? NCOL : 1);             // the step's ratios, widths (FP32)
+  static constexpr int CST = PZ + (Z ? NCOL : 1);             // the step's ratios, widths
   static constexpr int total = CST + 12;
 };
 
@@ -269,9 +269,9 @@ __device__ __forceinline__ bool tv_sigma(const DevParams& P, const TileView& tv,
   tv_prim(tv, cb, Vc);
   tv_prim(tv, cb + sb, Vp);
   EigT<R> e;
-  if (!eig_make<SD>(Vc, e)) return false;
+  const bool ok = eig_make<SD>(Vc, e);
   trans_sigma<SD>(P, Vm, Vc, Vp, e, sig);
-  return true;
+  return ok;
 }
 
 // Whether the face between the cells at cbl and cbr takes HLL (HLL, or the
@@ -361,24 +361,19 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   const int klo = P.lo[2], khi = P.hi[2];
   DevStatus* st = L.status;
   bool bad = false;  // eigen failure seen by this thread
-  // The step's ratios of dt and the cell widths, and the widths, uniform
-  // over the tile.  The FP64 march keeps them in registers (the compiler
-  // hoists them); the FP32 march reads them from LDS, written once per
-  // column tile by one thread (stage B first reads them after a barrier, and
-  // the previous column tile ended on one): 12 fewer live registers.
+  // The step's ratios of dt and the cell widths, and the widths, uniform over
+  // the tile: read from LDS, written once per column tile by one thread (stage
+  // B first reads them after a barrier, and the previous column tile ended on
+  // one).  Held in registers they take 24 of the 168 an FP64 thread has (no
+  // scalar FP64 arithmetic makes them scalar).
   const R rat[12] = {R(dt / dx), R(dt / dy), R(dt / dz),
                      R(0.5 * dt / dx), R(0.5 * dt / dy), R(0.5 * dt / dz),
                      R(dt * dt / (6. * dy * dz)), R(dt * dt / (6. * dz * dx)),
                      R(dt * dt / (6. * dx * dy)), R(dx), R(dy), R(dz)};
   R* const CST = smem + M::CST;
-  if constexpr (sizeof(R) == 4) {
-    if (tid == 0)
-      for (int i = 0; i < 12; ++i) CST[i] = rat[i];
-  }
-  auto ratio = [&](int i) -> R {
-    if constexpr (sizeof(R) == 4) return CST[i];
-    else return rat[i];
-  };
+  if (tid == 0)
+    for (int i = 0; i < 12; ++i) CST[i] = rat[i];
+  auto ratio = [&](int i) -> R { return CST[i]; };
 
   auto ring = [](int k) { return NR == 3 ? (k % 3) : 0; };
   auto ringL = [](int k) { return M::NRL == 2 ? (k & 1) : 0; };
@@ -387,13 +382,13 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   auto sig_x_item = [&](int w, int kk) {
     R sg[8];
     const int a = w % TX, b = w / TX - 1;
-    if (!tv_sigma<0>(P, tv, cell_b(P, ox + a, oy + b, kk), sxb, sg)) { bad = true; return; }
+    bad |= !tv_sigma<0>(P, tv, cell_b(P, ox + a, oy + b, kk), sxb, sg);
     lds_put6(SX + ring(kk) * 6 * I::NRX, I::NRX, w, sg);
   };
   auto sig_y_item = [&](int w, int kk) {
     R sg[8];
     const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-    if (!tv_sigma<1>(P, tv, cell_b(P, ox + a, oy + b, kk), syb, sg)) { bad = true; return; }
+    bad |= !tv_sigma<1>(P, tv, cell_b(P, ox + a, oy + b, kk), syb, sg);
     lds_put6(SY + ring(kk) * 6 * I::NRY, I::NRY, w, sg);
   };
   // stage-A items along x (w < NUX) and y (w < NUY) at plane p: one cell's
@@ -425,7 +420,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     tv_prim(tv, cb, Vc);
     tv_prim(tv, cb + sxb, Vp);
     EigT<R> e;
-    if (!eig_make<0>(Vc, e)) { bad = true; return; }
+    bad |= !eig_make<0>(Vc, e);
     if (doS) {
       R sg[8];
       trans_sigma<0>(P, Vm, Vc, Vp, e, sg);
@@ -464,7 +459,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     tv_prim(tv, cb, Vc);
     tv_prim(tv, cb + syb, Vp);
     EigT<R> e;
-    if (!eig_make<1>(Vc, e)) { bad = true; return; }
+    bad |= !eig_make<1>(Vc, e);
     if (doS) {
       R sg[8];
       trans_sigma<1>(P, Vm, Vc, Vp, e, sg);
@@ -489,7 +484,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     tv_prim(tv, cb, Vc);
     tv_prim(tv, cb + szb, Vp);
     EigT<R> e;
-    if (!eig_make<2>(Vc, e)) { bad = true; return; }
+    bad |= !eig_make<2>(Vc, e);
     tvd_slope<2>(P, Vm, Vc, Vp, e, db);
     lds_put6(LZ + ring(m) * 6 * NCOL, NCOL, w, db);
     if (P.flat)
@@ -538,7 +533,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
         if (r >= I::NC) return;
         R v8[8];
         const int a = r % (TX + 2) - 1, b = r / (TX + 2) - 1;
-        if (!tv_sigma<2>(P, tv, cell_b(P, ox + a, oy + b, k), szb, v8)) { bad = true; return; }
+        bad |= !tv_sigma<2>(P, tv, cell_b(P, ox + a, oy + b, k), szb, v8);
         lds_put6(SZ, I::NC, r, v8);
         return;
       }
@@ -604,7 +599,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           lds_get6(lxk, I::NLX, I::lx(a - 1, b), dbN);
           lds_get6(lxk, I::NLX, I::lx(a, b), db0);
           lds_get6(lxk, I::NLX, I::lx(a + 1, b), dbP);
-          if (!eig_make<0>(Vc, e0)) { bad = true; return; }
+          bad |= !eig_make<0>(Vc, e0);
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * sxb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * sxb)) : R(0.);
           ppm_trace<0>(P, ratio(0), ratio(9), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
@@ -648,7 +643,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           lds_get6(lyk, I::NLY, I::ly(a, b - 1), dbN);
           lds_get6(lyk, I::NLY, I::ly(a, b), db0);
           lds_get6(lyk, I::NLY, I::ly(a, b + 1), dbP);
-          if (!eig_make<1>(Vc, e0)) { bad = true; return; }
+          bad |= !eig_make<1>(Vc, e0);
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * syb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * syb)) : R(0.);
           ppm_trace<1>(P, ratio(1), ratio(10), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
@@ -689,7 +684,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           lds_get6(LZ + ring(k - 1) * 6 * NCOL, NCOL, w2, dbN);
           lds_get6(LZ + ring(k) * 6 * NCOL, NCOL, w2, db0);
           lds_get6(LZ + ring(k + 1) * 6 * NCOL, NCOL, w2, dbP);
-          if (!eig_make<2>(Vc, e0)) { bad = true; return; }
+          bad |= !eig_make<2>(Vc, e0);
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * szb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * szb)) : R(0.);
           ppm_trace<2>(P, ratio(2), ratio(11), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
