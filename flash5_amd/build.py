@@ -32,6 +32,12 @@ HIP_FLAGS = [
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
 
+# The column march keeps its constants and addresses out of loop-invariant
+# code motion: hoisted in front of the plane loop, each takes a register that
+# the stages then lack (FP64 16x8 march 148 instead of 121, FP32 106 instead of
+# 81), while making them again per plane hides in the waits.
+MARCH_FLAGS = ["-mllvm", "-disable-machine-licm"]
+
 # The column-march kernels of each (solver family, real type) pair form a
 # translation unit of their own (fx_march_inst.hip), so the units build in
 # parallel; the main unit holds every other kernel and the C ABI.
@@ -58,7 +64,7 @@ def _units():
     inst = os.path.join(CSRC, "fx_march_inst.hip")
     out = [(main, [], os.path.join(OBJ_DIR, "fx_hydro.o"))]
     for rs, r in MARCH_UNITS:
-        out.append((inst, [f"-DFX_MARCH_RS={rs}", f"-DFX_MARCH_R={r}"],
+        out.append((inst, [*MARCH_FLAGS, f"-DFX_MARCH_RS={rs}", f"-DFX_MARCH_R={r}"],
                     os.path.join(OBJ_DIR, f"fx_march_{rs.lower()}_{r}.o")))
     return out
 

@@ -278,14 +278,16 @@ __device__ __forceinline__ UpdPart upd_start(const DevParams& P, double dt, doub
   return u;
 }
 
-// z term, sources, energy fix and EOS; out = dens, velx, vely, velz, ener,
-// eint, pres, temp, gamc, game (eintOld: the cell's e_int before the step,
-// used when the aux equation is off)
-__device__ __forceinline__ void upd_finish(const DevParams& P, double dt, double dz, UpdPart u,
-                                           const double FLz[8], const double FRz[8],
-                                           double eintOld, double out[10]) {
-  double Sz;
-  upd_dir(P, dt, dz, u.pres, FLz, FRz, u.U0, u.IntEner, Sz);
+// the updated cell, from which its other variables follow (upd_expand)
+struct UpdState {
+  double dens, vx, vy, vz, eint;
+};
+
+// sources, energy fix (hy_energyFix.F90:188-251) and the EOS's internal
+// energy, once u holds every direction's terms (eintOld: the cell's e_int
+// before the step, used when the aux equation is off)
+__device__ __forceinline__ UpdState upd_state(const DevParams& P, double dt, UpdPart u,
+                                              double eintOld, double Sz = 0.) {
   if (P.aux) u.IntEner = u.IntEner + dt * 0.0;
   const double Sphys[5] = {0., u.S1, u.S2, Sz, 0.};
 #pragma unroll
@@ -300,17 +302,33 @@ __device__ __forceinline__ void upd_finish(const DevParams& P, double dt, double
   if (!P.aux || eint > P.eintSwitch * (ekin + 0.0)) newEint = fmax(P.smallE, eint);
   else newEint = fmax(P.smallE, eintAux);
   const double enerFix = newEint + ekin;
-  const EosOut eo = eos_dens_ei(P, densNew, vx, vy, vz, newEint, enerFix);
-  out[0] = densNew;
-  out[1] = vx;
-  out[2] = vy;
-  out[3] = vz;
+  return UpdState{densNew, vx, vy, vz, eos_ie(P, ekin, newEint, enerFix)};
+}
+
+// every variable of the updated cell: dens, velx, vely, velz, ener, eint,
+// pres, temp, gamc, game
+__device__ __forceinline__ void upd_expand(const DevParams& P, const UpdState& s, double out[10]) {
+  const double ekin = 0.5 * (s.vx * s.vx + s.vy * s.vy + s.vz * s.vz);
+  const EosOut eo = eos_of_ie(P, s.dens, ekin, s.eint);
+  out[0] = s.dens;
+  out[1] = s.vx;
+  out[2] = s.vy;
+  out[3] = s.vz;
   out[4] = eo.ener;
   out[5] = eo.eint;
   out[6] = eo.pres;
   out[7] = eo.temp;
   out[8] = P.gamma;
   out[9] = eo.game;
+}
+
+// z term, sources, energy fix and EOS; out as upd_expand's
+__device__ __forceinline__ void upd_finish(const DevParams& P, double dt, double dz, UpdPart u,
+                                           const double FLz[8], const double FRz[8],
+                                           double eintOld, double out[10]) {
+  double Sz;
+  upd_dir(P, dt, dz, u.pres, FLz, FRz, u.U0, u.IntEner, Sz);
+  upd_expand(P, upd_state(P, dt, u, eintOld, Sz), out);
 }
 
 // U slots of upd_finish's outputs

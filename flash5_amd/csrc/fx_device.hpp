@@ -849,12 +849,15 @@ constexpr float kNoSeed = 3.0e38f;
 struct EosOut {
   double pres, temp, eint, ener, game;
 };
-__device__ __forceinline__ EosOut eos_dens_ei(const DevParams& P, double dens, double vx, double vy,
-                                              double vz, double eintIn, double enerIn) {
-  const double ekin = 0.5 * (vx * vx + vy * vy + vz * vz);
+// the internal energy the EOS takes, from the kinetic energy per mass
+__device__ __forceinline__ double eos_ie(const DevParams& P, double ekin, double eintIn,
+                                         double enerIn) {
   double ie = eintIn;
   if (enerIn - ekin > fmax(P.smallE, P.eintSwitch * ekin)) ie = enerIn - ekin;
-  ie = fmax(ie, P.smallE);
+  return fmax(ie, P.smallE);
+}
+// and what follows from it
+__device__ __forceinline__ EosOut eos_of_ie(const DevParams& P, double dens, double ekin, double ie) {
   EosOut o;
   o.eint = ie;
   o.pres = dens * ie * P.gam1inv;
@@ -862,6 +865,11 @@ __device__ __forceinline__ EosOut eos_dens_ei(const DevParams& P, double dens, d
   o.ener = ie + ekin;
   o.game = o.pres / (ie * dens) + 1;
   return o;
+}
+__device__ __forceinline__ EosOut eos_dens_ei(const DevParams& P, double dens, double vx, double vy,
+                                              double vz, double eintIn, double enerIn) {
+  const double ekin = 0.5 * (vx * vx + vy * vy + vz * vz);
+  return eos_of_ie(P, dens, ekin, eos_ie(P, ekin, eintIn, enerIn));
 }
 
 }  // namespace fx

@@ -559,6 +559,32 @@ k_update_cols(DevParams P, Launch L, const unsigned char* __restrict__ inPlace) 
   }
 }
 
+// The rest of the fused update: the march (FUSE) left each updated cell's
+// density, velocities and internal energy in scratch, component by component
+// over the interior cells; the other variables follow from them.  40 bytes
+// read and 80 written a cell, against the 268 and 80 of an update that reads
+// the face fluxes back.
+__global__ void __launch_bounds__(kThreads)
+k_update_finish(DevParams P, const fx_tile* __restrict__ tiles, int nTiles,
+                const double* __restrict__ upd) {
+  const unsigned n = (unsigned)P.icells, nx = (unsigned)P.nxb, ny = (unsigned)P.nyb;
+  const long total = P.icells * nTiles;
+  for (long gid = (long)blockIdx.x * blockDim.x + threadIdx.x; gid < total;
+       gid += (long)gridDim.x * blockDim.x) {
+    const long t = gid / n;
+    const unsigned r = (unsigned)(gid - t * n);
+    const double* const u = upd + t * (kUpdComps * P.icells) + r;
+    const UpdState s{u[0], u[P.icells], u[2 * P.icells], u[3 * P.icells], u[4 * P.icells]};
+    double out[10];
+    upd_expand(P, s, out);
+    gdouble* const U = as_global(tiles[t].U);
+    const long c = cidx(P, (int)(r % nx) + P.lo[0], (int)((r / nx) % ny) + P.lo[1],
+                        (int)(r / (nx * ny)) + P.lo[2]);
+#pragma unroll
+    for (int v = 0; v < 10; ++v) U[P.voff[upd_var(v)] + c] = out[v];
+  }
+}
+
 // the update over tiles of several block classes in one launch
 __global__ void __launch_bounds__(kThreads) k_update_multi(Launch L, ClassMap M,
                                                            const unsigned char* __restrict__ inPlace) {
@@ -813,6 +839,8 @@ struct Lib {
   size_t fluxCap = 0;
   double* pavg = nullptr; // library-owned face-averaged pressure arrays
   size_t pavgCap = 0;
+  double* upd = nullptr;  // updated states of a fused batch step (k_march's FUSE)
+  size_t updCap = 0;
   fx_tile* dtiles = nullptr;
   size_t dtilesCap = 0;
   fx_tile* dregTiles = nullptr;        // tile list of a register call
@@ -1056,6 +1084,36 @@ bool march_shape(const DevParams& P, int* TX, int* TY, int* NT) {
   }
   *NT = (P.ndim == 3 && *TX == 16) ? 512 : 256;
   return true;
+}
+
+// Whether a batch step runs the update inside the march: HLLC, HLL and the
+// hybrid switch, the whole pressure in the momentum flux (the update's
+// pressure source, which the fused form does not carry, is then zero), unless
+// the kernel path asks for a separate update.
+bool batch_fused(const DevParams& P) {
+  int TX, TY, NT;
+  return !g.legacy && !g.solveUpdOff && P.riemann != FX_EXACT && P.fP == 1.0 &&
+         march_shape(P, &TX, &TY, &NT);
+}
+
+// Where the update of n such blocks runs.  kFuseDirect gives a block's column
+// tiles to one workgroup in turn and saves k_update_finish: 6.10 against
+// 5.81 + 1.09 ms on 4096 x 16^3 (FP64), 2.08 against 1.85 + 0.51 on 2048 x
+// 16^3 (mixed), 6.58 against 6.32 + 0.58 on 16384 x 8^3.  It takes blocks one
+// column tile wide, no contact steepening (which reads planes that the update
+// has written by then), and a batch that fills the workgroups resident at a
+// time: whole blocks come in fewer, longer rounds than column tiles do, and
+// k_update_finish costs about an eighth of the march.  In 2-D the tiles are
+// short, and taking two in turn costs more than k_update_finish (4096 x 16^2
+// mixed: 190 against 152 + 25 us): blocks of one tile only.
+int batch_fuse_mode(const DevParams& P, int TX, int TY, long n) {
+  if (!batch_fused(P)) return kFuseNone;
+  const long tiles = P.nyb / TY;
+  if (P.nxb != TX || (P.ndim == 3 && P.steep) || (P.ndim == 2 && tiles > 1)) return kFuseScratch;
+  // resident workgroups: the FP64 16x8 tile takes a CU's LDS
+  const long slots = (long)g.numCU * (TX == 16 && P.precision != FX_PREC_MIXED ? 1 : 2);
+  const long direct = (n + slots - 1) / slots * tiles, scratch = (n * tiles + slots - 1) / slots;
+  return direct * 8 <= scratch * 9 ? kFuseDirect : kFuseScratch;
 }
 
 int grid_for(long items) {
@@ -1449,10 +1507,12 @@ void launch_face_solve(const DevParams& P, const FaceLaunch& F, long faces, bool
 // Flux stages of a step on the uploaded tiles (march path): the column march,
 // then the exact solver's face stage (records events 1 and 2).  Launches
 // only: scratch and work items are in place.
-int launch_flux_stages(int nTiles, double dt, int TX, int TY, bool solveUpdate = false) {
+int launch_flux_stages(int nTiles, double dt, int TX, int TY, bool solveUpdate = false,
+                       int fuse = kFuseNone) {
   const DevParams& P = g.cur;
   MarchLaunch M{g.dtiles, nTiles, g.multi ? 0 : P.nxb / TX,
-                g.multi ? 0 : (P.ndim > 1 ? P.nyb : 1) / TY, g.status, dt, nullptr, g.dtDev};
+                g.multi ? 0 : (P.ndim > 1 ? P.nyb : 1) / TY, g.status, dt, nullptr, g.dtDev,
+                fuse, fuse ? g.upd : nullptr};
   const dim3 grid((unsigned)(g.multi ? 1 : nTiles * M.tilesX * M.tilesY));
   if (P.riemann == FX_EXACT) {
     // exact solver: the march stores face states, a separate stage solves
@@ -1484,6 +1544,11 @@ int launch_flux_stages(int nTiles, double dt, int TX, int TY, bool solveUpdate =
     if (record(2)) return 4;
   }
   return 0;
+}
+
+void launch_update_finish(const DevParams& P, const fx_tile* tiles, int nTiles, const double* upd) {
+  hipLaunchKernelGGL(k_update_finish, dim3(grid_for(P.icells * nTiles)), dim3(kThreads), 0, g.stream,
+                     P, tiles, nTiles, upd);
 }
 
 // update stage of a step on the uploaded tiles (dIn: per-tile in-place flags
@@ -1592,8 +1657,11 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     if (solveUpdate && P.learned && ensure_seed_patch(g.hfaceStart[nTiles], nTiles, st)) return 4;
     if (!g.capturing) hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
     if (record(0)) return 4;
-    if (launch_flux_stages(nTiles, dt, TX, TY, solveUpdate)) return 4;
-    if (!solveUpdate) launch_update(nTiles, dt, dIn);
+    const int fuse = tilesUploaded && !tiles && !inPlace && !g.multi
+                         ? batch_fuse_mode(P, TX, TY, nTiles) : kFuseNone;
+    if (launch_flux_stages(nTiles, dt, TX, TY, solveUpdate, fuse)) return 4;
+    if (fuse == kFuseScratch) launch_update_finish(P, g.dtiles, nTiles, g.upd);
+    else if (fuse == kFuseNone && !solveUpdate) launch_update(nTiles, dt, dIn);
     if (record(3)) return 4;
   } else {
   if (grow(&g.states, &g.statesCap, (size_t)P.scellsPerTile * kStateComps * nTiles, st)) return 4;
@@ -1746,7 +1814,10 @@ int prepare_batch(double* U, long nBlocks, long blockStride, const double del[3]
       for (int d = 0; d < 3; ++d) t.del[d] = del[d];
       t.level = 1;
     }
-    if (upload_tiles(tl.data(), (int)nBlocks, true, st, false)) return 4;
+    // a fused step keeps no fluxes in memory, only the updated states
+    const bool fused = batch_fused(g.dp);
+    if (fused && grow(&g.upd, &g.updCap, (size_t)(kUpdComps * g.dp.icells * nBlocks), st)) return 4;
+    if (upload_tiles(tl.data(), (int)nBlocks, !fused, st, false)) return 4;
     g.batchU = U;
     g.batchN = nBlocks;
     g.batchStride = blockStride;
@@ -2075,7 +2146,7 @@ int fx_hydro_init(const fx_params* p) {
 }
 
 void fx_hydro_finalize(void) {
-  void* bufs[] = {g.strongList, g.strongCount, g.dwCell, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.dtiles, g.dinplace, g.status, g.partial,
+  void* bufs[] = {g.strongList, g.strongCount, g.dwCell, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.upd, g.dtiles, g.dinplace, g.status, g.partial,
                   g.dregTiles, g.dfaces, g.mlpPacked, g.seedPacked, g.seedY, g.fstates,
                   g.dnbr, g.dtBuf, g.dcls, g.dtcls, g.dcellStart, g.dfaceStart,
                   g.ditems, g.dregCls, g.seedFlux, g.seedBits};
@@ -2166,16 +2237,21 @@ int fx_hydro_advance_batch_noalloc(double* U, long nBlocks, long blockStride,
                      reinterpret_cast<double*>(s + Lay.flux), P.nface[0], P.nface[1], P.nface[2],
                      P.ndim, reinterpret_cast<double*>(s + Lay.pavg), P.icells);
   hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, status);
+  // the updated states of a fused step take the place of its fluxes
+  const int fuse = batch_fuse_mode(P, TX, TY, nBlocks);
+  double* const upd = reinterpret_cast<double*>(s + Lay.flux);
   MarchLaunch M{tiles, (int)nBlocks, P.nxb / TX, (P.ndim > 1 ? P.nyb : 1) / TY, status, dt,
-                nullptr, nullptr};
+                nullptr, nullptr, fuse, upd};
   const dim3 grid((unsigned)(nBlocks * M.tilesX * M.tilesY));
   if (P.riemann == FX_HLLC) launch_march<FX_HLLC>(P, M, TX, grid);
   else launch_march<FX_HYBR>(P, M, TX, grid);
   Launch L{tiles, (int)nBlocks, nullptr, status, dt, nullptr};
-  if (P.ndim == 3)
+  if (fuse == kFuseScratch)
+    launch_update_finish(P, tiles, (int)nBlocks, upd);
+  else if (fuse == kFuseNone && P.ndim == 3)
     hipLaunchKernelGGL(k_update_cols, dim3(grid_for((long)P.nxb * P.nyb * nBlocks)),
                        dim3(kThreads), 0, g.stream, P, L, nullptr);
-  else
+  else if (fuse == kFuseNone)
     hipLaunchKernelGGL((k_update<false, false>), dim3(grid_for(P.icells * nBlocks)),
                        dim3(kThreads), 0, g.stream, P, L, nullptr);
   HIPCALL(hipGetLastError(), st);

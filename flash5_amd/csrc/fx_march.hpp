@@ -19,7 +19,9 @@
 //            the aux internal-energy fluxes, hy_getFaceFlux.F90) to the
 //            tile's flux arrays and the
 //            face-averaged pressure of each interior cell to pavg.
-// The conservative update then runs as k_update from those arrays.
+// The conservative update then runs as k_update from those arrays; or, where
+// the call keeps no fluxes (batch steps), stage C leaves the fluxes in LDS and
+//   stage D  beside the next plane's stage B, updates the plane's cells.
 // x/y states exist for interior planes only; z states for planes lo-1..hi+1.
 
 #pragma once
@@ -41,14 +43,24 @@ template <int TX, int TY> struct TileIdx {
   static __device__ __forceinline__ int ly(int a, int b) { return (b + 2) * TX + a; }
   static constexpr int NRX = TX * (TY + 2), NRY = (TX + 2) * TY, NC = (TX + 2) * (TY + 2);
   static constexpr int NLX = (TX + 4) * TY, NLY = TX * (TY + 4);
+  // x faces: a in [0, TX], b in [0, TY); y faces: a in [0, TX), b in [0, TY]
+  static __device__ __forceinline__ int ux(int a, int b) { return b * (TX + 1) + a; }
+  static __device__ __forceinline__ int uy(int a, int b) { return b * TX + a; }
+  static constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1);
   // stage-A items along x: the cells of R_x and of the x slopes, rows
   // b = -1, [0,TY), TY; along y: the cells of R_y and of the y slopes,
   // rows b = -2, -1, [0,TY), TY, TY+1
   static constexpr int NUX = 2 * TX + (TX + 4) * TY, NUY = 4 * TX + (TX + 2) * TY;
 };
 
-// LDS of one column tile (march_tile), as offsets into one array of R
-template <int NDIM, int TX, int TY> struct MarchLds {
+// LDS of one column tile (march_tile), as offsets into one array of R.
+// FUSE: with the plane's face fluxes and face-averaged pressures.
+constexpr int kUpdFluxes = 7;  // face fluxes the update takes: all but the pressure slot
+// Where the update runs: in a kernel of its own, from flux arrays; in the
+// march, into scratch that k_update_finish spreads over the blocks; in the
+// march, into the blocks.
+enum : int { kFuseNone = 0, kFuseScratch = 1, kFuseDirect = 2 };
+template <int NDIM, int TX, int TY, int FUSE> struct MarchLds {
   using I = TileIdx<TX, TY>;
   static constexpr int NR = NDIM == 3 ? 3 : 1, NCOL = TX * TY, Z = NDIM == 3 ? 1 : 0;
   static constexpr int SX = 0;                                // sigma_x ring
@@ -64,10 +76,19 @@ template <int NDIM, int TX, int TY> struct MarchLds {
   static constexpr int WX = FZ + (Z ? 3 * NCOL : 1);          // x state cells' Wp
   static constexpr int WY = WX + 6 * I::NRY;                  // y state cells' Wp
   static constexpr int WZ = WY + 6 * I::NRX;                  // z state cells' Wp of the last plane done
-  static constexpr int PY = WZ + (Z ? 6 * NCOL : 1);          // Wn + Wp pressures of the y state cells
+  // (kept in registers where the fused FP64 8x8 tile would otherwise miss
+  // half a CU's LDS)
+  static constexpr bool WZ_LDS = Z && !(FUSE && TX == 8);
+  static constexpr int PY = WZ + (WZ_LDS ? 6 * NCOL : 1);     // Wn + Wp pressures of the y state cells
   static constexpr int PZ = PY + I::NRX;                      // and of the z state cells
   static constexpr int CST = PZ + (Z ? NCOL : 1);             // the step's ratios, widths
-  static constexpr int total = CST + 12;
+  // x-face fluxes; in 2-D over sigmas and slopes that stage B has done with
+  static constexpr int UX = Z ? CST + 12 : 0;
+  static constexpr int UY = UX + (FUSE ? kUpdFluxes * I::NFX : 0);  // y-face fluxes
+  static constexpr int UZ = UY + (FUSE ? kUpdFluxes * I::NFY : 0);  // z-face fluxes
+  static constexpr int PA = UZ + (FUSE && Z ? kUpdFluxes * NCOL : 0);  // face-averaged pressures
+  static constexpr int total = Z ? PA + (FUSE ? NCOL : 0) : CST + 12;
+  static_assert(Z || PA + NCOL <= FX, "the 2-D fluxes fit over the sigmas and slopes");
 };
 
 // components stored for sigma and slopes: dens, vx, vy, vz, pres, eint
@@ -81,7 +102,14 @@ struct MarchLaunch {
   double dt;
   void* fstates;       // RS_STATES: per-face states for the separate Riemann stage, in R
   const double* dtp;   // device-resident dt (graph-captured steps), or null
+  int fuse;            // where the update runs (kFuse*)
+  double* upd;         // fused update: updated states, [tile][component][interior cell]
 };
+// components of a cell's fused-update scratch: density, velocities, eint (the
+// sixth only in the FP32 march, on the way)
+constexpr int kUpdComps = 6;
+// rows below a column tile that its stages read (the guard layers of a block)
+constexpr int kSeamRows = 4;
 
 // Riemann-stage variant of the march: stage C stores each face's left and
 // right states (dens, vx, vy, vz, pres, eint) instead of solving there.
@@ -193,6 +221,12 @@ __device__ __forceinline__ void st_at(__attribute__((address_space(1))) T* base,
   *reinterpret_cast<__attribute__((address_space(1))) T*>(reinterpret_cast<gchar*>(base) + boff) = v;
 }
 
+template <typename T>
+__device__ __forceinline__ T ld_at(const __attribute__((address_space(1))) T* base, unsigned boff) {
+  return *reinterpret_cast<const __attribute__((address_space(1))) T*>(
+      reinterpret_cast<const gchar*>(base) + boff);
+}
+
 // The tile's primitives are read as one buffer (a scalar resource) with the
 // variable's byte offset in a scalar operand and the cell's in a vector
 // one, so no 64-bit address is formed per lane.  With 64-bit addresses the
@@ -204,6 +238,7 @@ struct TileView {
   __amdgpu_buffer_rsrc_t rs;  // the tile's guard-inclusive array
   unsigned ob[8];             // byte offsets of the primitive slots P_DENS .. P_EINT
   unsigned obShok;            // SHOK_VAR's (hybrid solver)
+  unsigned obEner;            // ENER_VAR's (fused update)
 };
 
 // The workgroup's tile is uniform; saying so (readfirstlane) keeps the
@@ -228,12 +263,18 @@ __device__ __forceinline__ TileView tile_view(const DevParams& P, const gdouble*
   tv.ob[P_GAMC] = fx_uniform((unsigned)P.voff[FX_GAMC] * 8u);
   tv.ob[P_GAME] = fx_uniform((unsigned)P.voff[FX_GAME] * 8u);
   tv.ob[P_EINT] = fx_uniform((unsigned)P.voff[FX_EINT] * 8u);
+  tv.obEner = fx_uniform((unsigned)P.voff[FX_ENER] * 8u);
   tv.obShok = fx_uniform(P.shokOff >= 0 ? (unsigned)P.shokOff * 8u : 0u);
   return tv;
 }
 // variable slot q (byte offset ob) of the cell at byte offset cb
 __device__ __forceinline__ double tv_ld(const TileView& tv, unsigned ob, unsigned cb) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(tv.rs, (int)cb, (int)ob, 0));
+}
+
+__device__ __forceinline__ void tv_st(const TileView& tv, unsigned ob, unsigned cb, double v) {
+  typedef unsigned v2u __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), tv.rs, (int)cb, (int)ob, 0);
 }
 
 // A stage's item number.  With OPAQUE it passes through an empty asm
@@ -251,6 +292,15 @@ __device__ __forceinline__ int item_index(int w) {
 // byte offset of cell (i, j, k) in its tile
 __device__ __forceinline__ unsigned cell_b(const DevParams& P, int i, int j, int k) {
   return (unsigned)((k * P.ny + j) * P.nx + i) * 8u;
+}
+
+// every variable of the updated cell at cb
+__device__ __forceinline__ void tv_expand(const DevParams& P, const TileView& tv, unsigned cb,
+                                          const UpdState& u) {
+  double out[10];
+  upd_expand(P, u, out);
+#pragma unroll
+  for (int v = 0; v < 10; ++v) tv_st(tv, fx_uniform((unsigned)P.voff[upd_var(v)] * 8u), cb, out[v]);
 }
 
 template <typename R>
@@ -298,6 +348,16 @@ __device__ __forceinline__ void write_flux_b(const DevParams& P, gdouble* Fo, un
   for (int q = 0; q < FX_NFLUX; ++q) st_at(Fo + q * nf, rb, F[q]);
 }
 
+// The march's barrier: a workgroup's threads exchange data through LDS alone
+// (the block's cells are only read, its outputs only written), so the LDS
+// accesses are waited for and the global ones stay in flight.  The plain
+// barrier also waits for every store to reach the cache, once per stage.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // One column tile (TX x TY columns at ox, oy, all planes) of tile t.  Every
 // thread of the workgroup calls it with the same arguments; it ends on a
 // barrier, so a workgroup may call it again for another column tile.  fsb:
@@ -323,12 +383,12 @@ __device__ __forceinline__ void write_flux_b(const DevParams& P, gdouble* Fo, un
 // tildes formed by the state cells) the step of 4096 x 16^3 went from 10.17
 // to 8.89 ms (FP64 HLLC), of 2048 x 16^3 from 3.41 to 3.07 ms (mixed) and of
 // 1024 x 16^3 from 3.52 to 3.15 ms (FP64 exact).
-template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE = (sizeof(R) == 4)>
-__device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch& L, int t, int ox,
-                                           int oy, R* fsb, ExactStats& es,
-                                           R* smem) {
+template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE, int FUSE>
+__device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch& L,
+                                           const fx_tile& T, int t, int ox, int oy, R* fsb,
+                                           ExactStats& es, R* smem) {
   using I = TileIdx<TX, TY>;
-  using M = MarchLds<NDIM, TX, TY>;
+  using M = MarchLds<NDIM, TX, TY, FUSE>;
   constexpr int NR = NDIM == 3 ? 3 : 1;        // ring depth
   constexpr int NCOL = TX * TY;
   constexpr int Z = NDIM == 3 ? 1 : 0;
@@ -346,16 +406,23 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   R* const WZ = smem + M::WZ;
   R* const PY = smem + M::PY;
   R* const PZ = smem + M::PZ;
+  R* const UX = smem + M::UX;
+  R* const UY = smem + M::UY;
+  R* const UZ = smem + M::UZ;
+  R* const PA = smem + M::PA;
 
   const int tid = threadIdx.x;
   // A tile owns its high x (y) face row only at the block's high side;
   // otherwise the neighbouring tile computes that row (and the states
-  // behind it) as its low row.
+  // behind it) as its low row.  The fused update needs that row's fluxes in
+  // either case, so there both tiles compute it.
   const bool ex = (ox + TX > P.hi[0]);
   const bool ey = (oy + TY > P.hi[1]);
-  const fx_tile& T = L.tiles[t];
   const TileView tv = tile_view(P, as_global(T.U));
-  const double dt = step_dt(L.dt, L.dtp);
+  double dt = step_dt(L.dt, L.dtp);
+  // (opaque: a workgroup that takes a block's tiles in turn would otherwise
+  // keep the ratios below live through all of them)
+  if constexpr (FUSE == kFuseDirect) asm volatile("" : "+v"(dt));
   const double dx = T.del[0], dy = T.del[1], dz = T.del[2];
   const unsigned sxb = 8u, syb = (unsigned)P.nx * 8u, szb = (unsigned)(P.nx * P.ny) * 8u;
   const int klo = P.lo[2], khi = P.hi[2];
@@ -492,6 +559,10 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * szb)), Vm[P_PRES], Vp[P_PRES],
                           R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * szb)), Vm[P_VELZ], Vp[P_VELZ]);
   };
+  // interior cell number within the tile's block
+  auto cell_r = [&](int i, int j, int k) -> unsigned {
+    return (unsigned)(((k - P.lo[2]) * P.nyb + (j - P.lo[1])) * P.nxb + (i - P.lo[0]));
+  };
   // FlatCoeff of the cell whose pressures across are pm, pp, from its own
   // tilde and its neighbours' (hy_getRiemannState.F90:408-453)
   auto flat_of = [&](R pm, R pp, R fm, R f0, R fp) -> R {
@@ -552,7 +623,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     }
   }
   stageA(kBeg);
-  __syncthreads();
+  lds_barrier();
 
   // roles of stages B and C, one state cell and one face per thread: x state
   // cells (a in [-1, TX], with the face below each), y ones (b in [-1, TY]),
@@ -566,9 +637,115 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   // Wn of the thread's state cell from stage B to C; in a column, Wp of the
   // plane below (the left state of the z face) as well, and the sum of the
   // state pressures for pavg in the x role
-  R Wk[6], Wo[6], psum = R(0.);
+  R Wk[6], Wo[6], Wt[6], psum = R(0.);
 #pragma unroll
-  for (int q = 0; q < 6; ++q) Wk[q] = Wo[q] = R(0.);
+  for (int q = 0; q < 6; ++q) Wk[q] = Wo[q] = Wt[q] = R(0.);
+
+  // ------------------------------ stage D ------------------------------
+  // The fused update: hy_unsplitUpdate, hy_energyFix and the EOS input of
+  // one column's cells from the fluxes in LDS, as update_cell takes them.
+  // Beside stage B of plane k it takes the x and y terms of the cell at plane
+  // k-1 and the z term of the one at plane k-2, whose upper face's flux
+  // stage C(k-1) left.  Where the block's cells are still to be read by other
+  // column tiles, the new state (density, velocities, eint: the rest follows
+  // from them) goes to scratch, to be spread later: every cell of
+  // kFuseScratch (k_update_finish), the top kSeamRows rows of a kFuseDirect
+  // tile with another above it (march_block).  The column's own planes are
+  // done with: no stage reads below plane k-1 by then (contact steepening
+  // does, and takes kFuseScratch).  The fluxes' way through memory (3.6 GB
+  // written, read back by an update of its own) cost 1.8 ms of 8.0 on 4096 x
+  // 16^3 in FP64; beside stage B, on wavefronts that have no state cell, the
+  // update costs 0.1 ms, and 0.25 with the stores into the blocks.
+  constexpr int D0 = (NT >= B3 + NCOL) ? B3 : 0;  // wavefronts without a role, if there are
+  // carried from plane to plane: the cell after its x and y terms, its
+  // face-averaged pressure, the flux through its lower z face.  The FP32
+  // march carries the FP64 ones through the cell's scratch (kUpdComps
+  // components, final values over them): in registers they would take it past
+  // the 128 that two workgroups on a CU leave, and with one workgroup the
+  // march of 2048 x 16^3 takes 2.50 ms; asking the compiler for 4 waves per
+  // SIMD instead makes it load in small batches (2.76 ms).
+  constexpr bool CARRY = sizeof(R) == 8;
+  double cU[5] = {0., 0., 0., 0., 0.}, cI = 0.;
+  R cP = R(0.), zlow[kUpdFluxes];
+#pragma unroll
+  for (int q = 0; q < kUpdFluxes; ++q) zlow[q] = R(0.);
+  auto put_flux = [](R* U, int n, int idx, const double F[8]) {
+#pragma unroll
+    for (int q = 0; q < kUpdFluxes; ++q) U[q * n + idx] = R(F[q < 5 ? q : q + 1]);
+  };
+  auto get_flux = [](const R* U, int n, int idx, double F[8]) {
+#pragma unroll
+    for (int q = 0; q < kUpdFluxes; ++q) F[q < 5 ? q : q + 1] = double(U[q * n + idx]);
+    F[5] = 0.;
+  };
+  auto stageD = [&](int k) {
+    const int w = item_index<OPAQUE>(tid) - D0;
+    if (w < 0 || w >= NCOL) return;
+    const int a = w % TX, b = w / TX;
+    double F0[8], F1[8];
+    double S;  // the pressure source: zero (the whole pressure is in the flux)
+    gdouble* const upd = as_global(L.upd + (long)t * (kUpdComps * P.icells));
+    auto put_new = [&](int kk, double eintOld) {
+      UpdPart part;
+#pragma unroll
+      for (int q = 0; q < 5; ++q) part.U0[q] = cU[q];
+      part.IntEner = cI;
+      part.S1 = part.S2 = 0.;
+      const UpdState u = upd_state(P, dt, part, eintOld);
+      if (FUSE == kFuseDirect && (b < TY - kSeamRows || ey)) {
+        tv_expand(P, tv, cell_b(P, ox + a, oy + b, kk), u);
+        return;
+      }
+      const unsigned r = cell_r(ox + a, oy + b, kk) * 8u;
+      st_at(upd, r, u.dens);
+      st_at(upd + P.icells, r, u.vx);
+      st_at(upd + 2 * P.icells, r, u.vy);
+      st_at(upd + 3 * P.icells, r, u.vz);
+      st_at(upd + 4 * P.icells, r, u.eint);
+    };
+    if (Z && k - 2 >= klo) {  // z term and the rest of plane k-2
+      if (!CARRY) {
+        const unsigned r = cell_r(ox + a, oy + b, k - 2) * 8u;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) cU[q] = ld_at(upd + q * P.icells, r);
+        cI = ld_at(upd + 5 * P.icells, r);
+      }
+#pragma unroll
+      for (int q = 0; q < kUpdFluxes; ++q) F0[q < 5 ? q : q + 1] = double(zlow[q]);
+      F0[5] = 0.;
+      get_flux(UZ, NCOL, w, F1);
+      upd_dir(P, dt, dz, double(cP), F0, F1, cU, cI, S);
+      put_new(k - 2, P.aux ? 0. : tv_ld(tv, tv.ob[P_EINT], cell_b(P, ox + a, oy + b, k - 2)));
+    }
+    const int kc = Z ? k - 1 : k;
+    if (kc >= klo && kc <= khi) {
+      const unsigned cb = cell_b(P, ox + a, oy + b, kc);
+      if (P.aux) cP = PA[w];
+      const UpdPart part = upd_init(P, tv_ld(tv, tv.ob[P_DENS], cb), tv_ld(tv, tv.ob[P_VELX], cb),
+                                    tv_ld(tv, tv.ob[P_VELY], cb), tv_ld(tv, tv.ob[P_VELZ], cb),
+                                    tv_ld(tv, tv.obEner, cb), tv_ld(tv, tv.ob[P_EINT], cb), 0.);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) cU[q] = part.U0[q];
+      cI = part.IntEner;
+      get_flux(UX, I::NFX, I::ux(a, b), F0);
+      get_flux(UX, I::NFX, I::ux(a + 1, b), F1);
+      upd_dir(P, dt, dx, double(cP), F0, F1, cU, cI, S);
+      get_flux(UY, I::NFY, I::uy(a, b), F0);
+      get_flux(UY, I::NFY, I::uy(a, b + 1), F1);
+      upd_dir(P, dt, dy, double(cP), F0, F1, cU, cI, S);
+      if (Z && !CARRY) {
+        const unsigned r = cell_r(ox + a, oy + b, kc) * 8u;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) st_at(upd + q * P.icells, r, cU[q]);
+        st_at(upd + 5 * P.icells, r, cI);
+      }
+      if (!Z) put_new(kc, tv_ld(tv, tv.ob[P_EINT], cb));
+    }
+    if (Z) {
+#pragma unroll
+      for (int q = 0; q < kUpdFluxes; ++q) zlow[q] = UZ[q * NCOL + w];
+    }
+  };
 
   for (int k = kBeg; k <= kEnd; ++k) {
     const bool interior = !Z || (k >= klo && k <= khi);
@@ -587,8 +764,9 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
         if (w < B1) {
           if (!interior || w >= NBX) return;
           const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-          if (a == TX && !ex) return;
-          const bool own = a >= 0 || ox == P.lo[0];  // (counts its reset)
+          if (a == TX && !ex && !FUSE) return;
+          // the tile owns this state cell (and counts its reset)
+          const bool own = (a >= 0 || ox == P.lo[0]) && (a < TX || ex);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - sxb, Vm);
           tv_prim(tv, cb, Vc);
@@ -631,8 +809,8 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const int w2 = w - B1;
           if (!interior || w2 >= NBY) return;
           const int a = w2 % TX, b = w2 / TX - 1;
-          if (b == TY && !ey) return;
-          const bool own = b >= 0 || oy == P.lo[1];
+          if (b == TY && !ey && !FUSE) return;
+          const bool own = (b >= 0 || oy == P.lo[1]) && (b < TY || ey);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - syb, Vm);
           tv_prim(tv, cb, Vc);
@@ -709,15 +887,20 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           }
           // the column's Wp stays with its thread: last plane's out, this one's in
 #pragma unroll
-          for (int q = 0; q < 6; ++q) Wo[q] = WZ[q * NCOL + w2];
-          lds_put6(WZ, NCOL, w2, Wp);
+          for (int q = 0; q < 6; ++q) {
+            Wo[q] = M::WZ_LDS ? WZ[q * NCOL + w2] : Wt[q];
+            if (!M::WZ_LDS) Wt[q] = Wp[comp_slot(q)];
+          }
+          if (M::WZ_LDS) lds_put6(WZ, NCOL, w2, Wp);
           PZ[w2] = Wn[P_PRES] + Wp[P_PRES];
           keep(Wn);
         }
       };
+      // first, so that its stores are on their way during the state cell
+      if (FUSE && Z) stageD(k);
       itemB(item_index<OPAQUE>(tid));
     }
-    __syncthreads();
+    lds_barrier();
 
     // ------------------------------ stage C ------------------------------
     {
@@ -737,7 +920,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
         if (w < B1) {
           if (!interior || w >= NBX) return;
           const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-          if (a < 0 || (a == TX && !ex)) return;
+          if (a < 0 || (a == TX && !ex && !FUSE)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           if (P.aux && a < TX) {
             // face-averaged pressure (hy_getFaceFlux.F90:507-561 and the
@@ -745,8 +928,8 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             R pres = R(0.5) * psum;
             pres = pres * R(0.5) + PY[I::rx(a, b)] * R(0.25);
             if (Z) pres = div_const<6>(pres * R(4.0) + PZ[b * TX + a]);
-            const unsigned r = (unsigned)(((k - P.lo[2]) * P.nyb + (oy + b - P.lo[1])) * P.nxb + (ox + a - P.lo[0]));
-            st_at(as_global(T.pavg), r * 8u, double(pres));
+            if constexpr (FUSE) PA[b * TX + a] = pres;
+            else st_at(as_global(T.pavg), cell_r(ox + a, oy + b, k) * 8u, double(pres));
           }
           lds_get6(WX, I::NRY, I::ry(a - 1, b), VL);
           right(VR);
@@ -756,13 +939,14 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             write_face_states<0>(P, fsb + fstate_dir_offset(P, 0), fr, VL, VR);
           } else {
             if (face_flux<0, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - sxb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 0); return; }
-            write_flux_b<0>(P, as_global(T.flux[0]), fr * 8u, F);
+            if constexpr (FUSE) put_flux(UX, I::NFX, I::ux(a, b), F);
+            else write_flux_b<0>(P, as_global(T.flux[0]), fr * 8u, F);
           }
         } else if (w < B2) {
           const int w2 = w - B1;
           if (!interior || w2 >= NBY) return;
           const int a = w2 % TX, b = w2 / TX - 1;
-          if (b < 0 || (b == TY && !ey)) return;
+          if (b < 0 || (b == TY && !ey && !FUSE)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           lds_get6(WY, I::NRX, I::rx(a, b - 1), VL);
           right(VR);
@@ -772,7 +956,8 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             write_face_states<1>(P, fsb + fstate_dir_offset(P, 1), fr, VL, VR);
           } else {
             if (face_flux<1, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - syb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 1); return; }
-            write_flux_b<1>(P, as_global(T.flux[1]), fr * 8u, F);
+            if constexpr (FUSE) put_flux(UY, I::NFY, I::uy(a, b), F);
+            else write_flux_b<1>(P, as_global(T.flux[1]), fr * 8u, F);
           }
         } else if (Z && w < B3) {
           if (k < klo) return;
@@ -788,16 +973,49 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             write_face_states<2>(P, fsb + fstate_dir_offset(P, 2), fr, VL, VR);
           } else {
             if (face_flux<2, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - szb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 2); return; }
-            write_flux_b<2>(P, as_global(T.flux[2]), fr * 8u, F);
+            if constexpr (FUSE) put_flux(UZ, NCOL, w2, F);
+            else write_flux_b<2>(P, as_global(T.flux[2]), fr * 8u, F);
           }
         }
       };
       itemC(item_index<OPAQUE>(tid));
     }
     if (k < kEnd) stageA(k + 1);
-    __syncthreads();
+    lds_barrier();
+  }
+  if constexpr (FUSE != kFuseNone) {  // the last plane
+    stageD(Z ? kEnd + 1 : kEnd);
+    __syncthreads();  // (and the scratch rows reach the cache)
   }
   if (bad) report_error(st, 1, t, ox, oy, -1, -1);
+}
+
+// The column tiles of a block one column tile wide, in rising y, updated in
+// place (kFuseDirect).  A tile reads the block from kSeamRows rows below its
+// own up, so the top kSeamRows rows of each tile but the last wait in scratch
+// until the next tile is done.
+template <int NDIM, int TX, int TY, int NT, int RS, typename R>
+__device__ __forceinline__ void march_block(const DevParams& P, const MarchLaunch& L, int t,
+                                            ExactStats& es, R* smem) {
+  // read before anything is stored: scalar loads
+  const fx_tile T = L.tiles[t];
+  for (int ty = 0; ty < L.tilesY; ++ty) {
+    const int oy = P.lo[1] + ty * TY;
+    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseDirect>(P, L, T, t, P.lo[0], oy, nullptr, es, smem);
+    if (ty == 0) continue;
+    const TileView tv = tile_view(P, as_global(T.U));
+    const gdouble* const upd = as_global(L.upd + (long)t * (kUpdComps * P.icells));
+    const int j0 = oy - kSeamRows, items = P.nzb * kSeamRows * TX;
+    for (int w = threadIdx.x; w < items; w += NT) {
+      const int i = P.lo[0] + w % TX, j = j0 + (w / TX) % kSeamRows;
+      const int k = P.lo[2] + w / (TX * kSeamRows);
+      const unsigned r =
+          (unsigned)(((k - P.lo[2]) * P.nyb + (j - P.lo[1])) * P.nxb + (i - P.lo[0])) * 8u;
+      tv_expand(P, tv, cell_b(P, i, j, k),
+                UpdState{ld_at(upd, r), ld_at(upd + P.icells, r), ld_at(upd + 2 * P.icells, r),
+                         ld_at(upd + 3 * P.icells, r), ld_at(upd + 4 * P.icells, r)});
+    }
+  }
 }
 
 // One workgroup per column tile of a batch of equal-shape tiles.  OCC > 0
@@ -806,9 +1024,15 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
 // threads: its LDS allows one workgroup per CU, stage A has 12 wavefronts of
 // items, and 3 waves per SIMD leave 168 registers (at 512 threads the march
 // took 8.83 instead of 8.41 ms on 4096 x 16^3).
-template <int NDIM, int TX, int TY, int NT, int RS, typename R, int OCC = 0>
+template <int NDIM, int TX, int TY, int NT, int RS, typename R, int OCC = 0, int FUSE = kFuseNone>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 k_march(DevParams P, MarchLaunch L) {
+  if constexpr (FUSE == kFuseDirect) {  // one workgroup per block
+    ExactStats es{0ULL, 0ULL};
+    __shared__ R smem[MarchLds<NDIM, TX, TY, FUSE>::total];
+    march_block<NDIM, TX, TY, NT, RS, R>(P, L, (int)blockIdx.x, es, smem);
+    return;
+  }
   const int tilesPerBlock = L.tilesX * L.tilesY;
   const int t = blockIdx.x / tilesPerBlock;
   const int tr = blockIdx.x - t * tilesPerBlock;
@@ -816,8 +1040,8 @@ k_march(DevParams P, MarchLaunch L) {
   const int oy = P.lo[1] + (tr / L.tilesX) * TY;
   ExactStats es{0ULL, 0ULL};
   R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + t * fstate_tile_stride(P) : nullptr;
-  __shared__ R smem[MarchLds<NDIM, TX, TY>::total];
-  march_tile<NDIM, TX, TY, NT, RS, R, true>(P, L, t, ox, oy, fsb, es, smem);
+  __shared__ R smem[MarchLds<NDIM, TX, TY, FUSE>::total];
+  march_tile<NDIM, TX, TY, NT, RS, R, true, FUSE>(P, L, L.tiles[t], t, ox, oy, fsb, es, smem);
   flush_exact(L.status, es);
 }
 
@@ -837,13 +1061,13 @@ k_march_multi(const DevParams* __restrict__ cls,
                                                     const MarchItem* __restrict__ items,
                                                     int nItems, const long* __restrict__ faceStart) {
   ExactStats es{0ULL, 0ULL};
-  __shared__ R smem[MarchLds<NDIM, TX, TY>::total];
+  __shared__ R smem[MarchLds<NDIM, TX, TY, kFuseNone>::total];
   for (int it = blockIdx.x; it < nItems; it += gridDim.x) {
     const MarchItem w = items[it];
     const DevParams& P = cls[w.cls];
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
-    march_tile<NDIM, TX, TY, NT, RS, R, true>(P, L, w.t, w.ox, w.oy, fsb, es, smem);
+    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
   }
   flush_exact(L.status, es);
 }
@@ -856,15 +1080,16 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0
 k_march_mixw(const DevParams* __restrict__ cls, MarchLaunch L,
              const MarchItem* __restrict__ items, int nItems, const long* __restrict__ faceStart) {
   ExactStats es{0ULL, 0ULL};
-  constexpr int n16 = MarchLds<NDIM, 16, 8>::total, n8 = MarchLds<NDIM, 8, 8>::total;
+  constexpr int n16 = MarchLds<NDIM, 16, 8, kFuseNone>::total,
+                n8 = MarchLds<NDIM, 8, 8, kFuseNone>::total;
   __shared__ R smem[n16 > n8 ? n16 : n8];
   for (int it = blockIdx.x; it < nItems; it += gridDim.x) {
     const MarchItem w = items[it];
     const DevParams& P = cls[w.cls];
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
-    if (w.tx == 16) march_tile<NDIM, 16, 8, NT, RS, R, true>(P, L, w.t, w.ox, w.oy, fsb, es, smem);
-    else march_tile<NDIM, 8, 8, NT, RS, R, true>(P, L, w.t, w.ox, w.oy, fsb, es, smem);
+    if (w.tx == 16) march_tile<NDIM, 16, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
+    else march_tile<NDIM, 8, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
   }
   flush_exact(L.status, es);
 }

@@ -11,11 +11,12 @@
 
 namespace fx {
 
-template <int RS, typename R>
-void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
+// FUSE: with the update; RS_STATES has no fluxes to update from
+template <int RS, typename R, int FUSE>
+void launch_march_f(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
                     const MarchHost& H) {
   constexpr int OCC = sizeof(R) == 8 ? 3 : 0;  // waves per SIMD
-  if constexpr (sizeof(R) == 4) {  // FP32 3-D: the autotuner may ask for 4 waves per SIMD
+  if constexpr (sizeof(R) == 4 && !FUSE) {  // FP32 3-D: the autotuner may ask for 4 waves per SIMD
     if (P.ndim == 3 && H.tuneOcc == 4) {
       if (TX == 16)
         hipLaunchKernelGGL((k_march<3, 16, 8, 512, RS, R, 4>), grid, dim3(512), 0, H.stream, P, M);
@@ -25,10 +26,26 @@ void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
     }
   }
   constexpr int NT3 = sizeof(R) == 8 ? 768 : 512;  // FP64 3-D 16x8: 768 threads
-  if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, NT3, RS, R, OCC>), grid, dim3(NT3), 0, H.stream, P, M);
-  else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, OCC>), grid, dim3(384), 0, H.stream, P, M);
-  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, 384, RS, R, OCC>), grid, dim3(384), 0, H.stream, P, M);
-  else hipLaunchKernelGGL((k_march<2, 8, 8, 256, RS, R, OCC>), grid, dim3(256), 0, H.stream, P, M);
+  if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, NT3, RS, R, OCC, FUSE>), grid, dim3(NT3), 0, H.stream, P, M);
+  else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, OCC, FUSE>), grid, dim3(384), 0, H.stream, P, M);
+  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, 384, RS, R, OCC, FUSE>), grid, dim3(384), 0, H.stream, P, M);
+  else hipLaunchKernelGGL((k_march<2, 8, 8, 256, RS, R, OCC, FUSE>), grid, dim3(256), 0, H.stream, P, M);
+}
+
+template <int RS, typename R>
+void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
+                    const MarchHost& H) {
+  if constexpr (!is_states(RS)) {
+    if (M.fuse == kFuseDirect) {
+      launch_march_f<RS, R, kFuseDirect>(P, M, TX, dim3((unsigned)M.nTiles), H);
+      return;
+    }
+    if (M.fuse == kFuseScratch) {
+      launch_march_f<RS, R, kFuseScratch>(P, M, TX, grid, H);
+      return;
+    }
+  }
+  launch_march_f<RS, R, kFuseNone>(P, M, TX, grid, H);
 }
 
 // Persistent multi-class march: as many workgroups as stay resident (or
