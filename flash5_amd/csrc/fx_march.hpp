@@ -199,9 +199,10 @@ __device__ __forceinline__ R flat_tilde_vals(R pm2, R pm1, R pp1, R pp2, R vm1, 
   const R dp1 = (pp1 - pm1);
   const R dp2 = (pp2 - pm2);
   const R dv1 = vp1 - vm1;
-  const R Sp = (fabs(dp2) > R(1.e-15)) ? dp1 / dp2 - R(0.75) : R(0.);
+  const R qp = quot(dp1, dp2);
+  const R Sp = (fabs(dp2) > R(1.e-15)) ? qp - R(0.75) : R(0.);
   R ft = fmax(R(0.0), fmin(R(1.0), R(10.0) * Sp));
-  if ((fabs(dp1) / fmin(pm1, pp1) < R(1.) / R(3.)) || dv1 > R(0.)) ft = R(0.);
+  if ((quot(fabs(dp1), fmin(pm1, pp1)) < R(1.) / R(3.)) || dv1 > R(0.)) ft = R(0.);
   return ft;
 }
 
