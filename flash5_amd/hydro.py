@@ -119,6 +119,8 @@ EXPORTS = {
     "fx_hydro_set_seed_params": ([C.POINTER(C.c_float)], C.c_int),
     "fx_mlp_set_gate": ([C.c_double], C.c_int),
     "fx_hydro_face_states": ([_DP, C.c_long, C.POINTER(C.c_long)], C.c_int),
+    "fx_grid_fill_guards_var": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_int,
+                                 C.POINTER(FxStatus)], C.c_int),
     "fx_grid_fill_guards": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.POINTER(FxStatus)],
                             C.c_int),
     "fx_grid_run_graph": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_double * 3, C.c_double,

@@ -288,6 +288,10 @@ enum { FX_BC_OUTFLOW = -1,   /* zero gradient */
        FX_BC_REFLECT = -2 }; /* mirror, normal velocity negated */
 int fx_grid_fill_guards(double* U, long nBlocks, long blockStride, const int* nbr,
                         fx_status* st);
+/* The same for the variable slot var alone (< 0: every variable): after the
+ * shock detector only SHOK_VAR's guard cells are out of date. */
+int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int* nbr, int var,
+                            fx_status* st);
 
 /* Whole steps of a uniform grid captured in a HIP graph: each captured step
  * fills the guard cells (as fx_grid_fill_guards), computes the CFL dt on
