@@ -896,6 +896,7 @@ struct Lib {
   unsigned char* dregCls = nullptr;    // tile classes of a register call
   size_t dregClsCap = 0;
   std::vector<unsigned char> hregCls;
+  float* gradPart = nullptr;           // k_mlp_grad's rows, one per workgroup
   MlpPacked* mlpPacked = nullptr;      // BF16 fragments for fx_mlp_* / fx_riemann_batch
   MlpPacked* seedPacked = nullptr;     // network seeding the exact solver in hydro steps
   bool seedReady = false;
@@ -2199,7 +2200,7 @@ int fx_hydro_init(const fx_params* p) {
 
 void fx_hydro_finalize(void) {
   void* bufs[] = {g.strongList, g.strongCount, g.dwCell, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.upd, g.dtiles, g.dinplace, g.status, g.partial,
-                  g.dregTiles, g.dfaces, g.mlpPacked, g.seedPacked, g.seedY, g.fstates,
+                  g.dregTiles, g.dfaces, g.mlpPacked, g.gradPart, g.seedPacked, g.seedY, g.fstates,
                   g.dnbr, g.dtBuf, g.dcls, g.dtcls, g.dcellStart, g.dfaceStart,
                   g.ditems, g.dregCls, g.seedFlux, g.seedBits};
   for (void* b : bufs)
@@ -2400,8 +2401,16 @@ int fx_mlp_grad(const float* params, const float* x, const float* t, long n, flo
   if (n <= 0) return 0;
   if (!params || !x || !t || !grad || !loss) return 3;
   if (ensure_status(nullptr) || pack_mlp(params, &g.mlpPacked, nullptr)) return 4;
-  hipLaunchKernelGGL(k_mlp_grad, wave_grid(n), dim3(kLearnThreads), 0, g.stream, g.mlpPacked, x,
-                     t, n, scale, grad, loss);
+  // one workgroup per CU at most
+  if (!g.gradPart &&
+      hipMalloc((void**)&g.gradPart, sizeof(float) * kGradStride * g.numCU) != hipSuccess)
+    return 4;
+  const long per = kGradWaves * kGradCols;
+  const unsigned rows = (unsigned)std::min((n + per - 1) / per, (long)g.numCU);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(kGradWaves * 64), 0, g.stream, g.mlpPacked, x, t,
+                     n, scale, g.gradPart);
+  hipLaunchKernelGGL(k_mlp_grad_sum, dim3(MLP_NPARAM / 64 + 1), dim3(kThreads), 0, g.stream,
+                     g.gradPart, (int)rows, grad, loss);
   return sync_or_async(nullptr);
 }
 

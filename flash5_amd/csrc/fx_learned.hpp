@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(kLearnThreads) k_mlp_forward(const MlpPacked* 
     const long i = base + lane;
     const bool act = i < n;
     stage_x(x, n, i, act, xs[wv], lane);
-    MlpActs A;
+    MlpActs<4> A;
     float yo;
     mlp_forward_wave(*W, xs[wv], lane, A, yo);
     if (act) y[i] = yo;
@@ -62,32 +62,100 @@ __global__ void __launch_bounds__(kLearnThreads) k_mlp_forward(const MlpPacked* 
   }
 }
 
-// grad += d/dparams of scale * sum (y - t)^2 ; loss += scale * sum (y - t)^2
-__global__ void __launch_bounds__(kLearnThreads) k_mlp_grad(const MlpPacked* __restrict__ W,
-                                                            const float* __restrict__ x,
-                                                            const float* __restrict__ t, long n,
-                                                            float scale, float* grad, float* loss) {
-  __shared__ float xs[kLearnWaves][64 * 8];
-  // 16-byte aligned: the weight-gradient products read 8 bf16 at a time
-  __shared__ __attribute__((aligned(16))) unsigned short sZ[kLearnWaves][64 * 64];
-  __shared__ __attribute__((aligned(16))) unsigned short sH[kLearnWaves][64 * 64];
-  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
-  const long nw = (long)gridDim.x * kLearnWaves;
+// d/dparams of scale * sum (y - t)^2 and, after the MLP_NPARAM parameters, the
+// sum itself: each workgroup stores one row of part; k_mlp_grad_sum adds the
+// rows.  A wavefront takes 32 interfaces (64: twice as long, and it spills).
+// 8192 of them: an atomic per wavefront and parameter on the gradient itself
+// 114 us, nearly all of it atomics on the same 4673 words; FP32 LDS atomics (some
+// 125 cycles each) and rows 33 us; sums in registers and rows 11 us, with 4 us
+// for k_mlp_grad_sum.  65536 of them 20 us, 262144 59 us.
+constexpr int kGradStride = 4736;           // row of part, 64-float multiples
+constexpr int kGradSegs = kThreads / 64;    // k_mlp_grad_sum: rows split over wavefronts
+__global__ void __launch_bounds__(kGradWaves * 64) k_mlp_grad(const MlpPacked* __restrict__ W,
+                                                              const float* __restrict__ x,
+                                                              const float* __restrict__ t, long n,
+                                                              float scale,
+                                                              float* __restrict__ part) {
+  __shared__ float xs[kGradWaves][kGradCols * 8];
+  __shared__ __attribute__((aligned(16))) __bf16 sZ[64 * kGradRow];
+  __shared__ __attribute__((aligned(16))) __bf16 sH[64 * kGradRow];
+  __shared__ float sU[kGradWaves][64][16];   // MlpGradAcc::unit by unit
+  __shared__ float sB[kGradWaves][2];        // b3, loss
+  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64, g = lane / 16, c = lane % 16;
+  MlpGradAcc acc{};
   float lsum = 0.f;
-  for (long base = ((long)blockIdx.x * kLearnWaves + wv) * 64; base < n; base += nw * 64) {
-    const long i = base + lane;
-    const bool act = i < n;
-    stage_x(x, n, i, act, xs[wv], lane);
-    MlpActs A;
+  for (long base = (long)blockIdx.x * (kGradWaves * kGradCols); base < n;
+       base += (long)gridDim.x * (kGradWaves * kGradCols)) {
+    const long i = base + wv * kGradCols + lane;
+    const bool act = lane < kGradCols && i < n;
+    if (lane < kGradCols) stage_x(x, n, i, act, xs[wv], lane);
+    wave_lds_sync();
+    MlpActs<kGradNT> A;
     float yo;
     mlp_forward_wave(*W, xs[wv], lane, A, yo);
     const float r = act ? yo - t[i] : 0.f;
     lsum += scale * r * r;
-    mlp_backward_wave(*W, xs[wv], lane, A, 2.f * scale * r, sZ[wv], sH[wv], grad);
+    mlp_backward_wave(*W, xs[wv], lane, A, 2.f * scale * r, sZ + wv * kGradCols,
+                      sH + wv * kGradCols, acc);
+    __syncthreads();
+    mlp_grad_w2(wv, lane, sZ, sH, acc);
+    __syncthreads();
+  }
+  float b3 = acc.b3;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    lsum += __shfl_xor(lsum, o);
+    b3 += __shfl_xor(b3, o);
+  }
+  if (lane == 0) {
+    sB[wv][0] = b3;
+    sB[wv][1] = lsum;
   }
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) lsum += __shfl_xor(lsum, o);
-  if (lane == 0) atomicAdd(loss, lsum);
+  for (int q = 0; q < 16; ++q) sU[wv][16 * (q / 4) + 4 * g + q % 4][c] = acc.unit[q];
+  __syncthreads();
+  float* const row = part + (long)blockIdx.x * kGradStride;
+#pragma unroll
+  for (int ut = 0; ut < 4; ++ut)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      row[OFF_W2 + (16 * wv + 4 * g + i) * MLP_H + 16 * ut + c] = acc.w2[ut][i];
+  for (int e = threadIdx.x; e < 64 * 16; e += kGradWaves * 64) {
+    const int u = e / 16, q = e % 16;
+    if (q > 8) continue;
+    float v = sU[0][u][q];
+#pragma unroll
+    for (int w = 1; w < kGradWaves; ++w) v += sU[w][u][q];
+    row[q < MLP_IN ? OFF_W1 + u * MLP_IN + q
+                   : (q == 6 ? OFF_B1 : (q == 7 ? OFF_B2 : OFF_W3)) + u] = v;
+  }
+  if (threadIdx.x < 2) {
+    float v = sB[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kGradWaves; ++w) v += sB[w][threadIdx.x];
+    row[threadIdx.x == 0 ? OFF_B3 : MLP_NPARAM] = v;
+  }
+}
+
+// grad += and loss += the sums of part's rows
+__global__ void __launch_bounds__(kThreads) k_mlp_grad_sum(const float* __restrict__ part, int rows,
+                                                           float* grad, float* loss) {
+  __shared__ float seg[kGradSegs][64];
+  const int lane = threadIdx.x % 64, s = threadIdx.x / 64;
+  const int k = blockIdx.x * 64 + lane;
+  float v = 0.f;
+  if (k <= MLP_NPARAM) {
+#pragma unroll 8
+    for (int r = s; r < rows; r += kGradSegs) v += part[(long)r * kGradStride + k];
+  }
+  seg[s][lane] = v;
+  __syncthreads();
+  if (s == 0 && k <= MLP_NPARAM) {
+#pragma unroll
+    for (int q = 1; q < kGradSegs; ++q) v += seg[q][lane];
+    if (k == MLP_NPARAM) *loss += v;
+    else grad[k] += v;
+  }
 }
 
 __global__ void __launch_bounds__(kThreads) k_mlp_adam(float* __restrict__ prm,
@@ -137,7 +205,7 @@ __global__ void __launch_bounds__(kLearnThreads) k_mlp_seed_states(
     xs[wv][lane * 8 + 6] = 0.f;
     xs[wv][lane * 8 + 7] = 0.f;
     wave_lds_sync();
-    MlpActs A;
+    MlpActs<4> A;
     float yo;
     mlp_forward_wave(*W, xs[wv], lane, A, yo);
     if (act) y[i] = yo;
@@ -537,7 +605,7 @@ __global__ void __launch_bounds__(kLearnThreads) k_face_seed(DevParams P0, FaceL
     xs[wv][lane * 8 + 6] = 0.f;
     xs[wv][lane * 8 + 7] = 0.f;
     wave_lds_sync();
-    MlpActs A;
+    MlpActs<4> A;
     float yo;
     mlp_forward_wave(*W, xs[wv], lane, A, yo);
     if (act) y[gid] = yo;

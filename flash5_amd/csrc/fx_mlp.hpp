@@ -34,23 +34,24 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) unsigned short u16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-__device__ __forceinline__ unsigned short f2bf(float f) {  // round to nearest even
-  unsigned u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
-
+// round to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ bf16x8 to_bf16x8(const float v[8]) {
-  u16x8 h;
+  bf16x8 h;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) h[j] = f2bf(v[j]);
-  return __builtin_bit_cast(bf16x8, h);
+  for (int j = 0; j < 8; ++j) h[j] = (__bf16)v[j];
+  return h;
 }
 
 // tanh from the hardware exponential: 1 - 2 / (exp(2x) + 1), saturating to
-// +-1 at both ends; a few ulp in FP32, ample for a Newton seed
+// +-1 at both ends; a few ulp in FP32, ample for a Newton seed.  The powers of
+// two are exact wherever they stand, so the first joins exp's log2(e) and the
+// second an FMA; a reciprocal below 2^-25 leaves 1 whatever its value, so no
+// operand needs scaling.  Inference is bound by these two quarter-rate
+// operations (12 instructions a unit -> 6: 4M interfaces 311 -> 236 us,
+// with v_cvt_pk_bf16_f32 for the operands).
 __device__ __forceinline__ float act_tanh(float x) {
-  return 1.f - __fdividef(2.f, __expf(2.f * x) + 1.f);
+  const float e = __builtin_amdgcn_exp2f(x * (2.f * 1.4426950408889634f));
+  return fmaf(-2.f, __builtin_amdgcn_rcpf(e + 1.f), 1.f);
 }
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -114,20 +115,22 @@ __device__ __forceinline__ void mlp_features(double g, double rl, double ul, dou
   x[3] = -hr; x[4] = -hp; x[5] = hu;
 }
 
-// Activations of one wavefront (64 interfaces): result tile [mt][nt] of
+// Activations of one wavefront (16 NT interfaces): result tile [mt][nt] of
 // each layer, 4 floats per lane (column 16nt + l%16, rows 16mt + 4g + i).
-struct MlpActs {
-  f32x4 h1[4][4];
-  f32x4 h2[4][4];
+template <int NT> struct MlpActs {
+  f32x4 h1[4][NT];
+  f32x4 h2[4][NT];
 };
 
-// xs: this wavefront's LDS block of 64 x 8 floats (features 0..5 used)
+// xs: this wavefront's LDS block of 16 NT x 8 floats (features 0..5 used);
+// yOut: interface lane's value in the first 16 NT lanes
+template <int NT>
 __device__ __forceinline__ void mlp_forward_wave(const MlpPacked& W, const float* xs, int lane,
-                                                 MlpActs& A, float& yOut) {
+                                                 MlpActs<NT>& A, float& yOut) {
   const int g = lane / 16, c = lane % 16;
-  bf16x8 bx[4];
+  bf16x8 bx[NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (g == 0 && j < MLP_IN) ? xs[(16 * nt + c) * 8 + j] : 0.f;
@@ -137,7 +140,7 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpPacked& W, const float
   for (int mt = 0; mt < 4; ++mt) {
     const bf16x8 a = W.w1[mt * 64 + lane];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       f32x4 d = mfma(a, bx[nt], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
       for (int i = 0; i < 4; ++i) d[i] = act_tanh(d[i] + W.b1[16 * mt + 4 * g + i]);
@@ -146,7 +149,7 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpPacked& W, const float
   }
   // layer 2: K = 64 as two K=32 steps over result tiles (2ks, 2ks+1)
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     bf16x8 b[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -168,9 +171,9 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpPacked& W, const float
     }
   }
   // layer 3 (64 -> 1) on the VALU: partial dot products, then across groups
-  float part[4];
+  float part[NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     float s = 0.f;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
@@ -183,7 +186,7 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpPacked& W, const float
   // interface n = lane: its sum sits in part[n/16] of lane n%16
   float y = 0.f;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     const float v = __shfl(part[nt], c);
     if (g == nt) y = v;
   }
@@ -198,31 +201,52 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// sum over the 16 lanes of a lane group (same g)
+// sum over the 16 lanes of a lane group (same g), a DPP row: pairs, quads by
+// permuting within four lanes, then eights and the row by mirroring
+template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                           0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
 __device__ __forceinline__ float group_sum(float v) {
-  v += __shfl_xor(v, 1);
-  v += __shfl_xor(v, 2);
-  v += __shfl_xor(v, 4);
-  v += __shfl_xor(v, 8);
-  return v;
+  v = dpp_add<0xB1>(v);    // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E>(v);    // quad_perm [2,3,0,1]
+  v = dpp_add<0x141>(v);   // row_half_mirror
+  return dpp_add<0x140>(v);   // row_mirror
 }
 
-// Gradient of sum_n dy[n] * y[n] with respect to every parameter, added to
-// grad (global FP32) with atomics.  dy: this lane's interface (0 for lanes
-// without one).  sZ, sH: this wavefront's LDS scratch, 64*64 bf16 each.
+// Gradient of sum_n dy[n] * y[n] with respect to the parameters, one workgroup
+// on kGradWaves * kGradCols interfaces at a time; every sum stays in registers
+// from one set to the next.
+constexpr int kGradNT = 2, kGradCols = 16 * kGradNT;   // interfaces of a wavefront
+constexpr int kGradWaves = 4;                          // = the row tiles of W2
+// rows of the bf16 operands of dW2, padded: 16-byte reads, and the four lane
+// groups' writes fall into different banks
+constexpr int kGradRow = kGradWaves * kGradCols + 8;
+struct MlpGradAcc {
+  f32x4 w2[4];      // dW2 rows 16 wave + 4g + i, columns 16ut + c, of all wavefronts' interfaces
+  float unit[16];   // unit 16mt + 4g + i at [4mt + i], this wavefront's interfaces: lanes
+                    // c = 0..5 dW1, 6 db1, 7 db2, 8 dw3
+  float b3;         // each lane's own
+};
+
+// This wavefront's part; dZ2 and H1 go to sZ and sH (64 rows of kGradRow, this
+// wavefront's columns) for mlp_grad_w2.  dy: this lane's interface (0 for lanes
+// without one).
 __device__ __forceinline__ void mlp_backward_wave(const MlpPacked& W, const float* xs, int lane,
-                                                  const MlpActs& A, float dy, unsigned short* sZ,
-                                                  unsigned short* sH, float* grad) {
+                                                  const MlpActs<kGradNT>& A, float dy, __bf16* sZ,
+                                                  __bf16* sH, MlpGradAcc& acc) {
+  constexpr int NT = kGradNT;
   const int g = lane / 16, c = lane % 16;
-  float dyc[4];
+  float dyc[NT], x[NT][MLP_IN];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) dyc[nt] = __shfl(dy, 16 * nt + c);
-  float b3 = dy;
+  for (int nt = 0; nt < NT; ++nt) {
+    dyc[nt] = __shfl(dy, 16 * nt + c);
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) b3 += __shfl_xor(b3, o);
-  if (lane == 0) atomicAdd(&grad[OFF_B3], b3);
+    for (int f = 0; f < MLP_IN; ++f) x[nt][f] = xs[(16 * nt + c) * 8 + f];
+  }
+  acc.b3 += dy;
   // output layer and layer-2 pre-activation gradient
-  f32x4 dz2[4][4];
+  f32x4 dz2[4][NT];
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -230,24 +254,23 @@ __device__ __forceinline__ void mlp_backward_wave(const MlpPacked& W, const floa
       const int u = 16 * mt + 4 * g + i;
       float s3 = 0.f, s2 = 0.f;
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
+      for (int nt = 0; nt < NT; ++nt) {
         const float h = A.h2[mt][nt][i];
         const float z = W.w3[u] * dyc[nt] * (1.f - h * h);
         dz2[mt][nt][i] = z;
         s3 += dyc[nt] * h;
         s2 += z;
+        sZ[u * kGradRow + 16 * nt + c] = (__bf16)z;
+        sH[u * kGradRow + 16 * nt + c] = (__bf16)A.h1[mt][nt][i];
       }
-      s3 = group_sum(s3);
       s2 = group_sum(s2);
-      if (c == 0) {
-        atomicAdd(&grad[OFF_W3 + u], s3);
-        atomicAdd(&grad[OFF_B2 + u], s2);
-      }
+      s3 = group_sum(s3);
+      acc.unit[4 * mt + i] += c == 7 ? s2 : (c == 8 ? s3 : 0.f);
     }
   // dH1 = W2^T dZ2, chained from the dz2 tiles
-  f32x4 dh1[4][4];
+  f32x4 dh1[4][NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     bf16x8 b[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -270,58 +293,41 @@ __device__ __forceinline__ void mlp_backward_wave(const MlpPacked& W, const floa
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int u = 16 * mt + 4 * g + i;
-      float sb = 0.f, sw[MLP_IN] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      float sum[MLP_IN + 1] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
+      for (int nt = 0; nt < NT; ++nt) {
         const float h = A.h1[mt][nt][i];
         const float z = dh1[mt][nt][i] * (1.f - h * h);
-        sb += z;
+        sum[MLP_IN] += z;
 #pragma unroll
-        for (int f = 0; f < MLP_IN; ++f) sw[f] += z * xs[(16 * nt + c) * 8 + f];
+        for (int f = 0; f < MLP_IN; ++f) sum[f] += z * x[nt][f];
       }
-      sb = group_sum(sb);
-      if (c == 0) atomicAdd(&grad[OFF_B1 + u], sb);
+      float mine = 0.f;
 #pragma unroll
-      for (int f = 0; f < MLP_IN; ++f) {
-        const float v = group_sum(sw[f]);
-        if (c == 0) atomicAdd(&grad[OFF_W1 + u * MLP_IN + f], v);
+      for (int f = 0; f <= MLP_IN; ++f) {
+        const float v = group_sum(sum[f]);
+        mine = c == f ? v : mine;
       }
+      acc.unit[4 * mt + i] += mine;
     }
-  // dW2[o][in] = sum_n dZ2[o][n] H1[in][n]: transpose both through LDS
+}
+
+// dW2[o][in] += sum_n dZ2[o][n] H1[in][n] over the workgroup's interfaces:
+// wavefront wv takes rows 16 wv .. 16 wv + 15.
+__device__ __forceinline__ void mlp_grad_w2(int wv, int lane, const __bf16* sZ, const __bf16* sH,
+                                            MlpGradAcc& acc) {
+  const int g = lane / 16, c = lane % 16;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int ks = 0; ks < kGradWaves * kGradCols / 32; ++ks) {
+    const bf16x8 az =
+        *reinterpret_cast<const bf16x8*>(&sZ[(16 * wv + c) * kGradRow + 32 * ks + 8 * g]);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int u = 16 * mt + 4 * g + i, n = 16 * nt + c;
-        sZ[u * 64 + n] = f2bf(dz2[mt][nt][i]);
-        sH[u * 64 + n] = f2bf(A.h1[mt][nt][i]);
-      }
-  wave_lds_sync();
-  bf16x8 bh[2][4];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-      bh[ks][nt] = *reinterpret_cast<const bf16x8*>(&sH[(16 * nt + c) * 64 + 32 * ks + 8 * g]);
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    bf16x8 az[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      az[ks] = *reinterpret_cast<const bf16x8*>(&sZ[(16 * mt + c) * 64 + 32 * ks + 8 * g]);
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      f32x4 d = mfma(az[0], bh[0][nt], f32x4{0.f, 0.f, 0.f, 0.f});
-      d = mfma(az[1], bh[1][nt], d);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        atomicAdd(&grad[OFF_W2 + (16 * mt + 4 * g + i) * MLP_H + 16 * nt + c], d[i]);
-    }
+    for (int ut = 0; ut < 4; ++ut)
+      acc.w2[ut] = mfma(az,
+                        *reinterpret_cast<const bf16x8*>(
+                            &sH[(16 * ut + c) * kGradRow + 32 * ks + 8 * g]),
+                        acc.w2[ut]);
   }
-  wave_lds_sync();
 }
 
 }  // namespace fx
