@@ -640,12 +640,6 @@ __device__ __forceinline__ int hll(const DevParams& P, const R* Vm, const R* Vp,
 // fan pressure's power is the density's times (c/ck)^2; and powers are taken
 // as exp2(e log2 x) (pow_pos) where the oracle calls pow.
 
-// R = double is the FP64 solver.  R = float serves the mixed-precision
-// mode: the pressure function, sampling and flux run in FP32, while the
-// Newton iterate and its convergence test stay in FP64 (the iterate is
-// rounded to FP32 only to evaluate the function).  The R = double
-// instantiation performs the FP64 operations in the order described above.
-
 // x^e for x > 0 as exp2(e log2 x).  In FP64 this is about 130 instructions
 // against pow's 230 (pow also handles signs, integer exponents and extra
 // precision that positive pressure and sound-speed ratios do not need); its
@@ -655,38 +649,102 @@ __device__ __forceinline__ int hll(const DevParams& P, const R* Vm, const R* Vp,
 __device__ __forceinline__ double pow_pos(double x, double e) { return exp2(e * log2(x)); }
 __device__ __forceinline__ float pow_pos(float x, float e) { return exp2f(e * log2f(x)); }
 
-// Tolerance floor of the FP32 solve.  FP32 evaluations of the pressure
-// function leave rounding noise of up to a few 1e-7 in p*, where Newton's
-// relative change can stall; a change of 1e-5 already puts the next iterate
-// (quadratic convergence) below FP32 resolution.
-constexpr double kExactTolF32 = 1.e-5;
+// The FP64 solver is bound by instruction issue, so it is built twice.  FAST
+// forms its quotients and roots without range handling (quot, recip_rn,
+// sqrt_fast): the same bits while the states are inside exact_window, which a
+// wavefront checks once per problem.  The other build serves wavefronts with a
+// state outside.  With what gamma and a side alone give taken out of the
+// iteration, and one copy of the sampling for both sides: k_solve_update on 1024
+// blocks of 16^3 1574 -> 1316 us, 4M seeded problems 1015 -> 880 us.
+template <bool FAST> struct ExactOps {
+  static __device__ __forceinline__ double div(double x, double y) {
+    return FAST ? quot(x, y) : x / y;
+  }
+  // several quotients by y
+  static __device__ __forceinline__ double recip(double y) { return FAST ? recip_rn(y) : y; }
+  static __device__ __forceinline__ double divr(double x, double y, double r) {
+    return FAST ? quot_r(x, y, r) : x / y;
+  }
+  static __device__ __forceinline__ double root(double x) { return FAST ? sqrt_fast(x) : sqrt(x); }
+};
 
-template <typename R>
-__device__ __forceinline__ void exact_fk(R p, R rk, R pk, R ck, R g, R& f, R& fd) {
-  if (p <= pk) {
+// Densities and pressures within 2^-96 .. 2^96, velocity differences up to 2^96,
+// gamma - 1 within 2^-10 .. 2^10: with p* at most some 2^300 and an iterate of
+// 1e-30 or more every quotient and divisor stays far inside 2^+-1000 and every
+// root inside 2^+-410.
+__device__ __forceinline__ bool exact_window(double g, double rl, double pl, double rr, double pr,
+                                             double du) {
+  constexpr double W = 0x1p+96;
+  const double lo = fmin(fmin(rl, rr), fmin(pl, pr)), hi = fmax(fmax(rl, rr), fmax(pl, pr));
+  const double g1 = g - 1.;
+  return lo >= 1. / W && hi <= W && fabs(du) <= W && g1 >= 0x1p-10 && g1 <= 0x1p+10;
+}
+
+// what the pressure function and the sampling take from gamma alone, and from
+// one side's state
+struct ExactGas {
+  double g, t1, e1, gr, gp1, rp1;   // 2/(g-1), (g-1)/(2g), (g-1)/(g+1), g+1 and its reciprocal
+};
+struct ExactSide {
+  double rho, p, c;
+  double fr, ir;   // rarefaction: 2/(g-1) c, 1/(rho c)
+  double ak, bk;   // shock: 2/((g+1) rho), (g-1)/(g+1) p
+};
+template <bool FAST>
+__device__ __forceinline__ ExactGas exact_gas(double g) {
+  using O = ExactOps<FAST>;
+  ExactGas G;
+  G.g = g;
+  G.gp1 = g + 1.;
+  G.rp1 = O::recip(G.gp1);
+  G.t1 = O::div(2., g - 1.);
+  G.e1 = O::div(g - 1., 2. * g);
+  G.gr = O::divr(g - 1., G.gp1, G.rp1);
+  return G;
+}
+template <bool FAST>
+__device__ __forceinline__ ExactSide exact_side(const ExactGas& G, double rho, double p, double c) {
+  using O = ExactOps<FAST>;
+  ExactSide s;
+  s.rho = rho;
+  s.p = p;
+  s.c = c;
+  s.fr = G.t1 * c;
+  s.ir = O::div(1., rho * c);
+  s.ak = O::div(2., G.gp1 * rho);
+  s.bk = G.gr * p;
+  return s;
+}
+
+template <bool FAST>
+__device__ __forceinline__ void exact_fk(double p, const ExactGas& G, const ExactSide& s, double& f,
+                                         double& fd) {
+  using O = ExactOps<FAST>;
+  if (p <= s.p) {
     // rarefaction: the derivative's power is the value's divided by pratio,
     // since (g - 1)/(2g) + (g + 1)/(2g) = 1 (one pow instead of two)
-    const R pratio = p / pk;
-    const R q = pow_pos(pratio, (g - R(1.)) / (R(2.) * g));
-    f = R(2.) / (g - R(1.)) * ck * (q - R(1.));
-    fd = (R(1.) / (rk * ck)) * (q / pratio);
+    const double pratio = O::div(p, s.p);
+    const double q = pow_pos(pratio, G.e1);
+    f = s.fr * (q - 1.);
+    fd = s.ir * O::div(q, pratio);
   } else {
-    const R ak = R(2.) / ((g + R(1.)) * rk);
-    const R bk = (g - R(1.)) / (g + R(1.)) * pk;
-    const R qrt = sqrt(ak / (bk + p));
-    f = (p - pk) * qrt;
-    fd = (R(1.) - R(0.5) * (p - pk) / (bk + p)) * qrt;
+    const double bp = s.bk + p, rb = O::recip(bp);
+    const double qrt = O::root(O::divr(s.ak, bp, rb));
+    f = (p - s.p) * qrt;
+    fd = (1. - O::divr(0.5 * (p - s.p), bp, rb)) * qrt;
   }
 }
 
-template <typename R>
-__device__ __forceinline__ R two_shock_guess(R g, R rl, R ul, R pl, R cl, R rr, R ur, R pr, R cr) {
-  const R ppv = R(0.5) * (pl + pr) - R(0.125) * (ur - ul) * (rl + rr) * (cl + cr);
-  const R p0 = fmax(R(1.e-30), ppv);
-  const R gl = sqrt((R(2.) / ((g + R(1.)) * rl)) / ((g - R(1.)) / (g + R(1.)) * pl + p0));
-  const R gr = sqrt((R(2.) / ((g + R(1.)) * rr)) / ((g - R(1.)) / (g + R(1.)) * pr + p0));
-  const R pts = (gl * pl + gr * pr - (ur - ul)) / (gl + gr);
-  return fmax(R(1.e-30), pts);
+template <bool FAST>
+__device__ __forceinline__ double two_shock_guess(double ul, const ExactSide& L, double ur,
+                                             const ExactSide& Q) {
+  using O = ExactOps<FAST>;
+  const double ppv = 0.5 * (L.p + Q.p) - 0.125 * (ur - ul) * (L.rho + Q.rho) * (L.c + Q.c);
+  const double p0 = fmax(1.e-30, ppv);
+  const double gl = O::root(O::div(L.ak, L.bk + p0));
+  const double gr = O::root(O::div(Q.ak, Q.bk + p0));
+  const double pts = O::div(gl * L.p + gr * Q.p - (ur - ul), gl + gr);
+  return fmax(1.e-30, pts);
 }
 
 // Newton from the better of two starts: the pressure function is evaluated
@@ -694,22 +752,23 @@ __device__ __forceinline__ R two_shock_guess(R g, R rl, R ul, R pl, R cl, R rr, 
 // |f(p)| (its f and f' serve the first step).  pb <= 0 means no second
 // start: plain Newton from pa, in the CPU oracle's operation order.
 // Returns iterations, negative when maxit was reached; pick = 0 when pa was
-// taken.  The iterate p is FP64 whatever R is.
-template <typename R>
-__device__ __forceinline__ int exact_newton_pick(R g, R rl, R pl, R cl, R rr, R pr, R cr, R du,
-                                                 double pa, double pb, double tol, int maxit,
-                                                 double& pstar, int& pick) {
-  R fl, fld, fr, frd;
-  exact_fk(R(pa), rl, pl, cl, g, fl, fld);
-  exact_fk(R(pa), rr, pr, cr, g, fr, frd);
+// taken.
+template <bool FAST>
+__device__ __forceinline__ int exact_newton_pick(const ExactGas& G, const ExactSide& L,
+                                                 const ExactSide& Q, double du, double pa, double pb,
+                                                 double tol, int maxit, double& pstar, int& pick) {
+  using O = ExactOps<FAST>;
+  double fl, fld, fr, frd;
+  exact_fk<FAST>(pa, G, L, fl, fld);
+  exact_fk<FAST>(pa, G, Q, fr, frd);
   double p = pa;
-  R f = fl + fr + du, fd = fld + frd;
+  double f = fl + fr + du, fd = fld + frd;
   pick = 0;
   if (pb > 0.) {
-    R gl, gld, gr, grd;
-    exact_fk(R(pb), rl, pl, cl, g, gl, gld);
-    exact_fk(R(pb), rr, pr, cr, g, gr, grd);
-    const R fb = gl + gr + du;
+    double gl, gld, gr, grd;
+    exact_fk<FAST>(pb, G, L, gl, gld);
+    exact_fk<FAST>(pb, G, Q, gr, grd);
+    const double fb = gl + gr + du;
     if (!(fabs(f) <= fabs(fb))) {
       pick = 1;
       p = pb;
@@ -719,8 +778,191 @@ __device__ __forceinline__ int exact_newton_pick(R g, R rl, R pl, R cl, R rr, R 
   }
   for (int it = 1; it <= maxit; ++it) {
     if (it > 1) {
-      exact_fk(R(p), rl, pl, cl, g, fl, fld);
-      exact_fk(R(p), rr, pr, cr, g, fr, frd);
+      exact_fk<FAST>(p, G, L, fl, fld);
+      exact_fk<FAST>(p, G, Q, fr, frd);
+      f = fl + fr + du;
+      fd = fld + frd;
+    }
+    double pn = p - O::div(f, fd);
+    if (!(pn > 0.)) pn = 1.e-30;
+    const double change = 2. * fabs(O::div(pn - p, pn + p));
+    p = pn;
+    if (change <= tol) {
+      pstar = p;
+      return it;
+    }
+  }
+  pstar = p;
+  return -maxit;
+}
+
+struct ExactStats {
+  unsigned long long iters, fallbacks;
+};
+
+// state at x/t = 0 (Toro sec. 4.5); leftside tells which input supplies the
+// tangential velocities and gammas.  The right side is sampled as the left one
+// of the mirrored problem (velocities negated, which is exact), so that
+// wavefronts with faces on either side of the contact run one copy.
+template <bool FAST>
+__device__ __forceinline__ void exact_sample(const ExactGas& G, const ExactSide& L, double ul,
+                                             const ExactSide& Q, double ur, double pm, double um, double& r, double& u,
+                                             double& pp, bool& leftside) {
+  using O = ExactOps<FAST>;
+  const bool left = 0. <= um;
+  leftside = left;
+  const double rk = left ? L.rho : Q.rho, pk = left ? L.p : Q.p, ck = left ? L.c : Q.c;
+  const double v = left ? ul : -ur, w = left ? um : -um;
+  const double pmk = O::div(pm, pk);
+  if (left ? pm <= pk : !(pm > pk)) {
+    if (0. <= v - ck) {
+      r = rk; u = v; pp = pk;
+    } else {
+      const double cm = ck * pow_pos(pmk, G.e1);
+      const double st = w - cm;
+      // isentropic: rho = gamma p / c^2 behind the rarefaction
+      if (left ? 0. > st : 0. >= st) {
+        r = O::div(G.g * pm, cm * cm); u = w; pp = pm;
+      } else {
+        const double c = O::divr(2., G.gp1, G.rp1) * (ck + (G.g - 1.) * 0.5 * v);
+        u = left ? c : -(-c + 0.);   // a zero is +0 on either side
+        // in the fan, (c/ck)^(2g/(g-1)) = (c/ck)^(2/(g-1)) (c/ck)^2
+        const double x = O::div(c, ck);
+        const double q = pow_pos(x, G.t1), s2 = x * x;
+        r = rk * q;
+        pp = pk * (q * s2);
+      }
+    }
+  } else {
+    const double sk = v - ck * O::root(O::div(G.gp1, 2. * G.g) * pmk + G.e1);
+    if (0. <= sk) {
+      r = rk; u = v; pp = pk;
+    } else {
+      r = O::div(rk * (pmk + G.gr), O::divr(pmk * (G.g - 1.), G.gp1, G.rp1) + 1.);
+      u = w; pp = pm;
+    }
+  }
+  if (!left) u = -u;
+}
+
+// exact_riemann's problem once its states are known to be positive
+template <bool FAST, bool SEEDED>
+__device__ __forceinline__ int exact_solve(const DevParams& P, double g, double rl, double ul, double pl, double rr, double ur,
+                                           double pr, double guess, ExactStats& es, double& r, double& u, double& pp,
+                                           bool& left) {
+  using O = ExactOps<FAST>;
+  const double cl = O::root(O::div(g * pl, rl)), cr = O::root(O::div(g * pr, rr));
+  const ExactGas G = exact_gas<FAST>(g);
+  if (G.t1 * (cl + cr) <= ur - ul) return 2;
+  const double du = ur - ul;
+  const ExactSide L = exact_side<FAST>(G, rl, pl, cl), Q = exact_side<FAST>(G, rr, pr, cr);
+  const double ts = two_shock_guess<FAST>(ul, L, ur, Q);
+  const double tol = P.exactTol;
+  double pm;
+  int it, pick;
+  if constexpr (!SEEDED) {
+    it = exact_newton_pick<FAST>(G, L, Q, du, ts, -1.0, tol, P.exactMaxIter, pm, pick);
+    if (it < 0) es.fallbacks += 1;
+  } else {
+    double pb = guess;
+    for (;;) {
+      it = exact_newton_pick<FAST>(G, L, Q, du, ts, pb, tol, P.exactMaxIter, pm, pick);
+      if (it < 0 && (pb > 0. || guess <= 0.)) es.fallbacks += 1;   // a restart counts once
+      if (it >= 0 || pick == 0) break;
+      es.iters += (unsigned long long)(-it);
+      pb = -1.0;
+    }
+  }
+  es.iters += (unsigned long long)(it < 0 ? -it : it);
+  double fl, fld, fr, frd;
+  exact_fk<FAST>(pm, G, L, fl, fld);
+  exact_fk<FAST>(pm, G, Q, fr, frd);
+  const double um = 0.5 * (ul + ur) + 0.5 * (fr - fl);
+  exact_sample<FAST>(G, L, ul, Q, ur, pm, um, r, u, pp, left);
+  return 0;
+}
+
+// Exact solution at x/t = 0 of the face problem (rl, ul, pl | rr, ur, pr)
+// with the face-normal velocities ul, ur; returns 0 ok, 1 non-positive state,
+// 2 vacuum generated.  guess > 0 seeds Newton: it starts from the better of
+// the seed and the two-shock guess, and a seeded start that does not
+// converge restarts from the two-shock guess (counted as fallback).  One
+// Newton loop serves both passes, which keeps a seeded kernel's register
+// budget that of the unseeded one.  SEEDED = false ignores guess.
+template <bool SEEDED>
+__device__ __forceinline__ int exact_riemann(const DevParams& P, double g, double rl, double ul, double pl, double rr, double ur,
+                                             double pr, double guess, ExactStats& es, double& r, double& u,
+                                             double& pp, bool& left) {
+  if (!(rl > 0. && rr > 0. && pl > 0. && pr > 0.)) return 1;
+  if (__builtin_expect(__all(exact_window(g, rl, pl, rr, pr, ur - ul)), 1))
+    return exact_solve<true, SEEDED>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+  return exact_solve<false, SEEDED>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+}
+
+// ---- the FP32 solver (mixed-precision mode): the pressure function, sampling
+// and flux run in FP32, while the Newton iterate and its convergence test stay
+// in FP64 (the iterate is rounded to FP32 only to evaluate the function).  Its
+// expressions stand as they are written, apart from the FP64 ones: which of its
+// quotients the compiler rounds correctly and which it forms from a reciprocal
+// follows from how it merges the branches below, and the bits with it.
+
+// Tolerance floor of the FP32 solve.  FP32 evaluations of the pressure
+// function leave rounding noise of up to a few 1e-7 in p*, where Newton's
+// relative change can stall; a change of 1e-5 already puts the next iterate
+// (quadratic convergence) below FP32 resolution.
+constexpr double kExactTolF32 = 1.e-5;
+
+__device__ __forceinline__ void exact_fk_f32(float p, float rk, float pk, float ck, float g, float& f, float& fd) {
+  if (p <= pk) {
+    // rarefaction: the derivative's power is the value's divided by pratio,
+    // since (g - 1)/(2g) + (g + 1)/(2g) = 1 (one pow instead of two)
+    const float pratio = p / pk;
+    const float q = pow_pos(pratio, (g - 1.f) / (2.f * g));
+    f = 2.f / (g - 1.f) * ck * (q - 1.f);
+    fd = (1.f / (rk * ck)) * (q / pratio);
+  } else {
+    const float ak = 2.f / ((g + 1.f) * rk);
+    const float bk = (g - 1.f) / (g + 1.f) * pk;
+    const float qrt = sqrt(ak / (bk + p));
+    f = (p - pk) * qrt;
+    fd = (1.f - 0.5f * (p - pk) / (bk + p)) * qrt;
+  }
+}
+
+__device__ __forceinline__ float two_shock_guess_f32(float g, float rl, float ul, float pl, float cl, float rr, float ur, float pr, float cr) {
+  const float ppv = 0.5f * (pl + pr) - 0.125f * (ur - ul) * (rl + rr) * (cl + cr);
+  const float p0 = fmax(1.e-30f, ppv);
+  const float gl = sqrt((2.f / ((g + 1.f) * rl)) / ((g - 1.f) / (g + 1.f) * pl + p0));
+  const float gr = sqrt((2.f / ((g + 1.f) * rr)) / ((g - 1.f) / (g + 1.f) * pr + p0));
+  const float pts = (gl * pl + gr * pr - (ur - ul)) / (gl + gr);
+  return fmax(1.e-30f, pts);
+}
+
+__device__ __forceinline__ int exact_newton_pick_f32(float g, float rl, float pl, float cl, float rr, float pr, float cr, float du,
+                                                 double pa, double pb, double tol, int maxit,
+                                                 double& pstar, int& pick) {
+  float fl, fld, fr, frd;
+  exact_fk_f32(float(pa), rl, pl, cl, g, fl, fld);
+  exact_fk_f32(float(pa), rr, pr, cr, g, fr, frd);
+  double p = pa;
+  float f = fl + fr + du, fd = fld + frd;
+  pick = 0;
+  if (pb > 0.) {
+    float gl, gld, gr, grd;
+    exact_fk_f32(float(pb), rl, pl, cl, g, gl, gld);
+    exact_fk_f32(float(pb), rr, pr, cr, g, gr, grd);
+    const float fb = gl + gr + du;
+    if (!(fabs(f) <= fabs(fb))) {
+      pick = 1;
+      p = pb;
+      f = fb;
+      fd = gld + grd;
+    }
+  }
+  for (int it = 1; it <= maxit; ++it) {
+    if (it > 1) {
+      exact_fk_f32(float(p), rl, pl, cl, g, fl, fld);
+      exact_fk_f32(float(p), rr, pr, cr, g, fr, frd);
       f = fl + fr + du;
       fd = fld + frd;
     }
@@ -737,90 +979,75 @@ __device__ __forceinline__ int exact_newton_pick(R g, R rl, R pl, R cl, R rr, R 
   return -maxit;
 }
 
-struct ExactStats {
-  unsigned long long iters, fallbacks;
-};
-
-// state at x/t = 0 (Toro sec. 4.5); leftside tells which input supplies the
-// tangential velocities and gammas
-template <typename R>
-__device__ __forceinline__ void exact_sample(R g, R rl, R ul, R pl, R cl, R rr, R ur, R pr, R cr,
-                                             R pm, R um, R& r, R& u, R& pp, bool& leftside) {
-  if (R(0.) <= um) {
+__device__ __forceinline__ void exact_sample_f32(float g, float rl, float ul, float pl, float cl, float rr, float ur, float pr, float cr,
+                                             float pm, float um, float& r, float& u, float& pp, bool& leftside) {
+  if (0.f <= um) {
     leftside = true;
     if (pm <= pl) {
-      const R shl = ul - cl;
-      if (R(0.) <= shl) { r = rl; u = ul; pp = pl; return; }
-      const R cml = cl * pow_pos(pm / pl, (g - R(1.)) / (R(2.) * g));
-      const R stl = um - cml;
+      const float shl = ul - cl;
+      if (0.f <= shl) { r = rl; u = ul; pp = pl; return; }
+      const float cml = cl * pow_pos(pm / pl, (g - 1.f) / (2.f * g));
+      const float stl = um - cml;
       // isentropic: rho = gamma p / c^2 behind the rarefaction
-      if (R(0.) > stl) { r = g * pm / (cml * cml); u = um; pp = pm; return; }
-      const R c = R(2.) / (g + R(1.)) * (cl + (g - R(1.)) / R(2.) * (ul - R(0.)));
-      u = R(2.) / (g + R(1.)) * (cl + (g - R(1.)) / R(2.) * ul + R(0.));
+      if (0.f > stl) { r = g * pm / (cml * cml); u = um; pp = pm; return; }
+      const float c = 2.f / (g + 1.f) * (cl + (g - 1.f) / 2.f * (ul - 0.f));
+      u = 2.f / (g + 1.f) * (cl + (g - 1.f) / 2.f * ul + 0.f);
       // in the fan, (c/cl)^(2g/(g-1)) = (c/cl)^(2/(g-1)) (c/cl)^2
-      const R q = pow_pos(c / cl, R(2.) / (g - R(1.))), s2 = (c / cl) * (c / cl);
+      const float q = pow_pos(c / cl, 2.f / (g - 1.f)), s2 = (c / cl) * (c / cl);
       r = rl * q;
       pp = pl * (q * s2);
       return;
     }
-    const R pml = pm / pl;
-    const R sl = ul - cl * sqrt((g + R(1.)) / (R(2.) * g) * pml + (g - R(1.)) / (R(2.) * g));
-    if (R(0.) <= sl) { r = rl; u = ul; pp = pl; return; }
-    r = rl * (pml + (g - R(1.)) / (g + R(1.))) / (pml * (g - R(1.)) / (g + R(1.)) + R(1.));
+    const float pml = pm / pl;
+    const float sl = ul - cl * sqrt((g + 1.f) / (2.f * g) * pml + (g - 1.f) / (2.f * g));
+    if (0.f <= sl) { r = rl; u = ul; pp = pl; return; }
+    r = rl * (pml + (g - 1.f) / (g + 1.f)) / (pml * (g - 1.f) / (g + 1.f) + 1.f);
     u = um; pp = pm;
     return;
   }
   leftside = false;
   if (pm > pr) {
-    const R pmr = pm / pr;
-    const R sr = ur + cr * sqrt((g + R(1.)) / (R(2.) * g) * pmr + (g - R(1.)) / (R(2.) * g));
-    if (R(0.) >= sr) { r = rr; u = ur; pp = pr; return; }
-    r = rr * (pmr + (g - R(1.)) / (g + R(1.))) / (pmr * (g - R(1.)) / (g + R(1.)) + R(1.));
+    const float pmr = pm / pr;
+    const float sr = ur + cr * sqrt((g + 1.f) / (2.f * g) * pmr + (g - 1.f) / (2.f * g));
+    if (0.f >= sr) { r = rr; u = ur; pp = pr; return; }
+    r = rr * (pmr + (g - 1.f) / (g + 1.f)) / (pmr * (g - 1.f) / (g + 1.f) + 1.f);
     u = um; pp = pm;
     return;
   }
-  const R shr = ur + cr;
-  if (R(0.) >= shr) { r = rr; u = ur; pp = pr; return; }
-  const R cmr = cr * pow_pos(pm / pr, (g - R(1.)) / (R(2.) * g));
-  const R str = um + cmr;
-  if (R(0.) <= str) { r = g * pm / (cmr * cmr); u = um; pp = pm; return; }
-  const R c = R(2.) / (g + R(1.)) * (cr - (g - R(1.)) / R(2.) * (ur - R(0.)));
-  u = R(2.) / (g + R(1.)) * (-cr + (g - R(1.)) / R(2.) * ur + R(0.));
-  const R q = pow_pos(c / cr, R(2.) / (g - R(1.))), s2 = (c / cr) * (c / cr);
+  const float shr = ur + cr;
+  if (0.f >= shr) { r = rr; u = ur; pp = pr; return; }
+  const float cmr = cr * pow_pos(pm / pr, (g - 1.f) / (2.f * g));
+  const float str = um + cmr;
+  if (0.f <= str) { r = g * pm / (cmr * cmr); u = um; pp = pm; return; }
+  const float c = 2.f / (g + 1.f) * (cr - (g - 1.f) / 2.f * (ur - 0.f));
+  u = 2.f / (g + 1.f) * (-cr + (g - 1.f) / 2.f * ur + 0.f);
+  const float q = pow_pos(c / cr, 2.f / (g - 1.f)), s2 = (c / cr) * (c / cr);
   r = rr * q;
   pp = pr * (q * s2);
 }
 
-// Exact solution at x/t = 0 of the face problem (rl, ul, pl | rr, ur, pr)
-// with the face-normal velocities ul, ur; returns 0 ok, 1 non-positive state,
-// 2 vacuum generated.  guess > 0 seeds Newton: it starts from the better of
-// the seed and the two-shock guess, and a seeded start that does not
-// converge restarts from the two-shock guess (counted as fallback).  One
-// Newton loop serves both passes, which keeps a seeded kernel's register
-// budget that of the unseeded one.  SEEDED = false ignores guess.  The FP32
-// solve (R = float) converges to max(exactTol, kExactTolF32), and a seed is
-// held at 1e-30 or above, inside FP32's normal range.
-template <bool SEEDED, typename R>
-__device__ __forceinline__ int exact_riemann(const DevParams& P, R g, R rl, R ul, R pl, R rr, R ur,
-                                             R pr, double guess, ExactStats& es, R& r, R& u,
-                                             R& pp, bool& left) {
-  constexpr bool kF32 = sizeof(R) == sizeof(float);
-  if (!(rl > R(0.) && rr > R(0.) && pl > R(0.) && pr > R(0.))) return 1;
-  const R cl = sqrt(g * pl / rl), cr = sqrt(g * pr / rr);
-  if (R(2.) / (g - R(1.)) * (cl + cr) <= ur - ul) return 2;
-  const R du = ur - ul;
-  const R ts = two_shock_guess(g, rl, ul, pl, cl, rr, ur, pr, cr);
-  const double tol = kF32 ? fmax(P.exactTol, kExactTolF32) : P.exactTol;
+// As exact_riemann.  Converges to max(exactTol, kExactTolF32), and a seed is held
+// at 1e-30 or above, inside FP32's normal range.
+template <bool SEEDED>
+__device__ __forceinline__ int exact_riemann_f32(const DevParams& P, float g, float rl, float ul, float pl, float rr, float ur,
+                                             float pr, double guess, ExactStats& es, float& r, float& u,
+                                             float& pp, bool& left) {
+  if (!(rl > 0.f && rr > 0.f && pl > 0.f && pr > 0.f)) return 1;
+  const float cl = sqrt(g * pl / rl), cr = sqrt(g * pr / rr);
+  if (2.f / (g - 1.f) * (cl + cr) <= ur - ul) return 2;
+  const float du = ur - ul;
+  const float ts = two_shock_guess_f32(g, rl, ul, pl, cl, rr, ur, pr, cr);
+  const double tol = fmax(P.exactTol, kExactTolF32);
   double pm;
   int it, pick;
   if constexpr (!SEEDED) {
-    it = exact_newton_pick(g, rl, pl, cl, rr, pr, cr, du, double(ts), -1.0, tol, P.exactMaxIter,
+    it = exact_newton_pick_f32(g, rl, pl, cl, rr, pr, cr, du, double(ts), -1.0, tol, P.exactMaxIter,
                            pm, pick);
     if (it < 0) es.fallbacks += 1;
   } else {
-    double pb = (kF32 && guess > 0.) ? fmax(guess, 1.e-30) : guess;
+    double pb = guess > 0. ? fmax(guess, 1.e-30) : guess;
     for (;;) {
-      it = exact_newton_pick(g, rl, pl, cl, rr, pr, cr, du, double(ts), pb, tol, P.exactMaxIter,
+      it = exact_newton_pick_f32(g, rl, pl, cl, rr, pr, cr, du, double(ts), pb, tol, P.exactMaxIter,
                              pm, pick);
       if (it < 0 && (pb > 0. || guess <= 0.)) es.fallbacks += 1;   // a restart counts once
       if (it >= 0 || pick == 0) break;
@@ -829,12 +1056,12 @@ __device__ __forceinline__ int exact_riemann(const DevParams& P, R g, R rl, R ul
     }
   }
   es.iters += (unsigned long long)(it < 0 ? -it : it);
-  const R pmr = R(pm);
-  R fl, fld, fr, frd;
-  exact_fk(pmr, rl, pl, cl, g, fl, fld);
-  exact_fk(pmr, rr, pr, cr, g, fr, frd);
-  const R um = R(0.5) * (ul + ur) + R(0.5) * (fr - fl);
-  exact_sample(g, rl, ul, pl, cl, rr, ur, pr, cr, pmr, um, r, u, pp, left);
+  const float pmr = float(pm);
+  float fl, fld, fr, frd;
+  exact_fk_f32(pmr, rl, pl, cl, g, fl, fld);
+  exact_fk_f32(pmr, rr, pr, cr, g, fr, frd);
+  const float um = 0.5f * (ul + ur) + 0.5f * (fr - fl);
+  exact_sample_f32(g, rl, ul, pl, cl, rr, ur, pr, cr, pmr, um, r, u, pp, left);
   return 0;
 }
 
@@ -875,8 +1102,11 @@ __device__ __forceinline__ int exact_face_flux(const DevParams& P, int d, const 
   const R ul = Lb[(1 + d) * s], ur = Rb[(1 + d) * s];
   R r, u, pp;
   bool left;
-  const int e = exact_riemann<SEEDED>(P, R(gamc), rl, ul, pl, rr, ur, pr, guess, es, r, u, pp,
-                                      left);
+  int e;
+  if constexpr (sizeof(R) == sizeof(double))
+    e = exact_riemann<SEEDED>(P, gamc, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+  else
+    e = exact_riemann_f32<SEEDED>(P, float(gamc), rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
   if (e) return e;
   // the sampled state takes its tangential velocities and game from the side
   // of the contact the face lies on

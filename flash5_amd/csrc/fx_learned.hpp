@@ -213,6 +213,37 @@ __global__ void __launch_bounds__(kLearnThreads) k_mlp_seed_states(
   }
 }
 
+// One problem of k_riemann_batch: p* in pm and the Newton iterations spent,
+// negative when even the two-shock start did not converge; false on vacuum.
+template <bool FAST, bool SEEDED>
+__device__ __forceinline__ bool riemann_star(double g, const IfaceState& s, const float* yseed,
+                                             double tol, int maxit, const SeedGate& gate,
+                                             ExactStats& es, double& pm, int& iters) {
+  using O = ExactOps<FAST>;
+  const double cl = O::root(O::div(g * s.pl, s.rl)), cr = O::root(O::div(g * s.pr, s.rr));
+  const ExactGas G = exact_gas<FAST>(g);
+  if (G.t1 * (cl + cr) <= s.ur - s.ul) return false;
+  const double du = s.ur - s.ul;
+  const ExactSide L = exact_side<FAST>(G, s.rl, s.pl, cl),
+                          Q = exact_side<FAST>(G, s.rr, s.pr, cr);
+  const double ts = two_shock_guess<FAST>(s.ul, L, s.ur, Q);
+  const bool use = SEEDED && seed_gate_pass(gate, g, s.rl, s.ul, s.pl, s.rr, s.ur, s.pr);
+  double pb = use ? seed_from_y(*yseed, s.pl, s.pr) : -1.0;
+  int it, total = 0;
+  // one Newton loop for the seeded start and its two-shock restart
+  for (;;) {
+    int pick;
+    it = exact_newton_pick<FAST>(G, L, Q, du, ts, pb, tol, maxit, pm, pick);
+    total += it < 0 ? -it : it;
+    if (it < 0 && (pb > 0. || !use)) es.fallbacks += 1;   // a restart counts once
+    if (it >= 0 || pick == 0) break;
+    pb = -1.0;
+  }
+  es.iters += (unsigned long long)total;
+  iters = it < 0 ? -total : total;
+  return true;
+}
+
 // Exact Riemann problems in a batch: p* by Newton (FP64 iterate and
 // convergence test) from the two-shock guess, or from the network's seed
 // (SEEDED); a seeded start that does not converge restarts from the
@@ -224,35 +255,26 @@ __global__ void __launch_bounds__(kThreads) k_riemann_batch(
     double tol, int maxit, double* __restrict__ pstar, int* __restrict__ iters, DevStatus* st,
     SeedGate gate) {
   ExactStats es{0ULL, 0ULL};
-  const double g = gamma;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long)gridDim.x * blockDim.x) {
     const IfaceState s = load_iface(S, n, i, true);
-    const double cl = sqrt(g * s.pl / s.rl), cr = sqrt(g * s.pr / s.rr);
-    if (!(s.rl > 0. && s.rr > 0. && s.pl > 0. && s.pr > 0.) ||
-        2. / (g - 1.) * (cl + cr) <= s.ur - s.ul) {
-      pstar[i] = 0.0;
-      iters[i] = 0;
+    double pm = 0.0;
+    int it = 0;
+    bool ok = s.rl > 0. && s.rr > 0. && s.pl > 0. && s.pr > 0.;
+    if (ok) {
+      const float* y = SEEDED ? yseed + i : nullptr;
+      if (__builtin_expect(__all(exact_window(gamma, s.rl, s.pl, s.rr, s.pr, s.ur - s.ul)), 1))
+        ok = riemann_star<true, SEEDED>(gamma, s, y, tol, maxit, gate, es, pm, it);
+      else
+        ok = riemann_star<false, SEEDED>(gamma, s, y, tol, maxit, gate, es, pm, it);
+    }
+    if (!ok) {
+      pm = 0.0;
+      it = 0;
       report_error(st, 2, -1, (int)(i & 0x7fffffff), 0, 0, 0);
-      continue;
     }
-    const double du = s.ur - s.ul;
-    const double ts = two_shock_guess(g, s.rl, s.ul, s.pl, cl, s.rr, s.ur, s.pr, cr);
-    const bool use = SEEDED && seed_gate_pass(gate, g, s.rl, s.ul, s.pl, s.rr, s.ur, s.pr);
-    double pm, pb = use ? seed_from_y(yseed[i], s.pl, s.pr) : -1.0;
-    int it, total = 0;
-    // one Newton loop for the seeded start and its two-shock restart
-    for (;;) {
-      int pick;
-      it = exact_newton_pick(g, s.rl, s.pl, cl, s.rr, s.pr, cr, du, ts, pb, tol, maxit, pm, pick);
-      total += it < 0 ? -it : it;
-      if (it < 0 && (pb > 0. || !use)) es.fallbacks += 1;   // a restart counts once
-      if (it >= 0 || pick == 0) break;
-      pb = -1.0;
-    }
-    es.iters += (unsigned long long)total;
     pstar[i] = pm;
-    iters[i] = it < 0 ? -total : total;
+    iters[i] = it;
   }
   flush_exact(st, es);
 }
