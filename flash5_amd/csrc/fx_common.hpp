@@ -30,13 +30,11 @@ struct Launch {
 };
 
 // Tiles of several block classes in one launch: each tile's class selects its
-// parameters, and per-tile prefix offsets map a flat cell (or face) index to
-// its tile.
+// parameters, each workgroup's chunk its tile and the first of its cells.
 struct ClassMap {
   const DevParams* cls;        // parameters per class
   const unsigned char* tcls;   // class of each tile
-  const long* start;           // items before tile t; start[nTiles] = all items
-  const int* wtab;             // tile of every 64th item (find_tile_w)
+  const int2* chunks;          // (tile, first cell) of each workgroup
 };
 
 // t with start[t] <= gid < start[t + 1] (start non-decreasing, start[0] = 0)

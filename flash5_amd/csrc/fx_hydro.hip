@@ -585,15 +585,15 @@ k_update_finish(DevParams P, const fx_tile* __restrict__ tiles, int nTiles,
   }
 }
 
-// the update over tiles of several block classes in one launch
+// the update over tiles of several block classes in one launch: workgroup w
+// takes kThreads cells of one tile, so its class is uniform and no cell is
+// searched for
 __global__ void __launch_bounds__(kThreads) k_update_multi(Launch L, ClassMap M,
                                                            const unsigned char* __restrict__ inPlace) {
-  const long total = M.start[L.nTiles];
-  for (long gid = (long)blockIdx.x * blockDim.x + threadIdx.x; gid < total;
-       gid += (long)gridDim.x * blockDim.x) {
-    const int t = find_tile_w(M.start, M.wtab, L.nTiles, gid);
-    update_cell<false, false>(M.cls[M.tcls[t]], L, t, gid - M.start[t], inPlace);
-  }
+  const int2 ch = M.chunks[blockIdx.x];
+  const DevParams& P = M.cls[M.tcls[ch.x]];
+  const int r = ch.y + (int)threadIdx.x;
+  if (r < (int)P.icells) update_cell<false, false>(P, L, ch.x, r, inPlace);
 }
 
 // the CFL dt of each block (one workgroup per block), as dt_pick_block
@@ -918,12 +918,15 @@ struct Lib {
   double runCfl = 0.;                  // the CFL argument of the graph-captured run
   hipStream_t capStream = nullptr;     // library stream for graph capture (default priority)
   std::vector<int> hnbr;               // neighbour table last uploaded (host copy)
+  int nbrDim = 0;                      // axes of hnbr that were checked, once on the device
   int* dnbr = nullptr;
   size_t dnbrCap = 0;
   long lastFaces = 0;                  // faces of the last exact-solver step
   int lastTiles = 0;
   unsigned char* dinplace = nullptr;
   size_t dinplaceCap = 0;
+  void* hpin = nullptr;                // pinned host memory that results are copied to
+  size_t hpinCap = 0;                  // bytes
   DevStatus* status = nullptr;
   double* partial = nullptr;
   int partialCap = 0;
@@ -942,13 +945,13 @@ struct Lib {
   std::vector<long> hcellStart, hfaceStart;
   unsigned char* dtcls = nullptr;
   size_t dtclsCap = 0;
-  long* dcellStart = nullptr;
-  size_t dcellStartCap = 0;
   long* dfaceStart = nullptr;
   size_t dfaceStartCap = 0;
-  std::vector<int> hwCell, hwFace;     // find_tile_w tables of the cell and face prefixes
-  int* dwCell = nullptr;
-  size_t dwCellCap = 0;
+  std::vector<int> hwFace;             // find_tile_w table of the face prefix
+  std::vector<int2> hcellChunks;       // multi-class: (tile, first cell) per kThreads cells
+  int2* dcellChunks = nullptr;
+  size_t cellChunksCap = 0;
+  int nCellChunks = 0;
   int* dwFace = nullptr;
   size_t dwFaceCap = 0;
   std::vector<int2> hgateChunks;       // multi-class: (tile, first face) per kThreads faces
@@ -1212,11 +1215,24 @@ bool cfl_varies(const fx_params& p) { return p.shockLowerCFL || fallback_cfl_cap
 
 // Synchronise and copy the device status record ds into st (nothing in
 // async mode, where the call returns before its kernels end).
+// The library's pinned buffer, of at least bytes.  A device-to-host copy into it
+// queues behind the kernels, so that a call waits once, for both.
+int pinned(size_t bytes, fx_status* st) {
+  if (g.hpinCap >= bytes) return 0;
+  if (g.hpin) HIPCALL(hipHostFree(g.hpin), st);
+  g.hpin = nullptr;
+  g.hpinCap = 0;
+  HIPCALL(hipHostMalloc(&g.hpin, bytes, hipHostMallocDefault), st);
+  g.hpinCap = bytes;
+  return 0;
+}
+
 int finish_from(const DevStatus* ds, fx_status* st) {
   if (g.async) return 0;
+  if (pinned(sizeof(DevStatus), st)) return 4;
+  HIPCALL(hipMemcpyAsync(g.hpin, ds, sizeof(DevStatus), hipMemcpyDeviceToHost, g.stream), st);
   HIPCALL(hipStreamSynchronize(g.stream), st);
-  DevStatus h{};
-  HIPCALL(hipMemcpy(&h, ds, sizeof h, hipMemcpyDeviceToHost), st);
+  const DevStatus h = *static_cast<const DevStatus*>(g.hpin);
   if (st) {
     st->code = h.code;
     st->first_tile = h.tile;
@@ -1352,10 +1368,25 @@ std::vector<int> wave_table(const std::vector<long>& start) {
   return w;
 }
 
+// Each tile's items (start[t] .. start[t + 1]) in chunks of kThreads, (tile,
+// first item of it), on the device.
+int upload_chunks(int nTiles, const std::vector<long>& start, std::vector<int2>& ch, int2** dev,
+                  size_t* cap, int* n, fx_status* st) {
+  ch.clear();
+  for (int t = 0; t < nTiles; ++t)
+    for (long e = 0; e < start[t + 1] - start[t]; e += kThreads) ch.push_back(make_int2(t, (int)e));
+  *n = (int)ch.size();
+  if (grow(dev, cap, ch.size(), st)) return 4;
+  HIPCALL(hipMemcpyAsync(*dev, ch.data(), sizeof(int2) * ch.size(), hipMemcpyHostToDevice, g.stream),
+          st);
+  return 0;
+}
+
 // Uploads the tile list, substituting library-owned flux arrays where a
 // tile has none.
+// cells: for a call that updates cells
 int upload_tiles(const fx_tile* tiles, int nTiles, bool needFlux, fx_status* st,
-                 bool useClasses = true) {
+                 bool useClasses = true, bool cells = true) {
   g.batchValid = false;
   ++g.uploadGen;
   if (classify_tiles(tiles, nTiles, useClasses)) {
@@ -1395,38 +1426,28 @@ int upload_tiles(const fx_tile* tiles, int nTiles, bool needFlux, fx_status* st,
           st);
   if (g.multi) {
     if (grow(&g.dtcls, &g.dtclsCap, (size_t)nTiles, st)) return 4;
-    if (grow(&g.dcellStart, &g.dcellStartCap, (size_t)nTiles + 1, st)) return 4;
-    if (grow(&g.dfaceStart, &g.dfaceStartCap, (size_t)nTiles + 1, st)) return 4;
     HIPCALL(hipMemcpyAsync(g.dtcls, g.htcls.data(), (size_t)nTiles, hipMemcpyHostToDevice, g.stream),
             st);
-    HIPCALL(hipMemcpyAsync(g.dcellStart, g.hcellStart.data(), sizeof(long) * (nTiles + 1),
-                           hipMemcpyHostToDevice, g.stream),
-            st);
+    g.nItems = 0;  // march items are built for the tile shape of the call
+    if (cells && upload_chunks(nTiles, g.hcellStart, g.hcellChunks, &g.dcellChunks,
+                               &g.cellChunksCap, &g.nCellChunks, st))
+      return 4;
+    // the tables by face, three times the cells' size, serve the exact solver's
+    // separate face stage alone
+    if (g.cur.riemann != FX_EXACT) return 0;
+    if (grow(&g.dfaceStart, &g.dfaceStartCap, (size_t)nTiles + 1, st)) return 4;
     HIPCALL(hipMemcpyAsync(g.dfaceStart, g.hfaceStart.data(), sizeof(long) * (nTiles + 1),
                            hipMemcpyHostToDevice, g.stream),
             st);
-    g.hwCell = wave_table(g.hcellStart);
     g.hwFace = wave_table(g.hfaceStart);
-    if (grow(&g.dwCell, &g.dwCellCap, g.hwCell.size(), st)) return 4;
     if (grow(&g.dwFace, &g.dwFaceCap, g.hwFace.size(), st)) return 4;
-    HIPCALL(hipMemcpyAsync(g.dwCell, g.hwCell.data(), sizeof(int) * g.hwCell.size(),
-                           hipMemcpyHostToDevice, g.stream),
-            st);
     HIPCALL(hipMemcpyAsync(g.dwFace, g.hwFace.data(), sizeof(int) * g.hwFace.size(),
                            hipMemcpyHostToDevice, g.stream),
             st);
-    g.nItems = 0;  // march items are built for the tile shape of the call
-    // the learned seed's gate pass: each tile's faces in chunks of kThreads
-    std::vector<int2>& ch = g.hgateChunks;
-    ch.clear();
-    for (int t = 0; t < nTiles; ++t)
-      for (long f = 0; f < g.hfaceStart[t + 1] - g.hfaceStart[t]; f += kThreads)
-        ch.push_back(make_int2(t, (int)f));
-    g.nGateChunks = (int)ch.size();
-    if (grow(&g.dgateChunks, &g.gateChunksCap, ch.size(), st)) return 4;
-    HIPCALL(hipMemcpyAsync(g.dgateChunks, ch.data(), sizeof(int2) * ch.size(),
-                           hipMemcpyHostToDevice, g.stream),
-            st);
+    // the learned seed's gate pass
+    if (g.cur.learned && upload_chunks(nTiles, g.hfaceStart, g.hgateChunks, &g.dgateChunks,
+                                       &g.gateChunksCap, &g.nGateChunks, st))
+      return 4;
   }
   return 0;
 }
@@ -1603,8 +1624,8 @@ void launch_update_finish(const DevParams& P, const fx_tile* tiles, int nTiles, 
 void launch_update(int nTiles, double dt, const unsigned char* dIn) {
   Launch L{g.dtiles, nTiles, nullptr, g.status, dt, g.dtDev};
   if (g.multi) {
-    const ClassMap C{g.dcls, g.dtcls, g.dcellStart, g.dwCell};
-    hipLaunchKernelGGL(k_update_multi, dim3(grid_for(g.hcellStart[nTiles])), dim3(kThreads), 0,
+    const ClassMap C{g.dcls, g.dtcls, g.dcellChunks};
+    hipLaunchKernelGGL(k_update_multi, dim3((unsigned)g.nCellChunks), dim3(kThreads), 0,
                        g.stream, L, C, dIn);
   } else if (g.cur.ndim == 3) {
     hipLaunchKernelGGL(k_update_cols,
@@ -1660,31 +1681,34 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
   }
   if (st) memset(st, 0, sizeof *st);
   if (nTiles <= 0) return 0;
+  bool anyInPlace = !inPlace;
+  for (int t = 0; !anyInPlace && t < nTiles; ++t) anyInPlace = inPlace[t] != 0;
   if (!tilesUploaded) {
-    const int rc = upload_tiles(tiles, nTiles, true, st);
+    const int rc = upload_tiles(tiles, nTiles, true, st, true, anyInPlace);
     if (rc) return rc;
   }
   const DevParams& P = g.cur;
   const unsigned char* dIn = nullptr;
-  bool anyFluxOnly = false;
   if (inPlace) {
     for (int t = 0; t < nTiles; ++t)
       if (!inPlace[t]) {
-        anyFluxOnly = true;
         if (P.aux && !tiles[t].pavg) {
           if (st) st->code = 3;
           return 3;
         }
       }
-    if (grow(&g.dinplace, &g.dinplaceCap, (size_t)nTiles, st)) return 4;
-    HIPCALL(hipMemcpyAsync(g.dinplace, inPlace, nTiles, hipMemcpyHostToDevice, g.stream), st);
-    dIn = g.dinplace;
   }
   int TX = 0, TY = 8, NT = 0;
   const bool march = g.multi ? multi_march_shape(&TX) : (!g.legacy && march_shape(P, &TX, &TY, &NT));
   if (P.learned && (!march || !g.seedReady)) {  // the seed needs the march path and a network
     if (st) st->code = 3;
     return 3;
+  }
+  // the march's update is not launched when no tile is in place
+  if (inPlace && (anyInPlace || !march)) {
+    if (grow(&g.dinplace, &g.dinplaceCap, (size_t)nTiles, st)) return 4;
+    HIPCALL(hipMemcpyAsync(g.dinplace, inPlace, nTiles, hipMemcpyHostToDevice, g.stream), st);
+    dIn = g.dinplace;
   }
   if (g.multi && !march) {  // classes admit only the march path
     if (st) st->code = 3;
@@ -1708,7 +1732,7 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
                          ? batch_fuse_mode(P, TX, TY, nTiles) : kFuseNone;
     if (launch_flux_stages(nTiles, dt, TX, TY, solveUpdate, fuse)) return 4;
     if (fuse == kFuseScratch) launch_update_finish(P, g.dtiles, nTiles, g.upd);
-    else if (fuse == kFuseNone && !solveUpdate) launch_update(nTiles, dt, dIn);
+    else if (fuse == kFuseNone && !solveUpdate && anyInPlace) launch_update(nTiles, dt, dIn);
     if (record(3)) return 4;
   } else {
   if (grow(&g.states, &g.statesCap, (size_t)P.scellsPerTile * kStateComps * nTiles, st)) return 4;
@@ -1729,7 +1753,6 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     else hipLaunchKernelGGL(k_fluxes<FX_HYBR>, gf, dim3(kThreads), 0, g.stream, P, L);
   }
   if (record(2)) return 4;
-  (void)anyFluxOnly;
   hipLaunchKernelGGL((k_update<true, false>), dim3(grid_for(P.icells * nTiles)), dim3(kThreads), 0,
                      g.stream, P, L, dIn);
   if (record(3)) return 4;
@@ -1880,6 +1903,11 @@ int upload_neighbors(double* U, long nBlocks, long blockStride, const int* nbr, 
   bool ok = g.init && U && nbr && nBlocks > 0 && blockStride >= P.ncell * P.nunk;
   for (int a = 0; ok && a < P.ndim; ++a)
     if (P.hi[a] - P.lo[a] + 1 < P.ng) ok = false;   // neighbours supply ng interior layers
+  // a table equal to the checked one on the device needs nothing more
+  const size_t n6 = ok ? (size_t)nBlocks * 6 : 0;
+  if (ok && g.nbrDim == P.ndim && g.hnbr.size() == n6 &&
+      memcmp(g.hnbr.data(), nbr, n6 * sizeof(int)) == 0)
+    return 0;
   for (long e = 0; ok && e < nBlocks * 6; ++e) {
     const int axis = (int)((e % 6) / 2);
     if (axis >= P.ndim) continue;
@@ -1890,12 +1918,11 @@ int upload_neighbors(double* U, long nBlocks, long blockStride, const int* nbr, 
     if (st) st->code = 3;
     return 3;
   }
-  const size_t n6 = (size_t)nBlocks * 6;
-  if (g.hnbr.size() != n6 || memcmp(g.hnbr.data(), nbr, n6 * sizeof(int)) != 0) {
-    if (grow(&g.dnbr, &g.dnbrCap, n6, st)) return 4;
-    g.hnbr.assign(nbr, nbr + n6);
-    HIPCALL(hipMemcpy(g.dnbr, g.hnbr.data(), n6 * sizeof(int), hipMemcpyHostToDevice), st);
-  }
+  g.nbrDim = 0;
+  if (grow(&g.dnbr, &g.dnbrCap, n6, st)) return 4;
+  g.hnbr.assign(nbr, nbr + n6);
+  HIPCALL(hipMemcpy(g.dnbr, g.hnbr.data(), n6 * sizeof(int), hipMemcpyHostToDevice), st);
+  g.nbrDim = P.ndim;
   return 0;
 }
 
@@ -2194,14 +2221,16 @@ int fx_hydro_init(const fx_params* p) {
   void* scratchAddr = nullptr;  // the no-allocation step's scratch on this device
   rc = noalloc_scratch(&scratchAddr, nullptr);
   if (rc) return rc;
+  if (pinned(sizeof(DevStatus), nullptr)) return 4;
   g.init = true;
   return 0;
 }
 
 void fx_hydro_finalize(void) {
-  void* bufs[] = {g.strongList, g.strongCount, g.dwCell, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.upd, g.dtiles, g.dinplace, g.status, g.partial,
+  if (g.hpin) (void)hipHostFree(g.hpin);
+  void* bufs[] = {g.strongList, g.strongCount, g.dcellChunks, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.upd, g.dtiles, g.dinplace, g.status, g.partial,
                   g.dregTiles, g.dfaces, g.mlpPacked, g.gradPart, g.seedPacked, g.seedY, g.fstates,
-                  g.dnbr, g.dtBuf, g.dcls, g.dtcls, g.dcellStart, g.dfaceStart,
+                  g.dnbr, g.dtBuf, g.dcls, g.dtcls, g.dfaceStart,
                   g.ditems, g.dregCls, g.seedFlux, g.seedBits};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -2237,8 +2266,8 @@ int fx_hydro_update_solution(const fx_tile* tiles, int nTiles, double dt, double
   Launch L{g.dtiles, nTiles, nullptr, g.status, dt, g.dtDev};
   hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
   if (g.multi) {
-    const ClassMap C{g.dcls, g.dtcls, g.dcellStart, g.dwCell};
-    hipLaunchKernelGGL(k_update_multi, dim3(grid_for(g.hcellStart[nTiles])), dim3(kThreads), 0,
+    const ClassMap C{g.dcls, g.dtcls, g.dcellChunks};
+    hipLaunchKernelGGL(k_update_multi, dim3((unsigned)g.nCellChunks), dim3(kThreads), 0,
                        g.stream, L, C, (const unsigned char*)nullptr);
   } else {
     hipLaunchKernelGGL((k_update<false, false>), dim3(grid_for(P.icells * nTiles)), dim3(kThreads),
@@ -2357,13 +2386,14 @@ int fx_hydro_compute_dt(const double* U, long nBlocks, long blockStride, const d
   }
   hipLaunchKernelGGL(k_dt, dim3(grid), dim3(kThreads), 0, g.stream, P, U, blockStride,
                      1. / del[0], 1. / del[1], 1. / del[2], cfl, nullptr, g.partial);
-  std::vector<double> h((size_t)grid);
-  if (hipMemcpyAsync(h.data(), g.partial, sizeof(double) * grid, hipMemcpyDeviceToHost, g.stream) !=
+  if (pinned(sizeof(double) * grid, nullptr)) return 4;
+  if (hipMemcpyAsync(g.hpin, g.partial, sizeof(double) * grid, hipMemcpyDeviceToHost, g.stream) !=
       hipSuccess)
     return 4;
   if (hipStreamSynchronize(g.stream) != hipSuccess) return 4;
+  const double* h = static_cast<const double*>(g.hpin);
   double m = 1.e300;  // Hydro_computeDt.F90:284-288: the smallest block dt
-  for (double v : h) m = v < m ? v : m;
+  for (int b = 0; b < grid; ++b) m = h[b] < m ? h[b] : m;
   *dtOut = m;
   return 0;
 }
@@ -2461,11 +2491,11 @@ int fx_riemann_batch(const double* states, long n, double gamma, const float* pa
 
 int fx_grid_fill_guards(double* U, long nBlocks, long blockStride, const int* nbr,
                         fx_status* st) {
-  return fx_grid_fill_guards_var(U, nBlocks, blockStride, nbr, -1, st);
+  return fx_grid_fill_guards_var(U, nBlocks, blockStride, nbr, -1, 1, st);
 }
 
 int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int* nbr, int var,
-                            fx_status* st) {
+                            int wait, fx_status* st) {
   if (st) memset(st, 0, sizeof *st);
   int rc = upload_neighbors(U, nBlocks, blockStride, nbr, st);
   if (!rc && var >= g.dp.nunk) {
@@ -2475,7 +2505,7 @@ int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int
   if (rc) return rc;
   launch_fill(U, nBlocks, blockStride, var);
   HIPCALL(hipGetLastError(), st);
-  if (g.async) return 0;
+  if (g.async || !wait) return 0;
   HIPCALL(hipStreamSynchronize(g.stream), st);
   return 0;
 }
@@ -2631,7 +2661,10 @@ int fx_hydro_set_block_classes(const int* nb, int nClasses) {
     if (p.ndim < 2 || p.nxb % 8 || p.nyb % 8) return 3;  // the column march's tiles
     cls.push_back(make_dev_params(p));
   }
-  if (nClasses > 0) {
+  // what is on the device already (every entry point sets its classes again)
+  // stays there
+  if (nClasses > 0 && (cls.size() != g.hcls.size() ||
+                       memcmp(cls.data(), g.hcls.data(), sizeof(DevParams) * nClasses) != 0)) {
     if (grow(&g.dcls, &g.dclsCap, (size_t)nClasses, nullptr)) return 4;
     if (hipMemcpy(g.dcls, cls.data(), sizeof(DevParams) * nClasses, hipMemcpyHostToDevice) !=
         hipSuccess)

@@ -183,14 +183,15 @@ class UniformGrid:
                            params.RiemannSolver.lower() == "hybrid")
         self._cfl_next = cfl          # the CFL the last step's flags and fallbacks left
 
-    def fill_guards(self, var: int = -1) -> None:
-        """Guard cells of every variable, or of the slot var alone."""
+    def fill_guards(self, var: int = -1, wait: bool = True) -> None:
+        """Guard cells of every variable, or of the slot var alone; wait=False
+        queues the fill in front of the next call on the library's stream."""
         import ctypes as C
         st = FxStatus()
         nb = self.U.shape[0]
         rc = self.lib.fx_grid_fill_guards_var(
             C.cast(C.c_void_p(self.U.data_ptr()), C.POINTER(C.c_double)), nb, self.U[0].numel(),
-            self.nbr.ctypes.data_as(C.POINTER(C.c_int)), var, C.byref(st))
+            self.nbr.ctypes.data_as(C.POINTER(C.c_int)), var, int(wait), C.byref(st))
         if rc:
             raise FxError("fx_grid_fill_guards_var", st, rc)
 
@@ -202,11 +203,11 @@ class UniformGrid:
         hy_fallbackLowerCFL the dt takes the CFL that the previous step's
         flags and fallbacks left (step_cfl)."""
         cfl = self._cfl_next
-        self.fill_guards()
+        self.fill_guards(wait=False)
         shock_cap = 0.0
         if self.detect:
             shock_cap = self.hydro.shock_detect_batch(self.U, self.deltas).min_cell_cfl
-            self.fill_guards(self.params.shokVar)
+            self.fill_guards(self.params.shokVar, wait=False)
         dt = min(self.hydro.compute_dt(self.U, self.deltas, cfl), dt_max)
         st = self.hydro.advance_batch(self.U, dt, self.deltas)
         self._cfl_next = step_cfl(self.cfl, cfl, self.detect, shock_cap, st.fallback_cfl)

@@ -20,7 +20,9 @@ from __future__ import annotations
 
 import ctypes as C
 import dataclasses
+import operator
 import os
+import struct
 from typing import List, Optional, Sequence
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -119,7 +121,7 @@ EXPORTS = {
     "fx_hydro_set_seed_params": ([C.POINTER(C.c_float)], C.c_int),
     "fx_mlp_set_gate": ([C.c_double], C.c_int),
     "fx_hydro_face_states": ([_DP, C.c_long, C.POINTER(C.c_long)], C.c_int),
-    "fx_grid_fill_guards_var": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_int,
+    "fx_grid_fill_guards_var": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_int, C.c_int,
                                  C.POINTER(FxStatus)], C.c_int),
     "fx_grid_fill_guards": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.POINTER(FxStatus)],
                             C.c_int),
@@ -273,15 +275,27 @@ class Tile:
     block_class: int = 0                  # index into Hydro.set_block_classes's shapes
 
 
-def _ptr(t) -> _DP:
+def _addr(t, tensor, float64) -> int:
+    """Device address of a checked tensor (0 for None); tensor and float64 are
+    torch's, looked up once by the caller."""
     if t is None:
-        return _DP()
-    import torch
-    if not isinstance(t, torch.Tensor):
+        return 0
+    if not isinstance(t, tensor):
         raise TypeError("expected a torch tensor")
-    if t.dtype != torch.float64 or not t.is_contiguous() or not t.is_cuda:
+    if t.dtype != float64 or not t.is_contiguous() or not t.is_cuda:
         raise ValueError("expected a contiguous float64 tensor on the GPU")
-    return C.cast(C.c_void_p(t.data_ptr()), _DP)
+    return t.data_ptr()
+
+
+def _ptr(t) -> _DP:
+    import torch
+    return C.cast(_addr(t, torch.Tensor, torch.float64), _DP)
+
+
+# FxTile's fields, packed in one call a tile (setting them one by one through
+# ctypes pointers took 12 us a tile)
+_TILE = struct.Struct("=5Q3d2i")
+assert _TILE.size == C.sizeof(FxTile)
 
 
 class Hydro:
@@ -437,17 +451,19 @@ class Hydro:
         self.lib.fx_hydro_set_stream(C.c_void_p(stream.cuda_stream if stream is not None else 0))
 
     def _tiles(self, tiles: Sequence[Tile]):
+        import torch
+        T, f8, pack, addr, size = torch.Tensor, torch.float64, _TILE.pack_into, _addr, _TILE.size
         arr = (FxTile * len(tiles))()
         for n, t in enumerate(tiles):
-            arr[n].U = _ptr(t.U)
-            for d in range(3):
-                f = t.flux[d] if (t.flux is not None and d < len(t.flux)) else None
-                arr[n].flux[d] = _ptr(f)
-            arr[n].pavg = _ptr(t.pavg)
-            for d in range(3):
-                arr[n].del_[d] = float(t.deltas[d]) if d < len(t.deltas) else 1.0
-            arr[n].level = t.level
-            arr[n].block_class = t.block_class
+            f = t.flux if t.flux is not None else ()
+            d = t.deltas
+            nf, nd = len(f), len(d)
+            pack(arr, n * size, addr(t.U, T, f8),
+                 addr(f[0], T, f8) if nf > 0 else 0, addr(f[1], T, f8) if nf > 1 else 0,
+                 addr(f[2], T, f8) if nf > 2 else 0, addr(t.pavg, T, f8),
+                 float(d[0]) if nd > 0 else 1.0, float(d[1]) if nd > 1 else 1.0,
+                 float(d[2]) if nd > 2 else 1.0, operator.index(t.level),
+                 operator.index(t.block_class))
         return arr
 
     def compute_fluxes(self, tiles: Sequence[Tile], dt: float, dtOld: float = 0.0,

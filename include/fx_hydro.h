@@ -289,9 +289,11 @@ enum { FX_BC_OUTFLOW = -1,   /* zero gradient */
 int fx_grid_fill_guards(double* U, long nBlocks, long blockStride, const int* nbr,
                         fx_status* st);
 /* The same for the variable slot var alone (< 0: every variable): after the
- * shock detector only SHOK_VAR's guard cells are out of date. */
+ * shock detector only SHOK_VAR's guard cells are out of date.  wait = 0 returns
+ * once the fill is queued on the library's stream, for a caller whose next call
+ * goes there too. */
 int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int* nbr, int var,
-                            fx_status* st);
+                            int wait, fx_status* st);
 
 /* Whole steps of a uniform grid captured in a HIP graph: each captured step
  * fills the guard cells (as fx_grid_fill_guards), computes the CFL dt on
