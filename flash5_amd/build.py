@@ -64,7 +64,8 @@ def _units():
     inst = os.path.join(CSRC, "fx_march_inst.hip")
     out = [(main, [], os.path.join(OBJ_DIR, "fx_hydro.o"))]
     for rs, r in MARCH_UNITS:
-        out.append((inst, [*MARCH_FLAGS, f"-DFX_MARCH_RS={rs}", f"-DFX_MARCH_R={r}"],
+        free = ["-DFX_MARCH_FREE"] if r == "double" and rs != "RS_STATES" else []
+        out.append((inst, [*MARCH_FLAGS, f"-DFX_MARCH_RS={rs}", f"-DFX_MARCH_R={r}", *free],
                     os.path.join(OBJ_DIR, f"fx_march_{rs.lower()}_{r}.o")))
     return out
 

@@ -1136,14 +1136,50 @@ bool march_shape(const DevParams& P, int* TX, int* TY, int* NT) {
   return true;
 }
 
-// Whether a batch step runs the update inside the march: HLLC, HLL and the
-// hybrid switch, the whole pressure in the momentum flux (the update's
+// Column tiles of a block that no fixed tile divides: the fewest equal ones
+// that fit the 16x8 layout, the last along an axis with what is left.
+bool free_shape(const DevParams& P, int* tx, int* ty) {
+  if (P.ndim < 2) return false;
+  int best = 1 << 30;
+  for (int nx = 1; nx <= P.nxb; ++nx)
+    for (int ny = 1; ny <= P.nyb; ++ny) {
+      const int x = (P.nxb + nx - 1) / nx, y = (P.nyb + ny - 1) / ny;
+      if (nx * ny < best && free_tile_fits<16, 8>(x, y)) {
+        best = nx * ny;
+        *tx = x;
+        *ty = y;
+      }
+    }
+  return best < 1 << 30;
+}
+
+// Whether n blocks step faster by free column tiles than by the three-kernel
+// path.  In 3-D a column tile takes a compute unit for its planes and three
+// more, about 4 us each and 6 more with all 128 columns in use; the three
+// kernels take about 0.27 ns a state cell and 40 us for their launches and
+// latency, however few the blocks.  Measured either side of the line, free
+// against three kernels: 12 blocks of 20^3 226 / 120 us and 200 887 / 1284,
+// 28 of 9 x 7 x 11 125 / 75 and 144 134 / 152, 59 of 12 x 10 x 14 158 / 134
+// and 238 179 / 395, 92 of 6^3 71 / 79.  In 2-D (one plane) free tiles were
+// faster at every size: 200 blocks of 10^2 32 / 52, 1250 of 20 x 16 173 / 175,
+// 16000 of 10^2 490 / 764.
+bool free_pays(const DevParams& P, long n, int tx, int ty) {
+  if (P.ndim == 2) return true;
+  const long tiles = (long)((P.nxb + tx - 1) / tx) * ((P.nyb + ty - 1) / ty);
+  const long rounds = (n * tiles + g.numCU - 1) / g.numCU;
+  const double cols = (double)(P.nxb * P.nyb) / (double)(tiles * 128);
+  return (double)(rounds * (P.nzb + 3)) * (4.0 + 6.0 * cols) <
+         40.0 + 0.27e-3 * (double)P.scellsPerTile * (double)n;
+}
+
+// Whether a batch step of n blocks runs the update inside the march: HLLC, HLL
+// and the hybrid switch, the whole pressure in the momentum flux (the update's
 // pressure source, which the fused form does not carry, is then zero), unless
 // the kernel path asks for a separate update.
-bool batch_fused(const DevParams& P) {
-  int TX, TY, NT;
-  return !g.legacy && !g.solveUpdOff && P.riemann != FX_EXACT && P.fP == 1.0 &&
-         march_shape(P, &TX, &TY, &NT);
+bool batch_fused(const DevParams& P, long n) {
+  int tx, ty, NT;
+  if (g.legacy || g.solveUpdOff || P.riemann == FX_EXACT || P.fP != 1.0) return false;
+  return march_shape(P, &tx, &ty, &NT) || (free_shape(P, &tx, &ty) && free_pays(P, n, tx, ty));
 }
 
 // Where the update of n such blocks runs.  kFuseDirect gives a block's column
@@ -1157,7 +1193,7 @@ bool batch_fused(const DevParams& P) {
 // short, and taking two in turn costs more than k_update_finish (4096 x 16^2
 // mixed: 190 against 152 + 25 us): blocks of one tile only.
 int batch_fuse_mode(const DevParams& P, int TX, int TY, long n) {
-  if (!batch_fused(P)) return kFuseNone;
+  if (!batch_fused(P, n)) return kFuseNone;
   const long tiles = P.nyb / TY;
   if (P.nxb != TX || (P.ndim == 3 && P.steep) || (P.ndim == 2 && tiles > 1)) return kFuseScratch;
   // resident workgroups: the FP64 16x8 tile takes a CU's LDS
@@ -1619,6 +1655,22 @@ void launch_update_finish(const DevParams& P, const fx_tile* tiles, int nTiles, 
                      P, tiles, nTiles, upd);
 }
 
+// a step of blocks that only free column tiles divide (free_shape), FP64
+int launch_free(const DevParams& P, int nTiles, double dt) {
+  MarchLaunch M{g.dtiles, nTiles, 0, 0, g.status, dt, nullptr, g.dtDev, kFuseScratch, g.upd};
+  free_shape(P, &M.tx, &M.ty);
+  M.tilesX = (P.nxb + M.tx - 1) / M.tx;
+  M.tilesY = (P.nyb + M.ty - 1) / M.ty;
+  // a block of one tile is updated in place, unless the steepening still
+  // reads planes that the update has written by then
+  if (M.tilesX * M.tilesY == 1 && !(P.ndim == 3 && P.steep)) M.fuse = kFuseDirect;
+  if (P.riemann == FX_HLLC) launch_march_free<FX_HLLC>(P, M, g.stream);
+  else launch_march_free<FX_HYBR>(P, M, g.stream);
+  if (record(1) || record(2)) return 4;
+  if (M.fuse == kFuseScratch) launch_update_finish(P, g.dtiles, nTiles, g.upd);
+  return 0;
+}
+
 // update stage of a step on the uploaded tiles (dIn: per-tile in-place flags
 // on the device, or null for all)
 void launch_update(int nTiles, double dt, const unsigned char* dIn) {
@@ -1733,6 +1785,11 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     if (launch_flux_stages(nTiles, dt, TX, TY, solveUpdate, fuse)) return 4;
     if (fuse == kFuseScratch) launch_update_finish(P, g.dtiles, nTiles, g.upd);
     else if (fuse == kFuseNone && !solveUpdate && anyInPlace) launch_update(nTiles, dt, dIn);
+    if (record(3)) return 4;
+  } else if (tilesUploaded && !tiles && !inPlace && !g.multi && batch_fused(P, nTiles)) {
+    if (!g.capturing) hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
+    if (record(0)) return 4;
+    if (launch_free(P, nTiles, dt)) return 4;
     if (record(3)) return 4;
   } else {
   if (grow(&g.states, &g.statesCap, (size_t)P.scellsPerTile * kStateComps * nTiles, st)) return 4;
@@ -1885,7 +1942,7 @@ int prepare_batch(double* U, long nBlocks, long blockStride, const double del[3]
       t.level = 1;
     }
     // a fused step keeps no fluxes in memory, only the updated states
-    const bool fused = batch_fused(g.dp);
+    const bool fused = batch_fused(g.dp, nBlocks);
     if (fused && grow(&g.upd, &g.updCap, (size_t)(kUpdComps * g.dp.icells * nBlocks), st)) return 4;
     if (upload_tiles(tl.data(), (int)nBlocks, !fused, st, false)) return 4;
     g.batchU = U;

@@ -29,29 +29,89 @@
 
 namespace fx {
 
-// LDS index helpers, tile-local coordinates a = i - ox, b = j - oy
+// array sizes and stage-A item counts of a column tile of TX x TY columns
 template <int TX, int TY> struct TileIdx {
-  // R_x: a in [0,TX), b in [-1,TY]   (sigma_x, y-face states)
-  static __device__ __forceinline__ int rx(int a, int b) { return (b + 1) * TX + a; }
-  // R_y: a in [-1,TX], b in [0,TY)   (sigma_y, x-face states)
-  static __device__ __forceinline__ int ry(int a, int b) { return b * (TX + 2) + (a + 1); }
-  // C: a in [-1,TX], b in [-1,TY]    (sigma_z)
-  static __device__ __forceinline__ int cc(int a, int b) { return (b + 1) * (TX + 2) + (a + 1); }
-  // slopes along x: a in [-2,TX+1], b in [0,TY)
-  static __device__ __forceinline__ int lx(int a, int b) { return b * (TX + 4) + (a + 2); }
-  // slopes along y: a in [0,TX), b in [-2,TY+1]
-  static __device__ __forceinline__ int ly(int a, int b) { return (b + 2) * TX + a; }
   static constexpr int NRX = TX * (TY + 2), NRY = (TX + 2) * TY, NC = (TX + 2) * (TY + 2);
   static constexpr int NLX = (TX + 4) * TY, NLY = TX * (TY + 4);
-  // x faces: a in [0, TX], b in [0, TY); y faces: a in [0, TX), b in [0, TY]
-  static __device__ __forceinline__ int ux(int a, int b) { return b * (TX + 1) + a; }
-  static __device__ __forceinline__ int uy(int a, int b) { return b * TX + a; }
   static constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1);
   // stage-A items along x: the cells of R_x and of the x slopes, rows
   // b = -1, [0,TY), TY; along y: the cells of R_y and of the y slopes,
   // rows b = -2, -1, [0,TY), TY, TY+1
   static constexpr int NUX = 2 * TX + (TX + 4) * TY, NUY = 4 * TX + (TX + 2) * TY;
 };
+
+// The extents of a column tile and the row arithmetic of its items.  Fixed:
+// the template's.  Free: any extents that fit the TX x TY layout's arrays and
+// thread roles (free_tile_fits), for blocks that no fixed tile divides; the
+// component strides stay the layout's, only the rows' are the tile's own.
+template <int TX, int TY> struct FixedShape {
+  static constexpr bool kFree = false;
+  static __device__ __forceinline__ int tx() { return TX; }
+  static __device__ __forceinline__ int ty() { return TY; }
+  // rows of tx, tx + 2 and tx + 4 items: a the place in the row, b the row
+  static __device__ __forceinline__ void row(int w, int& a, int& b) { a = w % TX; b = w / TX; }
+  static __device__ __forceinline__ void row2(int w, int& a, int& b) {
+    a = w % (TX + 2);
+    b = w / (TX + 2);
+  }
+  static __device__ __forceinline__ void row4(int w, int& a, int& b) {
+    a = w % (TX + 4);
+    b = w / (TX + 4);
+  }
+};
+struct FreeShape {
+  static constexpr bool kFree = true;
+  int x, y;
+  unsigned m0, m2, m4;  // reciprocals of x, x + 2 and x + 4
+  __device__ __forceinline__ FreeShape(int x_, int y_)
+      : x(x_), y(y_), m0(65536u / (unsigned)x_ + 1u), m2(65536u / (unsigned)(x_ + 2) + 1u),
+        m4(65536u / (unsigned)(x_ + 4) + 1u) {}
+  __device__ __forceinline__ int tx() const { return x; }
+  __device__ __forceinline__ int ty() const { return y; }
+  // w / d = (w m) >> 16: exact while w d < 65536 (w < 256, d <= 140 here)
+  static __device__ __forceinline__ void part(int w, int d, unsigned m, int& a, int& b) {
+    b = (int)(__umul24((unsigned)w, m) >> 16);
+    a = w - b * d;
+  }
+  __device__ __forceinline__ void row(int w, int& a, int& b) const { part(w, x, m0, a, b); }
+  __device__ __forceinline__ void row2(int w, int& a, int& b) const { part(w, x + 2, m2, a, b); }
+  __device__ __forceinline__ void row4(int w, int& a, int& b) const { part(w, x + 4, m4, a, b); }
+};
+// LDS index helpers, tile-local coordinates a = i - ox, b = j - oy, and item
+// counts of a tile of tx x ty columns:
+//   R_x (rx)  a in [0, tx), b in [-1, ty]      sigma_x, y state cells
+//   R_y (ry)  a in [-1, tx], b in [0, ty)      sigma_y, x state cells
+//   C (cc)    a in [-1, tx], b in [-1, ty]     sigma_z
+//   lx        a in [-2, tx + 1], b in [0, ty)  slopes along x
+//   ly        a in [0, tx), b in [-2, ty + 1]  slopes along y
+//   ux        a in [0, tx], b in [0, ty)       x faces
+//   uy        a in [0, tx), b in [0, ty]       y faces
+template <typename S> struct ShapeIdx {
+  S s;
+  __device__ __forceinline__ int rx(int a, int b) const { return (b + 1) * s.tx() + a; }
+  __device__ __forceinline__ int ry(int a, int b) const { return b * (s.tx() + 2) + (a + 1); }
+  __device__ __forceinline__ int cc(int a, int b) const { return (b + 1) * (s.tx() + 2) + (a + 1); }
+  __device__ __forceinline__ int lx(int a, int b) const { return b * (s.tx() + 4) + (a + 2); }
+  __device__ __forceinline__ int ly(int a, int b) const { return (b + 2) * s.tx() + a; }
+  __device__ __forceinline__ int ux(int a, int b) const { return b * (s.tx() + 1) + a; }
+  __device__ __forceinline__ int uy(int a, int b) const { return b * s.tx() + a; }
+  __device__ __forceinline__ int nrx() const { return s.tx() * (s.ty() + 2); }
+  __device__ __forceinline__ int nry() const { return (s.tx() + 2) * s.ty(); }
+  __device__ __forceinline__ int nc() const { return (s.tx() + 2) * (s.ty() + 2); }
+  __device__ __forceinline__ int ncol() const { return s.tx() * s.ty(); }
+  __device__ __forceinline__ int nux() const { return 2 * s.tx() + (s.tx() + 4) * s.ty(); }
+  __device__ __forceinline__ int nuy() const { return 4 * s.tx() + (s.tx() + 2) * s.ty(); }
+};
+// Whether a free tile of tx x ty columns fits the TX x TY layout: its LDS
+// arrays, its wave-aligned stage-A segments and its one state cell per thread
+template <int TX, int TY> constexpr bool free_tile_fits(int tx, int ty) {
+  using I = TileIdx<TX, TY>;
+  return tx >= 1 && ty >= 1 && tx * (ty + 2) <= I::NRX && (tx + 2) * ty <= I::NRY &&
+         (tx + 2) * (ty + 2) <= I::NC && (tx + 4) * ty <= I::NLX && tx * (ty + 4) <= I::NLY &&
+         (tx + 1) * ty <= I::NFX && tx * (ty + 1) <= I::NFY && tx * ty <= TX * TY &&
+         2 * tx + (tx + 4) * ty <= (I::NUX + 63) / 64 * 64 &&
+         4 * tx + (tx + 2) * ty <= (I::NUY + 63) / 64 * 64;
+}
 
 // LDS of one column tile (march_tile), as offsets into one array of R.
 // FUSE: with the plane's face fluxes and face-averaged pressures.
@@ -104,6 +164,7 @@ struct MarchLaunch {
   const double* dtp;   // device-resident dt (graph-captured steps), or null
   int fuse;            // where the update runs (kFuse*)
   double* upd;         // fused update: updated states, [tile][component][interior cell]
+  int tx, ty;          // free tiles: columns of a tile (the last along an axis may have fewer)
 };
 // components of a cell's fused-update scratch: density, velocities, eint (the
 // sixth only in the FP32 march, on the way)
@@ -384,10 +445,10 @@ __device__ __forceinline__ void lds_barrier() {
 // tildes formed by the state cells) the step of 4096 x 16^3 went from 10.17
 // to 8.89 ms (FP64 HLLC), of 2048 x 16^3 from 3.41 to 3.07 ms (mixed) and of
 // 1024 x 16^3 from 3.52 to 3.15 ms (FP64 exact).
-template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE, int FUSE>
+template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE, int FUSE, typename SH>
 __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch& L,
                                            const fx_tile& T, int t, int ox, int oy, R* fsb,
-                                           ExactStats& es, R* smem) {
+                                           ExactStats& es, R* smem, const SH shape) {
   using I = TileIdx<TX, TY>;
   using M = MarchLds<NDIM, TX, TY, FUSE>;
   constexpr int NR = NDIM == 3 ? 3 : 1;        // ring depth
@@ -413,12 +474,14 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   R* const PA = smem + M::PA;
 
   const int tid = threadIdx.x;
+  const ShapeIdx<SH> X{shape};
+  const int tx = shape.tx(), ty = shape.ty();
   // A tile owns its high x (y) face row only at the block's high side;
   // otherwise the neighbouring tile computes that row (and the states
   // behind it) as its low row.  The fused update needs that row's fluxes in
   // either case, so there both tiles compute it.
-  const bool ex = (ox + TX > P.hi[0]);
-  const bool ey = (oy + TY > P.hi[1]);
+  const bool ex = (ox + tx > P.hi[0]);
+  const bool ey = (oy + ty > P.hi[1]);
   const TileView tv = tile_view(P, as_global(T.U));
   double dt = step_dt(L.dt, L.dtp);
   // (opaque: a workgroup that takes a block's tiles in turn would otherwise
@@ -449,13 +512,17 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   // stage-A items: sigma_x (w < NRX) and sigma_y (w < NRY) of plane kk
   auto sig_x_item = [&](int w, int kk) {
     R sg[8];
-    const int a = w % TX, b = w / TX - 1;
+    int a, b;
+    shape.row(w, a, b);
+    --b;
     bad |= !tv_sigma<0>(P, tv, cell_b(P, ox + a, oy + b, kk), sxb, sg);
     lds_put6(SX + ring(kk) * 6 * I::NRX, I::NRX, w, sg);
   };
   auto sig_y_item = [&](int w, int kk) {
     R sg[8];
-    const int a = w % (TX + 2) - 1, b = w / (TX + 2);
+    int a, b;
+    shape.row2(w, a, b);
+    --a;
     bad |= !tv_sigma<1>(P, tv, cell_b(P, ox + a, oy + b, kk), syb, sg);
     lds_put6(SY + ring(kk) * 6 * I::NRY, I::NRY, w, sg);
   };
@@ -468,19 +535,18 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   // neighbour's in diverged branches) and five more loads.
   auto x_item = [&](int w, int p, bool sig, bool sl) {
     int a, b;
-    if (w < TX) {
+    if (w < tx) {
       a = w;
       b = -1;
-    } else if (w < TX + (TX + 4) * TY) {
-      const int u = w - TX;
-      a = u % (TX + 4) - 2;
-      b = u / (TX + 4);
+    } else if (w < tx + (tx + 4) * ty) {
+      shape.row4(w - tx, a, b);
+      a -= 2;
     } else {
-      a = w - TX - (TX + 4) * TY;
-      b = TY;
+      a = w - tx - (tx + 4) * ty;
+      b = ty;
     }
-    const bool doS = sig && a >= 0 && a < TX;
-    const bool doL = sl && b >= 0 && b < TY;
+    const bool doS = sig && a >= 0 && a < tx;
+    const bool doL = sl && b >= 0 && b < ty;
     if (!doS && !doL) return;
     const unsigned cb = cell_b(P, ox + a, oy + b, p);
     R Vm[8], Vc[8], Vp[8];
@@ -492,34 +558,32 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     if (doS) {
       R sg[8];
       trans_sigma<0>(P, Vm, Vc, Vp, e, sg);
-      lds_put6(SX + ring(p) * 6 * I::NRX, I::NRX, I::rx(a, b), sg);
+      lds_put6(SX + ring(p) * 6 * I::NRX, I::NRX, X.rx(a, b), sg);
     }
     if (doL) {
       R db[8];
       tvd_slope<0>(P, Vm, Vc, Vp, e, db);
-      lds_put6(LX + ringL(p) * 6 * I::NLX, I::NLX, I::lx(a, b), db);
+      lds_put6(LX + ringL(p) * 6 * I::NLX, I::NLX, X.lx(a, b), db);
       if (P.flat)
-        FX[ringL(p) * I::NLX + I::lx(a, b)] =
+        FX[ringL(p) * I::NLX + X.lx(a, b)] =
             flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * sxb)), Vm[P_PRES], Vp[P_PRES],
                             R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * sxb)), Vm[P_VELX], Vp[P_VELX]);
     }
   };
   auto y_item = [&](int w, int p, bool sig, bool sl) {
     int a, b;
-    if (w < 2 * TX) {
-      a = w % TX;
-      b = w / TX - 2;
-    } else if (w < 2 * TX + (TX + 2) * TY) {
-      const int u = w - 2 * TX;
-      a = u % (TX + 2) - 1;
-      b = u / (TX + 2);
+    if (w < 2 * tx) {
+      shape.row(w, a, b);
+      b -= 2;
+    } else if (w < 2 * tx + (tx + 2) * ty) {
+      shape.row2(w - 2 * tx, a, b);
+      --a;
     } else {
-      const int u = w - 2 * TX - (TX + 2) * TY;
-      a = u % TX;
-      b = TY + u / TX;
+      shape.row(w - 2 * tx - (tx + 2) * ty, a, b);
+      b += ty;
     }
-    const bool doS = sig && b >= 0 && b < TY;
-    const bool doL = sl && a >= 0 && a < TX;
+    const bool doS = sig && b >= 0 && b < ty;
+    const bool doL = sl && a >= 0 && a < tx;
     if (!doS && !doL) return;
     const unsigned cb = cell_b(P, ox + a, oy + b, p);
     R Vm[8], Vc[8], Vp[8];
@@ -531,21 +595,22 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     if (doS) {
       R sg[8];
       trans_sigma<1>(P, Vm, Vc, Vp, e, sg);
-      lds_put6(SY + ring(p) * 6 * I::NRY, I::NRY, I::ry(a, b), sg);
+      lds_put6(SY + ring(p) * 6 * I::NRY, I::NRY, X.ry(a, b), sg);
     }
     if (doL) {
       R db[8];
       tvd_slope<1>(P, Vm, Vc, Vp, e, db);
-      lds_put6(LY + ringL(p) * 6 * I::NLY, I::NLY, I::ly(a, b), db);
+      lds_put6(LY + ringL(p) * 6 * I::NLY, I::NLY, X.ly(a, b), db);
       if (P.flat)
-        FY[ringL(p) * I::NLY + I::ly(a, b)] =
+        FY[ringL(p) * I::NLY + X.ly(a, b)] =
             flat_tilde_vals(R(tv_ld(tv, tv.ob[P_PRES], cb - 2 * syb)), Vm[P_PRES], Vp[P_PRES],
                             R(tv_ld(tv, tv.ob[P_PRES], cb + 2 * syb)), Vm[P_VELY], Vp[P_VELY]);
     }
   };
   // stage-A item: z-slope and z flattening tilde of column w at plane m
   auto zslope_item = [&](int w, int m) {
-    const int a = w % TX, b = w / TX;
+    int a, b;
+    shape.row(w, a, b);
     const unsigned cb = cell_b(P, ox + a, oy + b, m);
     R db[8], Vm[8], Vc[8], Vp[8];
     tv_prim(tv, cb - szb, Vm);
@@ -587,24 +652,27 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
     const bool wSig = !Z || k + 1 <= kEnd;
     const bool wL = !Z || (k + 1 >= klo && k + 1 <= khi);
     const bool uXY = wSig || wL;
-    const int nSz = (Z && interiorA) ? I::NC : 0;
-    const int nZs = Z ? NCOL : 0;
+    const int nSz = (Z && interiorA) ? X.nc() : 0;
+    const int nZs = Z ? X.ncol() : 0;
     constexpr int PUX = wave_up(I::NUX), PUY = wave_up(I::NUY), PZ4 = wave_up(I::NC);
     const int s1 = uXY ? PUX + PUY : 0, s2 = s1 + (nSz ? PZ4 : 0), sEnd = s2 + nZs;
     auto itemA = [&](int v) {
       if (v < s1) {
         if (v < PUX) {
-          if (v < I::NUX) x_item(v, pA, wSig, wL);
-        } else if (v - PUX < I::NUY) {
+          if (v < X.nux()) x_item(v, pA, wSig, wL);
+        } else if (v - PUX < X.nuy()) {
           y_item(v - PUX, pA, wSig, wL);
         }
         return;
       }
       if (v < s2) {
         const int r = v - s1;
-        if (r >= I::NC) return;
+        if (r >= X.nc()) return;
         R v8[8];
-        const int a = r % (TX + 2) - 1, b = r / (TX + 2) - 1;
+        int a, b;
+        shape.row2(r, a, b);
+        --a;
+        --b;
         bad |= !tv_sigma<2>(P, tv, cell_b(P, ox + a, oy + b, k), szb, v8);
         lds_put6(SZ, I::NC, r, v8);
         return;
@@ -616,10 +684,10 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   if (Z) {
     // prologue: sigma_x/y of plane kBeg, z slopes of kBeg-1 and kBeg
     constexpr int Q1 = wave_up(I::NRX), Q2 = Q1 + wave_up(I::NRY), Q3 = Q2 + wave_up(NCOL);
-    for (int w = tid; w < Q3 + NCOL; w += NT) {
-      if (w < Q1) { if (w < I::NRX) sig_x_item(w, kBeg); }
-      else if (w < Q2) { if (w - Q1 < I::NRY) sig_y_item(w - Q1, kBeg); }
-      else if (w < Q3) { if (w - Q2 < NCOL) zslope_item(w - Q2, kBeg - 1); }
+    for (int w = tid; w < Q3 + X.ncol(); w += NT) {
+      if (w < Q1) { if (w < X.nrx()) sig_x_item(w, kBeg); }
+      else if (w < Q2) { if (w - Q1 < X.nry()) sig_y_item(w - Q1, kBeg); }
+      else if (w < Q3) { if (w - Q2 < X.ncol()) zslope_item(w - Q2, kBeg - 1); }
       else zslope_item(w - Q3, kBeg);
     }
   }
@@ -681,8 +749,9 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   };
   auto stageD = [&](int k) {
     const int w = item_index<OPAQUE>(tid) - D0;
-    if (w < 0 || w >= NCOL) return;
-    const int a = w % TX, b = w / TX;
+    if (w < 0 || w >= X.ncol()) return;
+    int a, b;
+    shape.row(w, a, b);
     double F0[8], F1[8];
     double S;  // the pressure source: zero (the whole pressure is in the flux)
     gdouble* const upd = as_global(L.upd + (long)t * (kUpdComps * P.icells));
@@ -693,7 +762,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
       part.IntEner = cI;
       part.S1 = part.S2 = 0.;
       const UpdState u = upd_state(P, dt, part, eintOld);
-      if (FUSE == kFuseDirect && (b < TY - kSeamRows || ey)) {
+      if (FUSE == kFuseDirect && (b < ty - kSeamRows || ey)) {
         tv_expand(P, tv, cell_b(P, ox + a, oy + b, kk), u);
         return;
       }
@@ -728,11 +797,11 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
 #pragma unroll
       for (int q = 0; q < 5; ++q) cU[q] = part.U0[q];
       cI = part.IntEner;
-      get_flux(UX, I::NFX, I::ux(a, b), F0);
-      get_flux(UX, I::NFX, I::ux(a + 1, b), F1);
+      get_flux(UX, I::NFX, X.ux(a, b), F0);
+      get_flux(UX, I::NFX, X.ux(a + 1, b), F1);
       upd_dir(P, dt, dx, double(cP), F0, F1, cU, cI, S);
-      get_flux(UY, I::NFY, I::uy(a, b), F0);
-      get_flux(UY, I::NFY, I::uy(a, b + 1), F1);
+      get_flux(UY, I::NFY, X.uy(a, b), F0);
+      get_flux(UY, I::NFY, X.uy(a, b + 1), F1);
       upd_dir(P, dt, dy, double(cP), F0, F1, cU, cI, S);
       if (Z && !CARRY) {
         const unsigned r = cell_r(ox + a, oy + b, kc) * 8u;
@@ -763,29 +832,31 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
         R sm[8], sc[8], sp[8], tA[8], tB[8];
         EigT<R> e0, e1, e2;
         if (w < B1) {
-          if (!interior || w >= NBX) return;
-          const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-          if (a == TX && !ex && !FUSE) return;
+          if (!interior || w >= X.nry()) return;
+          int a, b;
+          shape.row2(w, a, b);
+          --a;
+          if (a == tx && !ex && !FUSE) return;
           // the tile owns this state cell (and counts its reset)
-          const bool own = (a >= 0 || ox == P.lo[0]) && (a < TX || ex);
+          const bool own = (a >= 0 || ox == P.lo[0]) && (a < tx || ex);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - sxb, Vm);
           tv_prim(tv, cb, Vc);
           tv_prim(tv, cb + sxb, Vp);
-          const R* fx = FX + ringL(k) * I::NLX + I::lx(a, b);
+          const R* fx = FX + ringL(k) * I::NLX + X.lx(a, b);
           const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], fx[-1], fx[0], fx[1]) : R(0.);
           const R* lxk = LX + ringL(k) * 6 * I::NLX;
-          lds_get6(lxk, I::NLX, I::lx(a - 1, b), dbN);
-          lds_get6(lxk, I::NLX, I::lx(a, b), db0);
-          lds_get6(lxk, I::NLX, I::lx(a + 1, b), dbP);
+          lds_get6(lxk, I::NLX, X.lx(a - 1, b), dbN);
+          lds_get6(lxk, I::NLX, X.lx(a, b), db0);
+          lds_get6(lxk, I::NLX, X.lx(a + 1, b), dbP);
           bad |= !eig_make<0>(Vc, e0);
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * sxb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * sxb)) : R(0.);
           ppm_trace<0>(P, ratio(0), ratio(9), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          lds_get6(syk, I::NRY, I::ry(a, b), sg);
+          lds_get6(syk, I::NRY, X.ry(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(4));
           if (Z) {
-            lds_get6(SZ, I::NC, I::cc(a, b), sc);
+            lds_get6(SZ, I::NC, X.cc(a, b), sc);
             sub_sigma(Wp, Wn, sc, ratio(5));
           }
           if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
@@ -794,42 +865,44 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             e1 = e2 = e0;
             e1.un = Vc[P_VELY];
             e2.un = Vc[P_VELZ];
-            lds_get6(SZ, I::NC, I::cc(a, b - 1), sm);
-            lds_get6(SZ, I::NC, I::cc(a, b + 1), sp);
+            lds_get6(SZ, I::NC, X.cc(a, b - 1), sm);
+            lds_get6(SZ, I::NC, X.cc(a, b + 1), sp);
             trans_sigma<1>(P, sm, sc, sp, e1, tA);
-            lds_get6(SY + ring(k - 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sm);
-            lds_get6(SY + ring(k + 1) * 6 * I::NRY, I::NRY, I::ry(a, b), sp);
+            lds_get6(SY + ring(k - 1) * 6 * I::NRY, I::NRY, X.ry(a, b), sm);
+            lds_get6(SY + ring(k + 1) * 6 * I::NRY, I::NRY, X.ry(a, b), sp);
             trans_sigma<2>(P, sm, sg, sp, e2, tB);
             add_ctu(Wp, Wn, tA, tB, ratio(6));
             if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
           }
-          lds_put6(WX, I::NRY, I::ry(a, b), Wp);
+          lds_put6(WX, I::NRY, X.ry(a, b), Wp);
           psum = Wn[P_PRES] + Wp[P_PRES];
           keep(Wn);
         } else if (w < B2) {
           const int w2 = w - B1;
-          if (!interior || w2 >= NBY) return;
-          const int a = w2 % TX, b = w2 / TX - 1;
-          if (b == TY && !ey && !FUSE) return;
-          const bool own = (b >= 0 || oy == P.lo[1]) && (b < TY || ey);
+          if (!interior || w2 >= X.nrx()) return;
+          int a, b;
+          shape.row(w2, a, b);
+          --b;
+          if (b == ty && !ey && !FUSE) return;
+          const bool own = (b >= 0 || oy == P.lo[1]) && (b < ty || ey);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - syb, Vm);
           tv_prim(tv, cb, Vc);
           tv_prim(tv, cb + syb, Vp);
-          const R* fy = FY + ringL(k) * I::NLY + I::ly(a, b);
-          const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], fy[-TX], fy[0], fy[TX]) : R(0.);
+          const R* fy = FY + ringL(k) * I::NLY + X.ly(a, b);
+          const R flat = P.flat ? flat_of(Vm[P_PRES], Vp[P_PRES], fy[-tx], fy[0], fy[tx]) : R(0.);
           const R* lyk = LY + ringL(k) * 6 * I::NLY;
-          lds_get6(lyk, I::NLY, I::ly(a, b - 1), dbN);
-          lds_get6(lyk, I::NLY, I::ly(a, b), db0);
-          lds_get6(lyk, I::NLY, I::ly(a, b + 1), dbP);
+          lds_get6(lyk, I::NLY, X.ly(a, b - 1), dbN);
+          lds_get6(lyk, I::NLY, X.ly(a, b), db0);
+          lds_get6(lyk, I::NLY, X.ly(a, b + 1), dbP);
           bad |= !eig_make<1>(Vc, e0);
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * syb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * syb)) : R(0.);
           ppm_trace<1>(P, ratio(1), ratio(10), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          lds_get6(sxk, I::NRX, I::rx(a, b), sg);
+          lds_get6(sxk, I::NRX, X.rx(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(3));
           if (Z) {
-            lds_get6(SZ, I::NC, I::cc(a, b), sc);
+            lds_get6(SZ, I::NC, X.cc(a, b), sc);
             sub_sigma(Wp, Wn, sc, ratio(5));
           }
           if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
@@ -838,21 +911,23 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             e1 = e2 = e0;
             e1.un = Vc[P_VELZ];
             e2.un = Vc[P_VELX];
-            lds_get6(SX + ring(k - 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sm);
-            lds_get6(SX + ring(k + 1) * 6 * I::NRX, I::NRX, I::rx(a, b), sp);
+            lds_get6(SX + ring(k - 1) * 6 * I::NRX, I::NRX, X.rx(a, b), sm);
+            lds_get6(SX + ring(k + 1) * 6 * I::NRX, I::NRX, X.rx(a, b), sp);
             trans_sigma<2>(P, sm, sg, sp, e1, tA);
-            lds_get6(SZ, I::NC, I::cc(a - 1, b), sm);
-            lds_get6(SZ, I::NC, I::cc(a + 1, b), sp);
+            lds_get6(SZ, I::NC, X.cc(a - 1, b), sm);
+            lds_get6(SZ, I::NC, X.cc(a + 1, b), sp);
             trans_sigma<0>(P, sm, sc, sp, e2, tB);
             add_ctu(Wp, Wn, tA, tB, ratio(7));
             if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
           }
-          lds_put6(WY, I::NRX, I::rx(a, b), Wp);
-          PY[I::rx(a, b)] = Wn[P_PRES] + Wp[P_PRES];
+          lds_put6(WY, I::NRX, X.rx(a, b), Wp);
+          PY[X.rx(a, b)] = Wn[P_PRES] + Wp[P_PRES];
           keep(Wn);
         } else if (Z && w < B3) {
           const int w2 = w - B2;
-          const int a = w2 % TX, b = w2 / TX;
+          if (SH::kFree && w2 >= X.ncol()) return;
+          int a, b;
+          shape.row(w2, a, b);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
           tv_prim(tv, cb - szb, Vm);
           tv_prim(tv, cb, Vc);
@@ -867,9 +942,9 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const R dmm = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb - 2 * szb)) : R(0.);
           const R dpp = P.steep ? R(tv_ld(tv, tv.ob[P_DENS], cb + 2 * szb)) : R(0.);
           ppm_trace<2>(P, ratio(2), ratio(11), Vm, Vc, Vp, dmm, dpp, dbN, db0, dbP, flat, e0, Wp, Wn);
-          lds_get6(sxk, I::NRX, I::rx(a, b), sc);
+          lds_get6(sxk, I::NRX, X.rx(a, b), sc);
           sub_sigma(Wp, Wn, sc, ratio(3));
-          lds_get6(syk, I::NRY, I::ry(a, b), sg);
+          lds_get6(syk, I::NRY, X.ry(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(4));
           if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
           if (P.ctu3d) {
@@ -877,11 +952,11 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             e1 = e2 = e0;
             e1.un = Vc[P_VELX];
             e2.un = Vc[P_VELY];
-            lds_get6(syk, I::NRY, I::ry(a - 1, b), sm);
-            lds_get6(syk, I::NRY, I::ry(a + 1, b), sp);
+            lds_get6(syk, I::NRY, X.ry(a - 1, b), sm);
+            lds_get6(syk, I::NRY, X.ry(a + 1, b), sp);
             trans_sigma<0>(P, sm, sg, sp, e1, tA);
-            lds_get6(sxk, I::NRX, I::rx(a, b - 1), sm);
-            lds_get6(sxk, I::NRX, I::rx(a, b + 1), sp);
+            lds_get6(sxk, I::NRX, X.rx(a, b - 1), sm);
+            lds_get6(sxk, I::NRX, X.rx(a, b + 1), sp);
             trans_sigma<1>(P, sm, sc, sp, e2, tB);
             add_ctu(Wp, Wn, tA, tB, ratio(8));
             if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
@@ -919,20 +994,22 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
         R VL[8], VR[8];
         double F[8];
         if (w < B1) {
-          if (!interior || w >= NBX) return;
-          const int a = w % (TX + 2) - 1, b = w / (TX + 2);
-          if (a < 0 || (a == TX && !ex && !FUSE)) return;
+          if (!interior || w >= X.nry()) return;
+          int a, b;
+          shape.row2(w, a, b);
+          --a;
+          if (a < 0 || (a == tx && !ex && !FUSE)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
-          if (P.aux && a < TX) {
+          if (P.aux && a < tx) {
             // face-averaged pressure (hy_getFaceFlux.F90:507-561 and the
             // y, z analogues)
             R pres = R(0.5) * psum;
-            pres = pres * R(0.5) + PY[I::rx(a, b)] * R(0.25);
-            if (Z) pres = div_const<6>(pres * R(4.0) + PZ[b * TX + a]);
-            if constexpr (FUSE) PA[b * TX + a] = pres;
+            pres = pres * R(0.5) + PY[X.rx(a, b)] * R(0.25);
+            if (Z) pres = div_const<6>(pres * R(4.0) + PZ[X.uy(a, b)]);
+            if constexpr (FUSE) PA[X.uy(a, b)] = pres;
             else st_at(as_global(T.pavg), cell_r(ox + a, oy + b, k) * 8u, double(pres));
           }
-          lds_get6(WX, I::NRY, I::ry(a - 1, b), VL);
+          lds_get6(WX, I::NRY, X.ry(a - 1, b), VL);
           right(VR);
           gammas(cb - sxb, cb, VL, VR);
           const unsigned fr = (unsigned)face_index(P, 0, ox + a, oy + b, k);
@@ -940,16 +1017,18 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             write_face_states<0>(P, fsb + fstate_dir_offset(P, 0), fr, VL, VR);
           } else {
             if (face_flux<0, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - sxb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 0); return; }
-            if constexpr (FUSE) put_flux(UX, I::NFX, I::ux(a, b), F);
+            if constexpr (FUSE) put_flux(UX, I::NFX, X.ux(a, b), F);
             else write_flux_b<0>(P, as_global(T.flux[0]), fr * 8u, F);
           }
         } else if (w < B2) {
           const int w2 = w - B1;
-          if (!interior || w2 >= NBY) return;
-          const int a = w2 % TX, b = w2 / TX - 1;
-          if (b < 0 || (b == TY && !ey && !FUSE)) return;
+          if (!interior || w2 >= X.nrx()) return;
+          int a, b;
+          shape.row(w2, a, b);
+          --b;
+          if (b < 0 || (b == ty && !ey && !FUSE)) return;
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
-          lds_get6(WY, I::NRX, I::rx(a, b - 1), VL);
+          lds_get6(WY, I::NRX, X.rx(a, b - 1), VL);
           right(VR);
           gammas(cb - syb, cb, VL, VR);
           const unsigned fr = (unsigned)face_index(P, 1, ox + a, oy + b, k);
@@ -957,13 +1036,14 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             write_face_states<1>(P, fsb + fstate_dir_offset(P, 1), fr, VL, VR);
           } else {
             if (face_flux<1, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - syb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 1); return; }
-            if constexpr (FUSE) put_flux(UY, I::NFY, I::uy(a, b), F);
+            if constexpr (FUSE) put_flux(UY, I::NFY, X.uy(a, b), F);
             else write_flux_b<1>(P, as_global(T.flux[1]), fr * 8u, F);
           }
         } else if (Z && w < B3) {
-          if (k < klo) return;
           const int w2 = w - B2;
-          const int a = w2 % TX, b = w2 / TX;
+          if (k < klo || (SH::kFree && w2 >= X.ncol())) return;
+          int a, b;
+          shape.row(w2, a, b);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
 #pragma unroll
           for (int q = 0; q < 6; ++q) VL[comp_slot(q)] = Wo[q];
@@ -1002,7 +1082,8 @@ __device__ __forceinline__ void march_block(const DevParams& P, const MarchLaunc
   const fx_tile T = L.tiles[t];
   for (int ty = 0; ty < L.tilesY; ++ty) {
     const int oy = P.lo[1] + ty * TY;
-    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseDirect>(P, L, T, t, P.lo[0], oy, nullptr, es, smem);
+    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseDirect>(P, L, T, t, P.lo[0], oy, nullptr, es, smem,
+                                                           FixedShape<TX, TY>{});
     if (ty == 0) continue;
     const TileView tv = tile_view(P, as_global(T.U));
     const gdouble* const upd = as_global(L.upd + (long)t * (kUpdComps * P.icells));
@@ -1042,8 +1123,33 @@ k_march(DevParams P, MarchLaunch L) {
   ExactStats es{0ULL, 0ULL};
   R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + t * fstate_tile_stride(P) : nullptr;
   __shared__ R smem[MarchLds<NDIM, TX, TY, FUSE>::total];
-  march_tile<NDIM, TX, TY, NT, RS, R, true, FUSE>(P, L, L.tiles[t], t, ox, oy, fsb, es, smem);
+  march_tile<NDIM, TX, TY, NT, RS, R, true, FUSE>(P, L, L.tiles[t], t, ox, oy, fsb, es, smem, FixedShape<TX, TY>{});
   flush_exact(L.status, es);
+}
+
+// One workgroup per column tile of a batch of blocks that no fixed tile
+// divides (extents not multiples of 8): tiles of L.tx x L.ty columns in the
+// 16x8 layout, with the update (kFuseScratch, or kFuseDirect for blocks of one
+// tile).  A row's length is then a value instead of a constant, which costs a
+// reciprocal multiplication per item; its loads, arithmetic and bits are the
+// fixed tile's.
+// Bound by FP64 issue and latency as k_march, and by what of the 128 columns a
+// tile leaves idle.  952 blocks of 12 x 10 x 14 679 us against 1464 by the three-
+// kernel path (face states through memory, transverse fluxes formed anew by
+// each state cell), 402 of 13 x 17 x 18 853 / 1399, 7407 of 6^3 1675 / 2033.
+template <int NDIM, int NT, int RS, typename R, int OCC, int FUSE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
+k_march_free(DevParams P, MarchLaunch L) {
+  const int tilesPerBlock = L.tilesX * L.tilesY;
+  const int t = blockIdx.x / tilesPerBlock;
+  const int tr = blockIdx.x - t * tilesPerBlock;
+  const int ox = P.lo[0] + (tr % L.tilesX) * L.tx;
+  const int oy = P.lo[1] + (tr / L.tilesX) * L.ty;
+  const FreeShape shape(min(L.tx, P.hi[0] + 1 - ox), min(L.ty, P.hi[1] + 1 - oy));
+  ExactStats es{0ULL, 0ULL};
+  __shared__ R smem[MarchLds<NDIM, 16, 8, FUSE>::total];
+  const fx_tile T = L.tiles[t];
+  march_tile<NDIM, 16, 8, NT, RS, R, true, FUSE>(P, L, T, t, ox, oy, nullptr, es, smem, shape);
 }
 
 // Tiles of several block classes in one persistent launch: workgroup b takes
@@ -1068,7 +1174,8 @@ k_march_multi(const DevParams* __restrict__ cls,
     const DevParams& P = cls[w.cls];
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
-    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
+    march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
+                                                         FixedShape<TX, TY>{});
   }
   flush_exact(L.status, es);
 }
@@ -1089,8 +1196,10 @@ k_march_mixw(const DevParams* __restrict__ cls, MarchLaunch L,
     const DevParams& P = cls[w.cls];
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
-    if (w.tx == 16) march_tile<NDIM, 16, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
-    else march_tile<NDIM, 8, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem);
+    if (w.tx == 16) march_tile<NDIM, 16, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
+                                                                         FixedShape<16, 8>{});
+    else march_tile<NDIM, 8, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
+                                                                 FixedShape<8, 8>{});
   }
   flush_exact(L.status, es);
 }

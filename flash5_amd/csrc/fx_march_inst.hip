@@ -48,6 +48,23 @@ void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
   launch_march_f<RS, R, kFuseNone>(P, M, TX, grid, H);
 }
 
+// Column tiles of free extents (M.tx x M.ty), FP64 with the update.
+template <int RS>
+void launch_march_free(const DevParams& P, const MarchLaunch& M, hipStream_t stream) {
+  const dim3 grid((unsigned)(M.nTiles * M.tilesX * M.tilesY));
+  if (P.ndim == 3 && M.fuse == kFuseDirect)
+    hipLaunchKernelGGL((k_march_free<3, 768, RS, double, 3, kFuseDirect>), grid, dim3(768), 0, stream, P, M);
+  else if (P.ndim == 3)
+    hipLaunchKernelGGL((k_march_free<3, 768, RS, double, 3, kFuseScratch>), grid, dim3(768), 0, stream, P, M);
+  else if (M.fuse == kFuseDirect)
+    hipLaunchKernelGGL((k_march_free<2, 384, RS, double, 3, kFuseDirect>), grid, dim3(384), 0, stream, P, M);
+  else
+    hipLaunchKernelGGL((k_march_free<2, 384, RS, double, 3, kFuseScratch>), grid, dim3(384), 0, stream, P, M);
+}
+#ifdef FX_MARCH_FREE
+template void launch_march_free<FX_MARCH_RS>(const DevParams&, const MarchLaunch&, hipStream_t);
+#endif
+
 // Persistent multi-class march: as many workgroups as stay resident (or
 // H.persist per CU), each taking every G-th column tile.
 template <int NDIM, int TX, int TY, int NT, int RS, typename R, int OCC = 0>

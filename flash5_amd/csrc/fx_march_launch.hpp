@@ -33,6 +33,12 @@ void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
 template <int RS, typename R>
 void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHost& H);
 
+// Column tiles of free extents (M.tx x M.ty) of a batch, in FP64 with the
+// update (M.fuse: kFuseScratch or kFuseDirect).
+template <int RS> void launch_march_free(const DevParams& P, const MarchLaunch& M, hipStream_t stream);
+extern template void launch_march_free<FX_HLLC>(const DevParams&, const MarchLaunch&, hipStream_t);
+extern template void launch_march_free<FX_HYBR>(const DevParams&, const MarchLaunch&, hipStream_t);
+
 #define FX_MARCH_DECLARE(RS_, R_)                                                        \
   extern template void launch_march_r<RS_, R_>(const DevParams&, const MarchLaunch&, int, \
                                                dim3, const MarchHost&);                  \
