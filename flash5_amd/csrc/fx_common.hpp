@@ -357,9 +357,18 @@ __device__ __forceinline__ void dt_pick_cell(DtPick& a, double dtl, double cfl, 
   if (prod > a.prod) a = DtPick{prod, dtl, idx};
 }
 
-// the workgroup's pick (kThreads lanes): the largest product, then the
-// lowest cell index; lane 0 returns the block's dt (1e300 when no cell had
-// a positive value, as the reference's huge(1.0))
+// of two lanes' picks the largest product, then the lowest cell index
+__device__ __forceinline__ void dt_pick_better(DtPick& a, const DtPick& b) {
+  if (b.prod > a.prod || (b.prod == a.prod && b.idx < a.idx)) a = b;
+}
+// a block's dt (1e300 when no cell had a positive value, as the reference's
+// huge(1.0))
+__device__ __forceinline__ double dt_of_pick(const DtPick& a, double cfl) {
+  return a.prod > 0. ? cfl / a.dtl : 1.e300;
+}
+
+// the workgroup's pick (kThreads lanes), as dt_pick_better; lane 0 returns
+// the block's dt
 __device__ __forceinline__ double dt_pick_block(DtPick a, double cfl) {
   __shared__ double sp[kThreads], sd[kThreads];
   __shared__ int si[kThreads];
@@ -376,7 +385,7 @@ __device__ __forceinline__ double dt_pick_block(DtPick a, double cfl) {
     }
     __syncthreads();
   }
-  return sp[0] > 0. ? cfl / sd[0] : 1.e300;
+  return dt_of_pick(DtPick{sp[0], sd[0], si[0]}, cfl);
 }
 
 }  // namespace fx

@@ -596,18 +596,13 @@ __global__ void __launch_bounds__(kThreads) k_update_multi(Launch L, ClassMap M,
   if (r < (int)P.icells) update_cell<false, false>(P, L, ch.x, r, inPlace);
 }
 
-// the CFL dt of each block (one workgroup per block), as dt_pick_block
-// describes; the CFL is cflDev[0] when cflDev is set (a lowered CFL kept on
-// the device), else cfl
-__global__ void __launch_bounds__(kThreads) k_dt(DevParams P, const double* __restrict__ Ubase,
-                                                 long stride, double idx, double idy, double idz,
-                                                 double cfl, const double* cflDev,
-                                                 double* __restrict__ dtBlock) {
-  const double c = cflDev ? cflDev[0] : cfl;
-  const double* U = Ubase + (long)blockIdx.x * stride;
+// one thread's part of a block's CFL dt: cells first, first + step, ...
+__device__ __forceinline__ DtPick dt_pick_cells(const DevParams& P, const double* U, double idx,
+                                                double idy, double idz, double c, int first,
+                                                int step) {
   const int nxi = P.nxb, nyi = P.ndim > 1 ? P.nyb : 1, n = (int)P.icells;
   DtPick best = dt_pick_none();
-  for (int r = threadIdx.x; r < n; r += blockDim.x) {
+  for (int r = first; r < n; r += step) {
     const int i = r % nxi + P.lo[0];
     const int j = (r / nxi) % nyi + P.lo[1];
     const int k = r / (nxi * nyi) + P.lo[2];
@@ -619,8 +614,91 @@ __global__ void __launch_bounds__(kThreads) k_dt(DevParams P, const double* __re
     if (P.ndim > 2) dtl = fmax(dtl, (fabs(U[P.voff[FX_VELZ] + cc] - 0.) + cs) * idz);
     dt_pick_cell(best, dtl, c, r);
   }
-  const double dt = dt_pick_block(best, c);
+  return best;
+}
+
+// the CFL dt of each block (one workgroup per block), as dt_pick_block
+// describes
+__global__ void __launch_bounds__(kThreads) k_dt(DevParams P, const double* __restrict__ Ubase,
+                                                 long stride, double idx, double idy, double idz,
+                                                 double cfl, double* __restrict__ dtBlock) {
+  const double dt = dt_pick_block(dt_pick_cells(P, Ubase + (long)blockIdx.x * stride, idx, idy,
+                                                idz, cfl, threadIdx.x, blockDim.x), cfl);
   if (threadIdx.x == 0) dtBlock[blockIdx.x] = dt;
+}
+
+// The grid's CFL dt beside a guard fill (k_fill_guards<true>).  The minimum
+// over the blocks is taken on the bits: dts are positive, so their bits order
+// as they do (a NaN lies above them all, as fmin leaves it out), and no
+// workgroup waits for another.  slot starts at kNoDt.
+// Blocks of up to kDtWaveCells cells take a wavefront each, which needs no
+// barrier and leaves one atomic for four blocks: with a workgroup and an
+// atomic on the one slot for each, an eager step of 4096 blocks of 16^2 took
+// 447 us instead of 423 (fill and dt as two launches: 427).
+constexpr double kNoDt = 1.e300;
+constexpr int kDtWaveCells = 1024;
+struct FillDt {
+  int nBlocks;            // blocks to take the dt of
+  unsigned wgs;           // workgroups for them, in front of the fill's
+  double idx, idy, idz, cfl;
+  const double* cflDev;   // a lowered CFL kept on the device, or null
+  double* slot;           // the minimum
+  double* next;           // set to kNoDt for a later call, or null
+};
+
+__device__ void grid_dt(const DevParams& P, const double* U, long stride, const FillDt& D,
+                        unsigned wg) {
+  const double c = D.cflDev ? D.cflDev[0] : D.cfl;
+  double dt = kNoDt;
+  if (P.icells <= kDtWaveCells) {
+    __shared__ double wdt[kThreads / 64];
+    const int wave = threadIdx.x / 64, b = (int)wg * (kThreads / 64) + wave;
+    if (b < D.nBlocks) {
+      DtPick a = dt_pick_cells(P, U + (long)b * stride, D.idx, D.idy, D.idz, c, threadIdx.x % 64, 64);
+      for (int s = 32; s > 0; s >>= 1)
+        dt_pick_better(a, DtPick{__shfl_xor(a.prod, s), __shfl_xor(a.dtl, s), __shfl_xor(a.idx, s)});
+      dt = dt_of_pick(a, c);
+    }
+    if (threadIdx.x % 64 == 0) wdt[wave] = dt;
+    __syncthreads();
+    for (int w = 0; w < kThreads / 64; ++w) dt = fmin(dt, wdt[w]);
+  } else {
+    dt = dt_pick_block(dt_pick_cells(P, U + (long)wg * stride, D.idx, D.idy, D.idz, c, threadIdx.x,
+                                     kThreads), c);
+  }
+  if (threadIdx.x == 0) {
+    atomicMin(reinterpret_cast<unsigned long long*>(D.slot),
+              (unsigned long long)__double_as_longlong(dt));
+    if (wg == 0 && D.next) *D.next = kNoDt;
+  }
+}
+
+// After the steps of a captured run: t += dt step by step, the last dt kept,
+// the slots ready for the next replay.
+__global__ void __launch_bounds__(64) k_close_steps(double* slots, int n, double* buf) {
+  __shared__ double s[64];
+  double t = buf[1], dt = buf[0];
+  for (int b = 0; b < n; b += 64) {
+    const int i = b + (int)threadIdx.x;
+    if (i < n) {
+      s[threadIdx.x] = slots[i];
+      slots[i] = kNoDt;
+    }
+    __syncthreads();
+    for (int j = 0; j < min(64, n - b); ++j) {
+      dt = s[j];
+      t = t + dt;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    buf[0] = dt;
+    buf[1] = t;
+  }
+}
+__global__ void k_open_slots(double* slots, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    slots[i] = kNoDt;
 }
 
 // dt = the minimum of the blocks' dts (Hydro_computeDt.F90:284-288), kept on
@@ -786,10 +864,24 @@ __host__ __device__ inline unsigned guard_cells(const DevParams& P) {
 
 // Blocks b0 .. b0 + nb - 1; blockIdx.y takes perGroup variables from
 // v0 + blockIdx.y * perGroup on, below v1.
+// With DT the first D.wgs workgroups take the blocks' CFL dt instead: it
+// reads interior cells, which the fill does not write, so neither waits for
+// the other, and the dt's chain of loads, divisions and roots runs beside the
+// copies: 60 captured steps of 256 blocks of 8^2 1654 -> 1245 us (four
+// launches a step become two), 216 blocks of 12 x 10 x 14 fill + dt 66 -> 56 us.
+template <bool DT>
 __global__ void __launch_bounds__(kThreads) k_fill_guards(DevParams P, double* __restrict__ U,
                                                           long b0, int nb, long stride,
                                                           const int* __restrict__ nbr, int v0,
-                                                          int v1, int perGroup) {
+                                                          int v1, int perGroup, FillDt D) {
+  unsigned wg = blockIdx.x;
+  if constexpr (DT) {
+    if (wg < D.wgs) {
+      if (blockIdx.y == 0) grid_dt(P, U, stride, D, wg);
+      return;
+    }
+    wg -= D.wgs;
+  }
   const unsigned nx = P.nx, np = (unsigned)P.nx * P.ny;
   const unsigned ixb = P.hi[0] - P.lo[0] + 1, iyb = P.hi[1] - P.lo[1] + 1;
   const unsigned izb = P.hi[2] - P.lo[2] + 1;
@@ -797,7 +889,7 @@ __global__ void __launch_bounds__(kThreads) k_fill_guards(DevParams P, double* _
   const unsigned G = guard_cells(P), total = G * (unsigned)nb;
   const int vb = v0 + (int)blockIdx.y * perGroup;
   const int nv = min(perGroup, v1 - vb);
-  const unsigned gid = blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned gid = wg * blockDim.x + threadIdx.x;
   if (gid >= total) return;
   const unsigned bl = gid / G;
   unsigned q = gid - bl * G;
@@ -915,6 +1007,11 @@ struct Lib {
   size_t seedBitsCap = 0;
   const double* dtDev = nullptr;       // set while capturing steps whose dt lives on the device
   double* dtBuf = nullptr;             // [dt, t, next dt's CFL, fallbacks so far] of graph runs
+  double* dtSlots = nullptr;           // the dt of each captured step of a uniform grid
+  size_t dtSlotsCap = 0;
+  double* fillDt = nullptr;            // fx_grid_fill_guards_dt: this call's minimum, the next one's
+  bool fillDtReady = false;
+  int fillDtTurn = 0;
   double runCfl = 0.;                  // the CFL argument of the graph-captured run
   hipStream_t capStream = nullptr;     // library stream for graph capture (default priority)
   std::vector<int> hnbr;               // neighbour table last uploaded (host copy)
@@ -1330,14 +1427,14 @@ NoAllocLayout noalloc_layout(const DevParams& P, long nBlocks) {
 
 // Inside a graph-captured run under shockLowerCFL or fallbackLowerCFL: the
 // device slot holding the next dt's CFL, or null (dt takes the CFL argument).
-const double* step_cfl_dev() { return cfl_varies(g.prm) && g.dtDev ? g.dtDev + 2 : nullptr; }
+const double* step_cfl_dev() { return cfl_varies(g.prm) && g.dtDev ? g.dtBuf + 2 : nullptr; }
 
 // Inside a graph-captured run under shockLowerCFL or fallbackLowerCFL, at
 // the end of a step: the next dt's CFL from this step's flags and fallbacks
 // (k_step_cfl).  Eager callers get the caps in fx_status.min_cell_cfl and
 // fallback_cfl instead.
 void launch_step_cfl() {
-  if (!cfl_varies(g.prm) || !g.dtDev) return;   // g.dtDev == g.dtBuf while capturing
+  if (!cfl_varies(g.prm) || !g.dtDev) return;   // (set while capturing)
   hipLaunchKernelGGL(k_step_cfl, dim3(1), dim3(1), 0, g.stream, g.status, g.runCfl,
                      shock_on(g.prm) ? 1 : 0,
                      g.prm.shockLowerCFL ? shock_cfl_max(g.prm.ndim) : 0.0,
@@ -1983,8 +2080,17 @@ int upload_neighbors(double* U, long nBlocks, long blockStride, const int* nbr, 
   return 0;
 }
 
-// onlyVar >= 0: that variable slot alone (the shock flags after detection)
-void launch_fill(double* U, long nBlocks, long blockStride, int onlyVar = -1) {
+FillDt fill_dt(long nBlocks, const double del[3], double cfl, const double* cflDev, double* slot,
+               double* next) {
+  const long per = g.dp.icells <= kDtWaveCells ? kThreads / 64 : 1;
+  return FillDt{(int)nBlocks, (unsigned)((nBlocks + per - 1) / per), 1. / del[0], 1. / del[1],
+                1. / del[2], cfl, cflDev, slot, next};
+}
+
+// onlyVar >= 0: that variable slot alone (the shock flags after detection);
+// D: the grid's dt beside the copies, or null
+void launch_fill(double* U, long nBlocks, long blockStride, int onlyVar = -1,
+                 const FillDt* D = nullptr) {
   const DevParams& P = g.dp;
   const int v0 = onlyVar >= 0 ? onlyVar : 0, v1 = onlyVar >= 0 ? onlyVar + 1 : P.nunk;
   const int groups = (v1 - v0 + kFillVars - 1) / kFillVars;
@@ -1993,9 +2099,14 @@ void launch_fill(double* U, long nBlocks, long blockStride, int onlyVar = -1) {
   const long most = (1L << 31) / G;   // the kernel's cell numbers have 32 bits
   for (long b0 = 0; b0 < nBlocks; b0 += most) {
     const long nb = std::min(most, nBlocks - b0);
-    const dim3 grid((unsigned)((nb * G + kThreads - 1) / kThreads), (unsigned)groups);
-    hipLaunchKernelGGL(k_fill_guards, grid, dim3(kThreads), 0, g.stream, P, U, b0, (int)nb,
-                       blockStride, g.dnbr, v0, v1, per);
+    const unsigned wgs = (unsigned)((nb * G + kThreads - 1) / kThreads);
+    if (D && b0 == 0)
+      hipLaunchKernelGGL(k_fill_guards<true>, dim3(wgs + D->wgs, (unsigned)groups),
+                         dim3(kThreads), 0, g.stream, P, U, b0, (int)nb, blockStride, g.dnbr, v0,
+                         v1, per, *D);
+    else
+      hipLaunchKernelGGL(k_fill_guards<false>, dim3(wgs, (unsigned)groups), dim3(kThreads), 0,
+                         g.stream, P, U, b0, (int)nb, blockStride, g.dnbr, v0, v1, per, FillDt{});
   }
 }
 
@@ -2287,7 +2398,7 @@ void fx_hydro_finalize(void) {
   if (g.hpin) (void)hipHostFree(g.hpin);
   void* bufs[] = {g.strongList, g.strongCount, g.dcellChunks, g.dwFace, g.dgateChunks, g.states, g.flux, g.pavg, g.upd, g.dtiles, g.dinplace, g.status, g.partial,
                   g.dregTiles, g.dfaces, g.mlpPacked, g.gradPart, g.seedPacked, g.seedY, g.fstates,
-                  g.dnbr, g.dtBuf, g.dcls, g.dtcls, g.dfaceStart,
+                  g.dnbr, g.dtBuf, g.dtSlots, g.fillDt, g.dcls, g.dtcls, g.dfaceStart,
                   g.ditems, g.dregCls, g.seedFlux, g.seedBits};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -2442,7 +2553,7 @@ int fx_hydro_compute_dt(const double* U, long nBlocks, long blockStride, const d
     g.partialCap = grid;
   }
   hipLaunchKernelGGL(k_dt, dim3(grid), dim3(kThreads), 0, g.stream, P, U, blockStride,
-                     1. / del[0], 1. / del[1], 1. / del[2], cfl, nullptr, g.partial);
+                     1. / del[0], 1. / del[1], 1. / del[2], cfl, g.partial);
   if (pinned(sizeof(double) * grid, nullptr)) return 4;
   if (hipMemcpyAsync(g.hpin, g.partial, sizeof(double) * grid, hipMemcpyDeviceToHost, g.stream) !=
       hipSuccess)
@@ -2567,6 +2678,41 @@ int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int
   return 0;
 }
 
+int fx_grid_fill_guards_dt(double* U, long nBlocks, long blockStride, const int* nbr,
+                           const double del[3], double cfl, double* dtOut, fx_status* st) {
+  if (st) memset(st, 0, sizeof *st);
+  if (!del || !dtOut || nBlocks > 0x7fffffffL) {
+    if (st) st->code = 3;
+    return 3;
+  }
+  const int rc = upload_neighbors(U, nBlocks, blockStride, nbr, st);
+  if (rc) return rc;
+  if (!(cfl > 0.) || !(del[0] > 0.) || !(del[1] > 0.) || !(del[2] > 0.)) {
+    // dts of any sign: one after the other
+    launch_fill(U, nBlocks, blockStride);
+    HIPCALL(hipGetLastError(), st);
+    return fx_hydro_compute_dt(U, nBlocks, blockStride, del, cfl, dtOut);
+  }
+  if (!g.fillDt) HIPCALL(hipMalloc((void**)&g.fillDt, 2 * sizeof(double)), st);
+  if (!g.fillDtReady) {
+    const double none[2] = {kNoDt, kNoDt};
+    HIPCALL(hipMemcpy(g.fillDt, none, sizeof none, hipMemcpyHostToDevice), st);
+    g.fillDtTurn = 0;
+  }
+  if (pinned(sizeof(double), st)) return 4;
+  g.fillDtReady = false;   // until the call is through
+  double* const slot = g.fillDt + g.fillDtTurn;
+  const FillDt D = fill_dt(nBlocks, del, cfl, nullptr, slot, g.fillDt + (1 - g.fillDtTurn));
+  launch_fill(U, nBlocks, blockStride, -1, &D);
+  HIPCALL(hipGetLastError(), st);
+  HIPCALL(hipMemcpyAsync(g.hpin, slot, sizeof(double), hipMemcpyDeviceToHost, g.stream), st);
+  HIPCALL(hipStreamSynchronize(g.stream), st);
+  *dtOut = *static_cast<const double*>(g.hpin);
+  g.fillDtTurn = 1 - g.fillDtTurn;
+  g.fillDtReady = true;
+  return 0;
+}
+
 int fx_grid_run_graph(double* U, long nBlocks, long blockStride, const int* nbr,
                       const double del[3], double cfl, int stepsPerGraph, int nReplays,
                       double* tOut, fx_status* st) {
@@ -2584,13 +2730,7 @@ int fx_grid_run_graph(double* U, long nBlocks, long blockStride, const int* nbr,
   if (!rc) rc = ensure_step_scratch((int)nBlocks, st);
   if (rc) return rc;
   const DevParams& P = g.dp;
-  const int dtGrid = (int)nBlocks;  // one workgroup per block
-  if (g.partialCap < dtGrid) {
-    if (g.partial) HIPCALL(hipFree(g.partial), st);
-    g.partial = nullptr;
-    HIPCALL(hipMalloc((void**)&g.partial, sizeof(double) * dtGrid), st);
-    g.partialCap = dtGrid;
-  }
+  if (grow(&g.dtSlots, &g.dtSlotsCap, (size_t)stepsPerGraph, st)) return 4;
   if (!g.dtBuf) HIPCALL(hipMalloc((void**)&g.dtBuf, 4 * sizeof(double)), st);
   if (!g.capStream) HIPCALL(hipStreamCreateWithFlags(&g.capStream, hipStreamNonBlocking), st);
   const hipStream_t saved = g.stream;
@@ -2611,13 +2751,12 @@ int fx_grid_run_graph(double* U, long nBlocks, long blockStride, const int* nbr,
   g.capturing = true;
   if (hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) err = 4;
   for (int s = 0; !err && s < stepsPerGraph; ++s) {
-    // dt from the interior cells (the guard fill does not change them), with
-    // the CFL the previous step's flags and fallbacks left
-    hipLaunchKernelGGL(k_dt, dim3(dtGrid), dim3(kThreads), 0, g.stream, P, U, blockStride,
-                       1. / del[0], 1. / del[1], 1. / del[2], cfl, step_cfl_dev(), g.partial);
-    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(kThreads), 0, g.stream, g.partial, dtGrid,
-                       g.dtBuf, g.dtBuf + 1);
-    launch_fill(U, nBlocks, blockStride);
+    // dt from the interior cells, beside the guard fill, with the CFL the
+    // previous step's flags and fallbacks left; a slot for each step, so that
+    // none is cleared between two steps
+    g.dtDev = g.dtSlots + s;
+    const FillDt D = fill_dt(nBlocks, del, cfl, step_cfl_dev(), g.dtSlots + s, nullptr);
+    launch_fill(U, nBlocks, blockStride, -1, &D);
     if (P.shokOff >= 0) {  // Hydro.F90:94-123: flag, then fill SHOK_VAR's guard cells
       hipLaunchKernelGGL(k_zero_shock_tiles, dim3(1), dim3(1), 0, g.stream, g.status);
       launch_shock_detect((int)nBlocks);
@@ -2626,12 +2765,18 @@ int fx_grid_run_graph(double* U, long nBlocks, long blockStride, const int* nbr,
     if (run_compute(nullptr, (int)nBlocks, 0.0, nullptr, nullptr, true)) err = 4;
     launch_step_cfl();
   }
+  if (!err)
+    hipLaunchKernelGGL(k_close_steps, dim3(1), dim3(64), 0, g.stream, g.dtSlots, stepsPerGraph,
+                       g.dtBuf);
   if (hipStreamEndCapture(g.stream, &graph) != hipSuccess) err = 4;
   g.capturing = false;
   if (!err && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) err = 4;
   // one status for the whole run: the replays keep the first error and sum
   // the counters of every step
   if (!err) hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
+  if (!err)
+    hipLaunchKernelGGL(k_open_slots, dim3(grid_for(stepsPerGraph)), dim3(kThreads), 0, g.stream,
+                       g.dtSlots, stepsPerGraph);
   for (int r = 0; !err && r < nReplays; ++r)
     if (hipGraphLaunch(exec, g.stream) != hipSuccess) err = 4;
   if (!err && hipStreamSynchronize(g.stream) != hipSuccess) err = 4;

@@ -195,6 +195,20 @@ class UniformGrid:
         if rc:
             raise FxError("fx_grid_fill_guards_var", st, rc)
 
+    def _fill_guards_dt(self, cfl: float) -> float:
+        """Guard cells of every variable and the CFL dt, in one launch."""
+        import ctypes as C
+        st = FxStatus()
+        dt = C.c_double(0.0)
+        self.hydro._reinit()
+        rc = self.lib.fx_grid_fill_guards_dt(
+            C.cast(C.c_void_p(self.U.data_ptr()), C.POINTER(C.c_double)), self.U.shape[0],
+            self.U[0].numel(), self.nbr.ctypes.data_as(C.POINTER(C.c_int)),
+            (C.c_double * 3)(*self.deltas), cfl, C.byref(dt), C.byref(st))
+        if rc:
+            raise FxError("fx_grid_fill_guards_dt", st, rc)
+        return dt.value
+
     def step(self, dt_max: float = math.inf) -> float:
         """Guard fill, CFL dt (capped by dt_max), unsplit update in place.
         With shock detection on: fill, flag, fill again, as Hydro.F90:94-123
@@ -203,12 +217,11 @@ class UniformGrid:
         hy_fallbackLowerCFL the dt takes the CFL that the previous step's
         flags and fallbacks left (step_cfl)."""
         cfl = self._cfl_next
-        self.fill_guards(wait=False)
+        dt = min(self._fill_guards_dt(cfl), dt_max)
         shock_cap = 0.0
         if self.detect:
             shock_cap = self.hydro.shock_detect_batch(self.U, self.deltas).min_cell_cfl
             self.fill_guards(self.params.shokVar, wait=False)
-        dt = min(self.hydro.compute_dt(self.U, self.deltas, cfl), dt_max)
         st = self.hydro.advance_batch(self.U, dt, self.deltas)
         self._cfl_next = step_cfl(self.cfl, cfl, self.detect, shock_cap, st.fallback_cfl)
         self.t += dt

@@ -123,6 +123,8 @@ EXPORTS = {
     "fx_hydro_face_states": ([_DP, C.c_long, C.POINTER(C.c_long)], C.c_int),
     "fx_grid_fill_guards_var": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_int, C.c_int,
                                  C.POINTER(FxStatus)], C.c_int),
+    "fx_grid_fill_guards_dt": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_double * 3,
+                                C.c_double, _DP, C.POINTER(FxStatus)], C.c_int),
     "fx_grid_fill_guards": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.POINTER(FxStatus)],
                             C.c_int),
     "fx_grid_run_graph": ([_DP, C.c_long, C.c_long, C.POINTER(C.c_int), C.c_double * 3, C.c_double,

@@ -294,6 +294,11 @@ int fx_grid_fill_guards(double* U, long nBlocks, long blockStride, const int* nb
  * goes there too. */
 int fx_grid_fill_guards_var(double* U, long nBlocks, long blockStride, const int* nbr, int var,
                             int wait, fx_status* st);
+/* The guard cells of every variable and, in the same launch, the CFL dt of
+ * fx_hydro_compute_dt (it reads interior cells only); returns when both are
+ * done. */
+int fx_grid_fill_guards_dt(double* U, long nBlocks, long blockStride, const int* nbr,
+                           const double del[3], double cfl, double* dtOut, fx_status* st);
 
 /* Whole steps of a uniform grid captured in a HIP graph: each captured step
  * fills the guard cells (as fx_grid_fill_guards), computes the CFL dt on
