@@ -1663,8 +1663,8 @@ template <typename R>
 void launch_face_solve(const DevParams& P, const FaceLaunch& F, long faces, bool multi,
                        bool withUpdate, double dt) {
   const dim3 gf(grid_for(faces));
-  if (P.learned) {  // the gate lists the strong faces for the seed kernel
-    float* y = withUpdate ? nullptr : g.seedY;
+  if (P.learned && !withUpdate) {  // the gate lists the strong faces for the seed kernel
+    float* y = g.seedY;
     hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, g.stream, g.strongCount);
     if (multi)
       hipLaunchKernelGGL((k_face_gate<true, R>), dim3((unsigned)g.nGateChunks), dim3(kThreads), 0,
@@ -1719,6 +1719,15 @@ int launch_flux_stages(int nTiles, double dt, int TX, int TY, bool solveUpdate =
     // exact solver: the march stores face states, a separate stage solves
     // (with the learned seed, after the gate and the seed kernel)
     M.fstates = g.fstates;
+    if (P.learned && solveUpdate) {
+      // one tile shape, no seed slot per face: the march has each face's states
+      // at hand and lists the strong ones itself
+      M.gate = make_seed_gate(g.seedGate);
+      M.strongList = g.strongList;
+      M.strongCount = g.strongCount;
+      M.strongCap = (unsigned)g.hfaceStart[nTiles];
+      hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, g.stream, g.strongCount);
+    }
     if (g.multi) launch_march_multi<RS_STATES>(P.ndim, P.precision, TX, M);
     else launch_march<RS_STATES>(P, M, TX, grid);
     if (record(1)) return 4;

@@ -165,6 +165,12 @@ struct MarchLaunch {
   int fuse;            // where the update runs (kFuse*)
   double* upd;         // fused update: updated states, [tile][component][interior cell]
   int tx, ty;          // free tiles: columns of a tile (the last along an axis may have fewer)
+  // RS_STATES with the learned seed (one tile shape): faces at or above the
+  // gate join the list; null: none do
+  SeedGate gate;
+  unsigned* strongList;
+  unsigned* strongCount;
+  unsigned strongCap;
 };
 // components of a cell's fused-update scratch: density, velocities, eint (the
 // sixth only in the FP32 march, on the way)
@@ -198,6 +204,29 @@ __device__ __forceinline__ void write_face_states(const DevParams& P, R* base, l
     base[q * nf + r] = VL[comp_slot(q)];
     base[(6 + q) * nf + r] = VR[comp_slot(q)];
   }
+}
+
+// The learned seed's gate (seed_gate_pass, in FP64 from the stored values) on a
+// face whose states are at hand: a strong one joins the list, one atomic per
+// wavefront, ranks by ballot over the lanes that are here.
+template <int D, typename R>
+__device__ __forceinline__ void list_strong_face(const DevParams& P, const MarchLaunch& L, int t,
+                                                 unsigned r, const R VL[8], const R VR[8]) {
+  const double rl = VL[P_DENS], ul = VL[P_VELX + D], pl = VL[P_PRES];
+  const double rr = VR[P_DENS], ur = VR[P_VELX + D], pr = VR[P_PRES];
+  const bool strong = rl > 0. && rr > 0. && pl > 0. && pr > 0. &&
+                      seed_gate_pass(L.gate, P.gamma, rl, ul, pl, rr, ur, pr);
+  const unsigned long long mask = __ballot(strong);
+  if (!mask) return;
+  const int lane = (int)(threadIdx.x & 63), leader = __builtin_ctzll(mask);
+  unsigned base = 0;
+  if (lane == leader) base = atomicAdd(L.strongCount, (unsigned)__popcll(mask));
+  base = __shfl(base, leader);
+  const unsigned slot = base + (unsigned)__popcll(mask & ((1ULL << lane) - 1ULL));
+  if (!strong || slot >= L.strongCap) return;
+  const long before = D == 0 ? 0 : (D == 1 ? P.nface[0] : P.nface[0] + P.nface[1]);
+  const long perTile = P.nface[0] + P.nface[1] + P.nface[2];
+  L.strongList[slot] = (unsigned)(t * perTile + before + r);
 }
 
 template <typename R>
@@ -1015,6 +1044,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const unsigned fr = (unsigned)face_index(P, 0, ox + a, oy + b, k);
           if constexpr (is_states(RS)) {
             write_face_states<0>(P, fsb + fstate_dir_offset(P, 0), fr, VL, VR);
+            if (L.strongList) list_strong_face<0>(P, L, t, fr, VL, VR);
           } else {
             if (face_flux<0, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - sxb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 0); return; }
             if constexpr (FUSE) put_flux(UX, I::NFX, X.ux(a, b), F);
@@ -1034,6 +1064,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const unsigned fr = (unsigned)face_index(P, 1, ox + a, oy + b, k);
           if constexpr (is_states(RS)) {
             write_face_states<1>(P, fsb + fstate_dir_offset(P, 1), fr, VL, VR);
+            if (L.strongList) list_strong_face<1>(P, L, t, fr, VL, VR);
           } else {
             if (face_flux<1, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - syb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 1); return; }
             if constexpr (FUSE) put_flux(UY, I::NFY, X.uy(a, b), F);
@@ -1052,6 +1083,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           const unsigned fr = (unsigned)face_index(P, 2, ox + a, oy + b, k);
           if constexpr (is_states(RS)) {
             write_face_states<2>(P, fsb + fstate_dir_offset(P, 2), fr, VL, VR);
+            if (L.strongList) list_strong_face<2>(P, L, t, fr, VL, VR);
           } else {
             if (face_flux<2, RS>(P, VL, VR, tv_use_hll<RS>(P, tv, cb - szb, cb), F, es)) { report_error(st, 2, t, ox + a, oy + b, k, 2); return; }
             if constexpr (FUSE) put_flux(UZ, NCOL, w2, F);
