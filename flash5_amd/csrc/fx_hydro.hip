@@ -1878,8 +1878,7 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     const bool solveUpdate = tilesUploaded && !tiles && !inPlace && !g.multi && !g.solveUpdOff &&
                              P.riemann == FX_EXACT && P.ndim == 3 &&
                              P.nxb * P.nyb <= kSolveMaxCols &&
-                             2 * (P.nxb + 1) * P.nyb + P.nxb * P.nyb <= kSolveMaxFaces &&
-                             P.nxb + 1 <= 17 && P.nyb + 1 <= 17 &&
+                             P.nxb <= kSolveMaxSide && P.nyb <= kSolveMaxSide &&
                              (!P.learned || seed_bit_words(P) <= kSolveMaxBitWords);
     if (g.multi && build_march_items(nTiles, TX, st)) return 4;
     if (ensure_step_scratch(nTiles, st)) return 4;
