@@ -1250,6 +1250,34 @@ bool free_shape(const DevParams& P, int* tx, int* ty) {
   return best < 1 << 30;
 }
 
+// How many segments along z the column tiles of a launch are cut into, and
+// their planes.  A segment marches its planes and about three more, so one
+// that is not resident at once costs more than it gives: cuts are taken while
+// they shorten the longest run of planes on a compute unit by a tenth.
+// 16^3 blocks, FP64 HLLC steps: one of them 190 -> 52 us, 24 190 -> 88, 64 190 ->
+// 131, 160 (320 column tiles) 370 -> 316; from 256 on, whole columns.
+struct ZSplit {
+  int n, per;
+  long planes;   // the longest run
+};
+ZSplit z_split(const DevParams& P, long columnTiles, long slots) {
+  const int nz = P.ndim == 3 ? P.nzb : 1;
+  ZSplit best{1, nz, (columnTiles + slots - 1) / slots * (nz + 3)};
+  if (P.ndim < 3) return best;
+  const long whole = best.planes;
+  for (int n = 2; n <= nz; ++n) {
+    const int per = (nz + n - 1) / n, m = (nz + per - 1) / per;
+    const long planes = (columnTiles * m + slots - 1) / slots * (per + 3);
+    if (planes < best.planes && planes * 10 <= whole * 9) best = ZSplit{m, per, planes};
+  }
+  return best;
+}
+
+// march workgroups resident at a time: the FP64 16x8 tile takes a CU's LDS
+long march_slots(const DevParams& P, int TX) {
+  return (long)g.numCU * (TX == 16 && P.precision != FX_PREC_MIXED ? 1 : 2);
+}
+
 // Whether n blocks step faster by free column tiles than by the three-kernel
 // path.  In 3-D a column tile takes a compute unit for its planes and three
 // more, about 4 us each and 6 more with all 128 columns in use; the three
@@ -1263,9 +1291,8 @@ bool free_shape(const DevParams& P, int* tx, int* ty) {
 bool free_pays(const DevParams& P, long n, int tx, int ty) {
   if (P.ndim == 2) return true;
   const long tiles = (long)((P.nxb + tx - 1) / tx) * ((P.nyb + ty - 1) / ty);
-  const long rounds = (n * tiles + g.numCU - 1) / g.numCU;
   const double cols = (double)(P.nxb * P.nyb) / (double)(tiles * 128);
-  return (double)(rounds * (P.nzb + 3)) * (4.0 + 6.0 * cols) <
+  return (double)z_split(P, n * tiles, g.numCU).planes * (4.0 + 6.0 * cols) <
          40.0 + 0.27e-3 * (double)P.scellsPerTile * (double)n;
 }
 
@@ -1293,9 +1320,9 @@ int batch_fuse_mode(const DevParams& P, int TX, int TY, long n) {
   if (!batch_fused(P, n)) return kFuseNone;
   const long tiles = P.nyb / TY;
   if (P.nxb != TX || (P.ndim == 3 && P.steep) || (P.ndim == 2 && tiles > 1)) return kFuseScratch;
-  // resident workgroups: the FP64 16x8 tile takes a CU's LDS
-  const long slots = (long)g.numCU * (TX == 16 && P.precision != FX_PREC_MIXED ? 1 : 2);
-  const long direct = (n + slots - 1) / slots * tiles, scratch = (n * tiles + slots - 1) / slots;
+  const long slots = march_slots(P, TX);
+  const long direct = (n + slots - 1) / slots * tiles * ((P.ndim == 3 ? P.nzb : 1) + 3);
+  const long scratch = z_split(P, n * tiles, slots).planes;
   return direct * 8 <= scratch * 9 ? kFuseDirect : kFuseScratch;
 }
 
@@ -1714,7 +1741,12 @@ int launch_flux_stages(int nTiles, double dt, int TX, int TY, bool solveUpdate =
   MarchLaunch M{g.dtiles, nTiles, g.multi ? 0 : P.nxb / TX,
                 g.multi ? 0 : (P.ndim > 1 ? P.nyb : 1) / TY, g.status, dt, nullptr, g.dtDev,
                 fuse, fuse ? g.upd : nullptr};
-  const dim3 grid((unsigned)(g.multi ? 1 : nTiles * M.tilesX * M.tilesY));
+  if (!g.multi && fuse != kFuseDirect) {
+    const ZSplit z = z_split(P, (long)nTiles * M.tilesX * M.tilesY, march_slots(P, TX));
+    M.tilesZ = z.n;
+    M.nzSeg = z.per;
+  }
+  const dim3 grid((unsigned)(g.multi ? 1 : nTiles * M.tilesX * M.tilesY * M.tilesZ));
   if (P.riemann == FX_EXACT) {
     // exact solver: the march stores face states, a separate stage solves
     // (with the learned seed, after the gate and the seed kernel)
@@ -1769,7 +1801,10 @@ int launch_free(const DevParams& P, int nTiles, double dt) {
   M.tilesY = (P.nyb + M.ty - 1) / M.ty;
   // a block of one tile is updated in place, unless the steepening still
   // reads planes that the update has written by then
-  if (M.tilesX * M.tilesY == 1 && !(P.ndim == 3 && P.steep)) M.fuse = kFuseDirect;
+  const ZSplit z = z_split(P, (long)nTiles * M.tilesX * M.tilesY, g.numCU);
+  if (M.tilesX * M.tilesY == 1 && z.n == 1 && !(P.ndim == 3 && P.steep)) M.fuse = kFuseDirect;
+  M.tilesZ = z.n;
+  M.nzSeg = z.per;
   if (P.riemann == FX_HLLC) launch_march_free<FX_HLLC>(P, M, g.stream);
   else launch_march_free<FX_HYBR>(P, M, g.stream);
   if (record(1) || record(2)) return 4;
@@ -2500,7 +2535,12 @@ int fx_hydro_advance_batch_noalloc(double* U, long nBlocks, long blockStride,
   double* const upd = reinterpret_cast<double*>(s + Lay.flux);
   MarchLaunch M{tiles, (int)nBlocks, P.nxb / TX, (P.ndim > 1 ? P.nyb : 1) / TY, status, dt,
                 nullptr, nullptr, fuse, upd};
-  const dim3 grid((unsigned)(nBlocks * M.tilesX * M.tilesY));
+  if (fuse != kFuseDirect) {
+    const ZSplit z = z_split(P, nBlocks * M.tilesX * M.tilesY, march_slots(P, TX));
+    M.tilesZ = z.n;
+    M.nzSeg = z.per;
+  }
+  const dim3 grid((unsigned)(nBlocks * M.tilesX * M.tilesY * M.tilesZ));
   if (P.riemann == FX_HLLC) launch_march<FX_HLLC>(P, M, TX, grid);
   else launch_march<FX_HYBR>(P, M, TX, grid);
   Launch L{tiles, (int)nBlocks, nullptr, status, dt, nullptr};

@@ -165,6 +165,8 @@ struct MarchLaunch {
   int fuse;            // where the update runs (kFuse*)
   double* upd;         // fused update: updated states, [tile][component][interior cell]
   int tx, ty;          // free tiles: columns of a tile (the last along an axis may have fewer)
+  int tilesZ = 1;      // segments of a column tile along z, of nzSeg planes (the last may have
+  int nzSeg = 1 << 20; // fewer): k_march and k_march_free, not kFuseDirect
   // RS_STATES with the learned seed (one tile shape): faces at or above the
   // gate join the list; null: none do
   SeedGate gate;
@@ -449,7 +451,7 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One column tile (TX x TY columns at ox, oy, all planes) of tile t.  Every
+// One column tile (TX x TY columns at ox, oy, planes klo to khi) of tile t.  Every
 // thread of the workgroup calls it with the same arguments; it ends on a
 // barrier, so a workgroup may call it again for another column tile.  fsb:
 // tile t's face-state scratch (RS_STATES).
@@ -477,7 +479,8 @@ __device__ __forceinline__ void lds_barrier() {
 template <int NDIM, int TX, int TY, int NT, int RS, typename R, bool OPAQUE, int FUSE, typename SH>
 __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch& L,
                                            const fx_tile& T, int t, int ox, int oy, R* fsb,
-                                           ExactStats& es, R* smem, const SH shape) {
+                                           ExactStats& es, R* smem, const SH shape, int klo,
+                                           int khi) {
   using I = TileIdx<TX, TY>;
   using M = MarchLds<NDIM, TX, TY, FUSE>;
   constexpr int NR = NDIM == 3 ? 3 : 1;        // ring depth
@@ -518,7 +521,6 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
   if constexpr (FUSE == kFuseDirect) asm volatile("" : "+v"(dt));
   const double dx = T.del[0], dy = T.del[1], dz = T.del[2];
   const unsigned sxb = 8u, syb = (unsigned)P.nx * 8u, szb = (unsigned)(P.nx * P.ny) * 8u;
-  const int klo = P.lo[2], khi = P.hi[2];
   DevStatus* st = L.status;
   bool bad = false;  // eigen failure seen by this thread
   // The step's ratios of dt and the cell widths, and the widths, uniform over
@@ -975,7 +977,8 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           sub_sigma(Wp, Wn, sc, ratio(3));
           lds_get6(syk, I::NRY, X.ry(a, b), sg);
           sub_sigma(Wp, Wn, sg, ratio(4));
-          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
+          const bool own = (k >= klo || klo == P.lo[2]) && (k <= khi || khi == P.hi[2]);
+          if (negative(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
           if (P.ctu3d) {
             // sigma_y over i with x's eigen system, sigma_x over j with y's
             e1 = e2 = e0;
@@ -988,7 +991,7 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
             lds_get6(sxk, I::NRX, X.rx(a, b + 1), sp);
             trans_sigma<1>(P, sm, sc, sp, e2, tB);
             add_ctu(Wp, Wn, tA, tB, ratio(8));
-            if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, true);
+            if (nonpositive(Wp, Wn)) fallback_first_order(Vc, Wp, Wn, st, own);
           }
           // the column's Wp stays with its thread: last plane's out, this one's in
 #pragma unroll
@@ -1072,7 +1075,9 @@ __device__ __forceinline__ void march_tile(const DevParams& P, const MarchLaunch
           }
         } else if (Z && w < B3) {
           const int w2 = w - B2;
-          if (k < klo || (SH::kFree && w2 >= X.ncol())) return;
+          // the face above a segment is the next one's, unless the update needs it here
+          if (k < klo || (!FUSE && k > khi && khi < P.hi[2])) return;
+          if (SH::kFree && w2 >= X.ncol()) return;
           int a, b;
           shape.row(w2, a, b);
           const unsigned cb = cell_b(P, ox + a, oy + b, k);
@@ -1115,7 +1120,7 @@ __device__ __forceinline__ void march_block(const DevParams& P, const MarchLaunc
   for (int ty = 0; ty < L.tilesY; ++ty) {
     const int oy = P.lo[1] + ty * TY;
     march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseDirect>(P, L, T, t, P.lo[0], oy, nullptr, es, smem,
-                                                           FixedShape<TX, TY>{});
+                                                           FixedShape<TX, TY>{}, P.lo[2], P.hi[2]);
     if (ty == 0) continue;
     const TileView tv = tile_view(P, as_global(T.U));
     const gdouble* const upd = as_global(L.upd + (long)t * (kUpdComps * P.icells));
@@ -1132,7 +1137,21 @@ __device__ __forceinline__ void march_block(const DevParams& P, const MarchLaunc
   }
 }
 
-// One workgroup per column tile of a batch of equal-shape tiles.  OCC > 0
+// the tile, column tile and first plane of a workgroup
+struct MarchPlace {
+  int t, tx, ty, klo;
+};
+__device__ __forceinline__ MarchPlace march_place(const DevParams& P, const MarchLaunch& L) {
+  const int cols = L.tilesX * L.tilesY, per = cols * L.tilesZ;
+  const int t = blockIdx.x / per, tr = blockIdx.x - t * per;
+  const int tz = tr / cols, tc = tr - tz * cols;
+  return MarchPlace{t, tc % L.tilesX, tc / L.tilesX, P.lo[2] + (L.tilesZ > 1 ? tz * L.nzSeg : 0)};
+}
+
+// One workgroup per column tile of a batch of equal-shape tiles, or per
+// segment of one along z where column tiles alone leave the chip idle (a
+// segment forms the states and sigmas of the planes next to it anew: three
+// planes' work).  OCC > 0
 // asks the compiler for OCC waves per SIMD (fewer registers, maybe spills);
 // the autotuner decides whether that pays.  The FP64 16x8 tile runs 768
 // threads: its LDS allows one workgroup per CU, stage A has 12 wavefronts of
@@ -1147,15 +1166,13 @@ k_march(DevParams P, MarchLaunch L) {
     march_block<NDIM, TX, TY, NT, RS, R>(P, L, (int)blockIdx.x, es, smem);
     return;
   }
-  const int tilesPerBlock = L.tilesX * L.tilesY;
-  const int t = blockIdx.x / tilesPerBlock;
-  const int tr = blockIdx.x - t * tilesPerBlock;
-  const int ox = P.lo[0] + (tr % L.tilesX) * TX;
-  const int oy = P.lo[1] + (tr / L.tilesX) * TY;
+  const MarchPlace w = march_place(P, L);
+  const int t = w.t, ox = P.lo[0] + w.tx * TX, oy = P.lo[1] + w.ty * TY, klo = w.klo;
   ExactStats es{0ULL, 0ULL};
   R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + t * fstate_tile_stride(P) : nullptr;
   __shared__ R smem[MarchLds<NDIM, TX, TY, FUSE>::total];
-  march_tile<NDIM, TX, TY, NT, RS, R, true, FUSE>(P, L, L.tiles[t], t, ox, oy, fsb, es, smem, FixedShape<TX, TY>{});
+  march_tile<NDIM, TX, TY, NT, RS, R, true, FUSE>(P, L, L.tiles[t], t, ox, oy, fsb, es, smem, FixedShape<TX, TY>{},
+                                                  klo, min(klo + L.nzSeg - 1, P.hi[2]));
   flush_exact(L.status, es);
 }
 
@@ -1172,16 +1189,14 @@ k_march(DevParams P, MarchLaunch L) {
 template <int NDIM, int NT, int RS, typename R, int OCC, int FUSE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 k_march_free(DevParams P, MarchLaunch L) {
-  const int tilesPerBlock = L.tilesX * L.tilesY;
-  const int t = blockIdx.x / tilesPerBlock;
-  const int tr = blockIdx.x - t * tilesPerBlock;
-  const int ox = P.lo[0] + (tr % L.tilesX) * L.tx;
-  const int oy = P.lo[1] + (tr / L.tilesX) * L.ty;
+  const MarchPlace w = march_place(P, L);
+  const int t = w.t, ox = P.lo[0] + w.tx * L.tx, oy = P.lo[1] + w.ty * L.ty, klo = w.klo;
   const FreeShape shape(min(L.tx, P.hi[0] + 1 - ox), min(L.ty, P.hi[1] + 1 - oy));
   ExactStats es{0ULL, 0ULL};
   __shared__ R smem[MarchLds<NDIM, 16, 8, FUSE>::total];
   const fx_tile T = L.tiles[t];
-  march_tile<NDIM, 16, 8, NT, RS, R, true, FUSE>(P, L, T, t, ox, oy, nullptr, es, smem, shape);
+  march_tile<NDIM, 16, 8, NT, RS, R, true, FUSE>(P, L, T, t, ox, oy, nullptr, es, smem, shape, klo,
+                                                  min(klo + L.nzSeg - 1, P.hi[2]));
 }
 
 // Tiles of several block classes in one persistent launch: workgroup b takes
@@ -1207,7 +1222,7 @@ k_march_multi(const DevParams* __restrict__ cls,
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
     march_tile<NDIM, TX, TY, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
-                                                         FixedShape<TX, TY>{});
+                                                         FixedShape<TX, TY>{}, P.lo[2], P.hi[2]);
   }
   flush_exact(L.status, es);
 }
@@ -1229,9 +1244,9 @@ k_march_mixw(const DevParams* __restrict__ cls, MarchLaunch L,
     const long faceBase = is_states(RS) ? faceStart[w.t] : 0;
     R* fsb = is_states(RS) ? static_cast<R*>(L.fstates) + kFaceComps * faceBase : nullptr;
     if (w.tx == 16) march_tile<NDIM, 16, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
-                                                                         FixedShape<16, 8>{});
+                                                                         FixedShape<16, 8>{}, P.lo[2], P.hi[2]);
     else march_tile<NDIM, 8, 8, NT, RS, R, true, kFuseNone>(P, L, L.tiles[w.t], w.t, w.ox, w.oy, fsb, es, smem,
-                                                                 FixedShape<8, 8>{});
+                                                                 FixedShape<8, 8>{}, P.lo[2], P.hi[2]);
   }
   flush_exact(L.status, es);
 }

@@ -51,7 +51,7 @@ void launch_march_r(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
 // Column tiles of free extents (M.tx x M.ty), FP64 with the update.
 template <int RS>
 void launch_march_free(const DevParams& P, const MarchLaunch& M, hipStream_t stream) {
-  const dim3 grid((unsigned)(M.nTiles * M.tilesX * M.tilesY));
+  const dim3 grid((unsigned)(M.nTiles * M.tilesX * M.tilesY * M.tilesZ));
   if (P.ndim == 3 && M.fuse == kFuseDirect)
     hipLaunchKernelGGL((k_march_free<3, 768, RS, double, 3, kFuseDirect>), grid, dim3(768), 0, stream, P, M);
   else if (P.ndim == 3)
