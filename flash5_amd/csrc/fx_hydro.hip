@@ -1273,6 +1273,20 @@ ZSplit z_split(const DevParams& P, long columnTiles, long slots) {
   return best;
 }
 
+// Whether n blocks of the exact solver's batch step take one workgroup each
+// for solve and update.  That takes the time of a block's rounds one after the
+// other however few the blocks; the face solve and the update as kernels of
+// their own take a time in proportion to the faces, up to about 30000 of them
+// (16000 in FP32) in the time of a round.  One / separate, the whole step:
+// 16^3 FP64 1 block 383 / 88 us, 100 556 / 509, 128 576 / 602, 512 1341 / 1783;
+// mixed 64 308 / 288, 100 350 / 420; 8^3 FP64 128 184 / 169, 256 223 / 246;
+// mixed 64 101 / 97, 128 113 / 126; 16 x 16 x 32 FP64 128 1190 / 1143.
+bool solve_update_pays(const DevParams& P, long n) {
+  const long faces = n * (P.nface[0] + P.nface[1] + P.nface[2]);
+  return faces > (P.precision == FX_PREC_MIXED ? 16000L : 30000L) *
+                     solve_rounds(P.nxb, P.nyb, P.nzb);
+}
+
 // march workgroups resident at a time: the FP64 16x8 tile takes a CU's LDS
 long march_slots(const DevParams& P, int TX) {
   return (long)g.numCU * (TX == 16 && P.precision != FX_PREC_MIXED ? 1 : 2);
@@ -1910,10 +1924,12 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
   if (march) {
     // batch steps with the exact solver: its face stage and the update run
     // as one kernel (k_solve_update) for 3-D blocks up to 16 x 16 across
+    // (where the batch is large enough for that)
     const bool solveUpdate = tilesUploaded && !tiles && !inPlace && !g.multi && !g.solveUpdOff &&
                              P.riemann == FX_EXACT && P.ndim == 3 &&
                              P.nxb * P.nyb <= kSolveMaxCols &&
                              P.nxb <= kSolveMaxSide && P.nyb <= kSolveMaxSide &&
+                             solve_update_pays(P, nTiles) &&
                              (!P.learned || seed_bit_words(P) <= kSolveMaxBitWords);
     if (g.multi && build_march_items(nTiles, TX, st)) return 4;
     if (ensure_step_scratch(nTiles, st)) return 4;

@@ -497,6 +497,14 @@ __host__ __device__ inline int solve_ahead(int nx, int ny, int nz) {
   return together < nz * ((low + high + T - 1) / T) ? n : 1;
 }
 
+// rounds of a block, the faces above the top plane among them
+inline long solve_rounds(int nx, int ny, int nz) {
+  const int T = kSolveThreads, n = solve_ahead(nx, ny, nz), low = 3 * nx * ny;
+  const long top = (nx * ny + T - 1) / T;
+  if (n == 1) return (long)nz * ((low + nx + ny + T - 1) / T) + top;
+  return (long)nz * ((low + T - 1) / T) + (nz + n - 1) / n + top;
+}
+
 template <bool SEEDED, typename R>
 __global__ void __launch_bounds__(kSolveThreads) __attribute__((amdgpu_waves_per_eu(2)))
 k_solve_update(DevParams P, FaceLaunch F, double dt0, const double* dtp, const R* over,

@@ -14,14 +14,17 @@ from tests.test_gpu_fused_update import _batch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("prec,seeded", [(PREC_FP64, False), (PREC_MIXED, False),
-                                         (PREC_MIXED, True)], ids=["fp64", "mixed", "learned"])
+@pytest.mark.parametrize("nblocks", [4, 260])        # apart as well, and in one kernel
+@pytest.mark.parametrize("prec,gate", [(PREC_FP64, None), (PREC_MIXED, None), (PREC_MIXED, 0.05),
+                                       (PREC_MIXED, 0.0), (PREC_FP64, 0.05)],
+                         ids=["fp64", "mixed", "learned", "learned_all", "fp64_learned"])
 @pytest.mark.parametrize("shape", [(16, 16, 2), (16, 16, 7), (16, 16, 8), (16, 16, 9),
                                    (16, 16, 17), (8, 16, 24), (16, 8, 5), (8, 8, 11)])
-def test_solve_and_update_at_every_height(shape, prec, seeded):
+def test_solve_and_update_at_every_height(shape, prec, gate, nblocks):
+    seeded = gate is not None
     hp = HydroParams(ndim=3, nxb=shape[0], nyb=shape[1], nzb=shape[2], gamma=1.4,
                      RiemannSolver="exact", precision=prec, learnedSeed=seeded)
-    U0 = _batch(hp, 4, 23)
+    U0 = _batch(hp, nblocks, 23)
     dx = tuple(1.0 / n for n in shape)
     dt = W.cfl_dt(U0, 3, 4, dx, 0.4)
     hy = Hydro(hp)
@@ -30,7 +33,7 @@ def test_solve_and_update_at_every_height(shape, prec, seeded):
         if seeded:
             gen = torch.Generator().manual_seed(5)
             hy.set_seed_params((torch.randn(L.NPARAM, generator=gen) * 0.1).float().cuda())
-            L.set_gate(0.05)
+            L.set_gate(gate)
         for path in (2, 0):
             hy.set_kernel_path(path)
             U = U0.cuda()
