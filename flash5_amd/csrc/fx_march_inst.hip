@@ -26,9 +26,13 @@ void launch_march_f(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
     }
   }
   constexpr int NT3 = sizeof(R) == 8 ? 768 : 512;  // FP64 3-D 16x8: 768 threads
+  // FP64 2-D 16x8: 448 threads, since stage A has seven wavefronts of items
+  // (4096 x 16^2 293 -> 270 us; two workgroups a CU either way).  FP32 runs
+  // four workgroups of 384 on a CU instead.
+  constexpr int NT2 = sizeof(R) == 8 ? 448 : 384;
   if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, NT3, RS, R, OCC, FUSE>), grid, dim3(NT3), 0, H.stream, P, M);
   else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, OCC, FUSE>), grid, dim3(384), 0, H.stream, P, M);
-  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, 384, RS, R, OCC, FUSE>), grid, dim3(384), 0, H.stream, P, M);
+  else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, NT2, RS, R, OCC, FUSE>), grid, dim3(NT2), 0, H.stream, P, M);
   else hipLaunchKernelGGL((k_march<2, 8, 8, 256, RS, R, OCC, FUSE>), grid, dim3(256), 0, H.stream, P, M);
 }
 
@@ -57,9 +61,9 @@ void launch_march_free(const DevParams& P, const MarchLaunch& M, hipStream_t str
   else if (P.ndim == 3)
     hipLaunchKernelGGL((k_march_free<3, 768, RS, double, 3, kFuseScratch>), grid, dim3(768), 0, stream, P, M);
   else if (M.fuse == kFuseDirect)
-    hipLaunchKernelGGL((k_march_free<2, 384, RS, double, 3, kFuseDirect>), grid, dim3(384), 0, stream, P, M);
+    hipLaunchKernelGGL((k_march_free<2, 448, RS, double, 3, kFuseDirect>), grid, dim3(448), 0, stream, P, M);
   else
-    hipLaunchKernelGGL((k_march_free<2, 384, RS, double, 3, kFuseScratch>), grid, dim3(384), 0, stream, P, M);
+    hipLaunchKernelGGL((k_march_free<2, 448, RS, double, 3, kFuseScratch>), grid, dim3(448), 0, stream, P, M);
 }
 #ifdef FX_MARCH_FREE
 template void launch_march_free<FX_MARCH_RS>(const DevParams&, const MarchLaunch&, hipStream_t);
