@@ -17,7 +17,7 @@ struct DevStatus {
   unsigned long long fallbacks;
   unsigned long long newtonIters;
   unsigned long long newtonFallbacks;
-  unsigned long long shockTiles;  // tiles with a flagged cell (k_shock_detect)
+  unsigned long long shockTiles;  // tiles, or their segments, with a flagged cell (k_shock_detect)
 };
 
 struct Launch {

@@ -287,7 +287,10 @@ k_fluxes(DevParams P, Launch L) {
   flush_exact(L.status, es);
 }
 
-// hy_shockDetectBlk.F90:93-229, one workgroup per tile.  SHOK_VAR := 0 on
+// hy_shockDetectBlk.F90:93-229, one workgroup per tile, or gridDim.y of them
+// along z where tiles alone are few (shock_segments).  Bound by the latency of
+// a plane's loads, division and root before the next plane's; a segment forms
+// the minima of the planes next to it anew.  SHOK_VAR := 0 on
 // guard cells; interior cells take the Balsara-Spicer flag (undivided
 // pressure jump >= 0.5 of the 3^d minimum pressure and undivided velocity
 // divergence <= -0.1 of the 3^d minimum sound speed).  The workgroup marches
@@ -323,13 +326,16 @@ __global__ void __launch_bounds__(kThreads) k_shock_detect(Launch L, DevParams P
   double* __restrict__ plane = sm;                 // [2][nplane]: p, then c
   double* __restrict__ hist = sm + 2 * nplane;     // 3-D: [2 planes][2][ncol] 3x3 minima
   // guard cells of SHOK_VAR (hy_shockDetectBlk.F90:117)
-  for (long c = threadIdx.x; c < P.ncell; c += blockDim.x) {
+  for (long c = (long)blockIdx.y * blockDim.x + threadIdx.x; c < P.ncell;
+       c += (long)blockDim.x * gridDim.y) {
     const int i = (int)(c % P.nx), j = (int)((c / P.nx) % P.ny), k = (int)(c / sz);
     if (i < P.lo[0] || i > P.hi[0] || j < P.lo[1] || j > P.hi[1] || k < P.lo[2] || k > P.hi[2])
       U[P.shokOff + c] = 0.;
   }
   int any = 0;
-  const int klo = P.lo[2] - k3, khi = P.hi[2] + k3;
+  const int per = (P.hi[2] - P.lo[2] + (int)gridDim.y) / (int)gridDim.y;
+  const int first = P.lo[2] + (int)blockIdx.y * per, last = min(first + per - 1, P.hi[2]);
+  const int klo = first - k3, khi = first <= last ? last + k3 : klo - 1;
   for (int k = klo; k <= khi; ++k) {
     for (int q = threadIdx.x; q < nplane; q += blockDim.x) {
       const int i = P.lo[0] - 1 + q % nx2, j = P.lo[1] - k2 + q / nx2;
@@ -1482,17 +1488,30 @@ void launch_step_cfl() {
                      fallback_cfl_cap(g.prm), g.dtBuf + 2);
 }
 
-// k_shock_detect over the uploaded tiles, one workgroup each, with the LDS
-// of the largest class present
+// Segments of a tile's planes for the detector: about four workgroups a
+// compute unit, of two planes at least.  18 blocks of 16^3 100 -> 38 us (the
+// call), 128 119 -> 56, 512 157 -> 116; from 1024 on one workgroup a tile.
+unsigned shock_segments(int nTiles, int nz) {
+  const long want = (4L * g.numCU + nTiles - 1) / nTiles;
+  return (unsigned)std::max(1L, std::min(want, (long)nz / 2));
+}
+
+// k_shock_detect over the uploaded tiles, with the LDS of the largest class
+// present
 void launch_shock_detect(int nTiles) {
+  if (nTiles < 1) return;
   Launch L{g.dtiles, nTiles, nullptr, g.status, 0.0, nullptr};
+  int nz = g.cur.ndim > 2 ? g.cur.nzb : 1;
   if (g.multi) {
     long lds = 0;
-    for (const DevParams& P : g.hcls) lds = std::max(lds, shock_lds_doubles(P));
-    hipLaunchKernelGGL(k_shock_detect, dim3(nTiles), dim3(kThreads), sizeof(double) * lds,
+    for (const DevParams& P : g.hcls) {
+      lds = std::max(lds, shock_lds_doubles(P));
+      nz = std::min(nz, P.ndim > 2 ? P.nzb : 1);
+    }
+    hipLaunchKernelGGL(k_shock_detect, dim3(nTiles, shock_segments(nTiles, nz)), dim3(kThreads), sizeof(double) * lds,
                        g.stream, L, g.cur, g.dcls, g.dtcls);
   } else {
-    hipLaunchKernelGGL(k_shock_detect, dim3(nTiles), dim3(kThreads),
+    hipLaunchKernelGGL(k_shock_detect, dim3(nTiles, shock_segments(nTiles, nz)), dim3(kThreads),
                        sizeof(double) * shock_lds_doubles(g.cur), g.stream, L, g.cur,
                        (const DevParams*)nullptr, (const unsigned char*)nullptr);
   }

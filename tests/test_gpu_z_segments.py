@@ -54,3 +54,28 @@ def test_segments_match_whole_columns(shape, nblocks, kw, prec, path):
     assert torch.isfinite(out[0][0]).all()
     assert torch.equal(out[0][0], out[1][0])
     assert not torch.equal(out[0][0], U0.cuda())
+
+
+@pytest.mark.parametrize("shape,nblocks", [((16, 16, 16), 1), ((8, 8, 17), 60), ((12, 10, 5), 7),
+                                           ((8, 8, 2), 3), ((16, 16), 5)])
+def test_detector_segments_match_whole_tiles(shape, nblocks):
+    ndim = len(shape)
+    s3 = tuple(shape) + (1,) * (3 - ndim)
+    hp = HydroParams(ndim=ndim, nxb=s3[0], nyb=s3[1], nzb=s3[2], gamma=1.4,
+                     RiemannSolver="hybrid", nunk=11, shokVar=10, shockLowerCFL=True)
+    U0 = _batch(hp, nblocks, 41)
+    gen = torch.Generator().manual_seed(3)
+    U0[:, 4] *= 1.0 + 4.0 * (torch.rand(U0[:, 4].shape, generator=gen) < 0.3)
+    U0[:, 1:4] *= 3.0
+    copies = -(-1100 // nblocks)
+    hy = Hydro(hp)
+    out = []
+    for n in (1, copies):
+        U = U0.cuda().repeat(n, 1, 1, 1, 1)
+        U[:, 10] = 7.0                                    # every cell is written
+        st = hy.shock_detect_batch(U, tuple(1.0 / k for k in s3))
+        out.append((U, st.min_cell_cfl))
+    flags = out[0][0][:, 10]
+    assert set(flags.unique().tolist()) == {0.0, 1.0}
+    assert out[0][1] == out[1][1] > 0.0
+    assert torch.equal(out[0][0].repeat(copies, 1, 1, 1, 1), out[1][0])
