@@ -1018,6 +1018,7 @@ struct Lib {
   double* fillDt = nullptr;            // fx_grid_fill_guards_dt: this call's minimum, the next one's
   bool fillDtReady = false;
   int fillDtTurn = 0;
+  int freeOf[2] = {0, 0}, freeTile[2] = {0, 0};  // free_shape's tile of these block extents
   double runCfl = 0.;                  // the CFL argument of the graph-captured run
   hipStream_t capStream = nullptr;     // library stream for graph capture (default priority)
   std::vector<int> hnbr;               // neighbour table last uploaded (host copy)
@@ -1240,20 +1241,27 @@ bool march_shape(const DevParams& P, int* TX, int* TY, int* NT) {
 }
 
 // Column tiles of a block that no fixed tile divides: the fewest equal ones
-// that fit the 16x8 layout, the last along an axis with what is left.
+// that fit the 16x8 layout, the last along an axis with what is left.  The
+// march addresses a block's array by 32-bit byte offsets, so larger blocks
+// keep the three-kernel path.
 bool free_shape(const DevParams& P, int* tx, int* ty) {
-  if (P.ndim < 2) return false;
-  int best = 1 << 30;
-  for (int nx = 1; nx <= P.nxb; ++nx)
-    for (int ny = 1; ny <= P.nyb; ++ny) {
-      const int x = (P.nxb + nx - 1) / nx, y = (P.nyb + ny - 1) / ny;
-      if (nx * ny < best && free_tile_fits<16, 8>(x, y)) {
+  if (P.ndim < 2 || P.ncell * P.nunk > 0x7fffffffL / 8) return false;
+  if (g.freeOf[0] != P.nxb || g.freeOf[1] != P.nyb) {
+    int best = 1 << 30;
+    for (int x = 1; x <= P.nxb && free_tile_fits<16, 8>(x, 1); ++x)
+      for (int y = 1; y <= P.nyb && free_tile_fits<16, 8>(x, y); ++y) {
+        const int nx = (P.nxb + x - 1) / x, ny = (P.nyb + y - 1) / y;
+        if ((long)nx * ny >= best) continue;
         best = nx * ny;
-        *tx = x;
-        *ty = y;
+        g.freeTile[0] = (P.nxb + nx - 1) / nx;
+        g.freeTile[1] = (P.nyb + ny - 1) / ny;
       }
-    }
-  return best < 1 << 30;
+    g.freeOf[0] = P.nxb;
+    g.freeOf[1] = P.nyb;
+  }
+  *tx = g.freeTile[0];
+  *ty = g.freeTile[1];
+  return true;
 }
 
 // How many segments along z the column tiles of a launch are cut into, and
@@ -1302,12 +1310,11 @@ long march_slots(const DevParams& P, int TX) {
 // path.  In 3-D a column tile takes a compute unit for its planes and three
 // more, about 4 us each and 6 more with all 128 columns in use; the three
 // kernels take about 0.27 ns a state cell and 40 us for their launches and
-// latency, however few the blocks.  Measured either side of the line, free
-// against three kernels: 12 blocks of 20^3 226 / 120 us and 200 887 / 1284,
-// 28 of 9 x 7 x 11 125 / 75 and 144 134 / 152, 59 of 12 x 10 x 14 158 / 134
-// and 238 179 / 395, 92 of 6^3 71 / 79.  In 2-D (one plane) free tiles were
-// faster at every size: 200 blocks of 10^2 32 / 52, 1250 of 20 x 16 173 / 175,
-// 16000 of 10^2 490 / 764.
+// latency, however few the blocks.  Free against three kernels: 11 blocks of
+// 12 x 10 x 14 56 / 63 us and 952 664 / 1460, 4 of 20^3 63 / 75 and 200 866 /
+// 1273, 92 of 6^3 62 / 76; blocks of 2^3, whose tiles are nearly empty, keep
+// the three kernels.  In 2-D (one plane) free tiles were faster at every size:
+// 200 blocks of 10^2 32 / 52, 1250 of 20 x 16 165 / 175, 16000 of 10^2 455 / 761.
 bool free_pays(const DevParams& P, long n, int tx, int ty) {
   if (P.ndim == 2) return true;
   const long tiles = (long)((P.nxb + tx - 1) / tx) * ((P.nyb + ty - 1) / ty);

@@ -683,7 +683,8 @@ __global__ void k_zero_count(unsigned* c) { c[threadIdx.x] = 0u; }
 // ones), which the face stage that reads a seed per face needs.  The batch
 // step's list-driven solve does not: there the march lists the strong faces
 // itself (list_strong_face), since this pass over the states took 251 us of
-// 3117 on 2048 x 16^3 mixed, and the list adds 69 us to the march (the step 3117 -> 3040 us).
+// 3117 on 2048 x 16^3 mixed, and the list adds 69 us to the march (the step
+// 3117 -> 3040 us).
 template <bool MULTI, typename S>
 __global__ void __launch_bounds__(kThreads) k_face_gate(DevParams P0, FaceLaunch F, SeedGate G,
                                                         float* __restrict__ y,

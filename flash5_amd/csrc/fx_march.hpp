@@ -1194,9 +1194,9 @@ k_march(DevParams P, MarchLaunch L) {
 // reciprocal multiplication per item; its loads, arithmetic and bits are the
 // fixed tile's.
 // Bound by FP64 issue and latency as k_march, and by what of the 128 columns a
-// tile leaves idle.  952 blocks of 12 x 10 x 14 679 us against 1464 by the three-
+// tile leaves idle.  952 blocks of 12 x 10 x 14 664 us against 1460 by the three-
 // kernel path (face states through memory, transverse fluxes formed anew by
-// each state cell), 402 of 13 x 17 x 18 853 / 1399, 7407 of 6^3 1675 / 2033.
+// each state cell), 402 of 13 x 17 x 18 853 / 1399, 7407 of 6^3 1669 / 2026.
 template <int NDIM, int NT, int RS, typename R, int OCC, int FUSE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 k_march_free(DevParams P, MarchLaunch L) {
