@@ -2157,6 +2157,9 @@ int upload_neighbors(double* U, long nBlocks, long blockStride, const int* nbr, 
     if (st) st->code = 3;
     return 3;
   }
+  // a queued fill (asynchronous calls, wait = 0) still reads the old table, on
+  // this stream or on one that the library worked on before
+  HIPCALL(hipDeviceSynchronize(), st);
   g.nbrDim = 0;
   if (grow(&g.dnbr, &g.dnbrCap, n6, st)) return 4;
   g.hnbr.assign(nbr, nbr + n6);
