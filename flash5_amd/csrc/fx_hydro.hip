@@ -995,6 +995,8 @@ struct Lib {
   size_t dregClsCap = 0;
   std::vector<unsigned char> hregCls;
   float* gradPart = nullptr;           // k_mlp_grad's rows, one per workgroup
+  hipEvent_t gradDone = nullptr;       // behind the last asynchronous call that uses them
+  bool gradBusy = false;               // such a call may still run
   MlpPacked* mlpPacked = nullptr;      // BF16 fragments for fx_mlp_* / fx_riemann_batch
   MlpPacked* seedPacked = nullptr;     // network seeding the exact solver in hydro steps
   bool seedReady = false;
@@ -2492,6 +2494,7 @@ void fx_hydro_finalize(void) {
     if (b) (void)hipFree(b);
   for (hipEvent_t e : g.ev)
     if (e) (void)hipEventDestroy(e);
+  if (g.gradDone) (void)hipEventDestroy(g.gradDone);
   if (g.capStream) (void)hipStreamDestroy(g.capStream);
   amr_free();
   g = Lib{};
@@ -2691,18 +2694,39 @@ int fx_mlp_grad(const float* params, const float* x, const float* t, long n, flo
                 float* grad, float* loss) {
   if (n <= 0) return 0;
   if (!params || !x || !t || !grad || !loss) return 3;
-  if (ensure_status(nullptr) || pack_mlp(params, &g.mlpPacked, nullptr)) return 4;
   // one workgroup per CU at most
+  if (ensure_status(nullptr)) return 4;
+  const long per = kGradWaves * kGradCols;
+  const unsigned rows = (unsigned)std::min((n + per - 1) / per, (long)g.numCU);
+  const dim3 block(kGradWaves * 64);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (g.async && g.stream) HIPCALL(hipStreamIsCapturing(g.stream, &cap), nullptr);
+  if (cap != hipStreamCaptureStatusNone) {
+    if (pack_mlp(params, &g.mlpPacked, nullptr)) return 4;
+    hipLaunchKernelGGL(k_mlp_grad<false>, dim3(rows), block, 0, g.stream, g.mlpPacked, x, t, n,
+                       scale, (float*)nullptr, grad, loss);
+    return sync_or_async(nullptr);
+  }
+  // the rows (and the packed network) of a call queued on another stream
+  if (g.gradBusy) HIPCALL(hipStreamWaitEvent(g.stream, g.gradDone, 0), nullptr);
+  if (pack_mlp(params, &g.mlpPacked, nullptr)) return 4;
   if (!g.gradPart &&
       hipMalloc((void**)&g.gradPart, sizeof(float) * kGradStride * g.numCU) != hipSuccess)
     return 4;
-  const long per = kGradWaves * kGradCols;
-  const unsigned rows = (unsigned)std::min((n + per - 1) / per, (long)g.numCU);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(kGradWaves * 64), 0, g.stream, g.mlpPacked, x, t,
-                     n, scale, g.gradPart);
+  hipLaunchKernelGGL(k_mlp_grad<true>, dim3(rows), block, 0, g.stream, g.mlpPacked, x, t, n, scale,
+                     g.gradPart, (float*)nullptr, (float*)nullptr);
   hipLaunchKernelGGL(k_mlp_grad_sum, dim3(MLP_NPARAM / 64 + 1), dim3(kThreads), 0, g.stream,
                      g.gradPart, (int)rows, grad, loss);
-  return sync_or_async(nullptr);
+  if (g.async) {
+    if (!g.gradDone)
+      HIPCALL(hipEventCreateWithFlags(&g.gradDone, hipEventDisableTiming), nullptr);
+    HIPCALL(hipEventRecord(g.gradDone, g.stream), nullptr);
+    g.gradBusy = true;
+    return sync_or_async(nullptr);
+  }
+  if (sync_or_async(nullptr)) return 4;
+  g.gradBusy = false;
+  return 0;
 }
 
 int fx_mlp_adam(float* params, const float* grad, float* m, float* v, int step, float lr) {

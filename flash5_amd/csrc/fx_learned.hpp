@@ -69,13 +69,17 @@ __global__ void __launch_bounds__(kLearnThreads) k_mlp_forward(const MlpPacked* 
 // 114 us, nearly all of it atomics on the same 4673 words; FP32 LDS atomics (some
 // 125 cycles each) and rows 33 us; sums in registers and rows 11 us, with 4 us
 // for k_mlp_grad_sum.  65536 of them 20 us, 262144 59 us.
+// ROWS = false adds a workgroup's sums to the gradient and the loss themselves,
+// for calls under capture: their replays may run beside another call, and the
+// library has one set of rows.
 constexpr int kGradStride = 4736;           // row of part, 64-float multiples
 constexpr int kGradSegs = kThreads / 64;    // k_mlp_grad_sum: rows split over wavefronts
+template <bool ROWS>
 __global__ void __launch_bounds__(kGradWaves * 64) k_mlp_grad(const MlpPacked* __restrict__ W,
                                                               const float* __restrict__ x,
                                                               const float* __restrict__ t, long n,
-                                                              float scale,
-                                                              float* __restrict__ part) {
+                                                              float scale, float* __restrict__ part,
+                                                              float* grad, float* loss) {
   __shared__ float xs[kGradWaves][kGradCols * 8];
   __shared__ __attribute__((aligned(16))) __bf16 sZ[64 * kGradRow];
   __shared__ __attribute__((aligned(16))) __bf16 sH[64 * kGradRow];
@@ -114,30 +118,35 @@ __global__ void __launch_bounds__(kGradWaves * 64) k_mlp_grad(const MlpPacked* _
 #pragma unroll
   for (int q = 0; q < 16; ++q) sU[wv][16 * (q / 4) + 4 * g + q % 4][c] = acc.unit[q];
   __syncthreads();
-  float* const row = part + (long)blockIdx.x * kGradStride;
+  float* const row = ROWS ? part + (long)blockIdx.x * kGradStride : nullptr;
+  auto put = [&](int k, float v) {
+    if (ROWS) row[k] = v;
+    else atomicAdd(k == MLP_NPARAM ? loss : grad + k, v);
+  };
 #pragma unroll
   for (int ut = 0; ut < 4; ++ut)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      row[OFF_W2 + (16 * wv + 4 * g + i) * MLP_H + 16 * ut + c] = acc.w2[ut][i];
+      put(OFF_W2 + (16 * wv + 4 * g + i) * MLP_H + 16 * ut + c, acc.w2[ut][i]);
   for (int e = threadIdx.x; e < 64 * 16; e += kGradWaves * 64) {
     const int u = e / 16, q = e % 16;
     if (q > 8) continue;
     float v = sU[0][u][q];
 #pragma unroll
     for (int w = 1; w < kGradWaves; ++w) v += sU[w][u][q];
-    row[q < MLP_IN ? OFF_W1 + u * MLP_IN + q
-                   : (q == 6 ? OFF_B1 : (q == 7 ? OFF_B2 : OFF_W3)) + u] = v;
+    put(q < MLP_IN ? OFF_W1 + u * MLP_IN + q
+                   : (q == 6 ? OFF_B1 : (q == 7 ? OFF_B2 : OFF_W3)) + u, v);
   }
   if (threadIdx.x < 2) {
     float v = sB[0][threadIdx.x];
 #pragma unroll
     for (int w = 1; w < kGradWaves; ++w) v += sB[w][threadIdx.x];
-    row[threadIdx.x == 0 ? OFF_B3 : MLP_NPARAM] = v;
+    put(threadIdx.x == 0 ? OFF_B3 : MLP_NPARAM, v);
   }
 }
 
-// grad += and loss += the sums of part's rows
+// grad += and loss += the sums of part's rows, by atomics: a replayed call may be
+// adding to the same gradient
 __global__ void __launch_bounds__(kThreads) k_mlp_grad_sum(const float* __restrict__ part, int rows,
                                                            float* grad, float* loss) {
   __shared__ float seg[kGradSegs][64];
@@ -153,8 +162,7 @@ __global__ void __launch_bounds__(kThreads) k_mlp_grad_sum(const float* __restri
   if (s == 0 && k <= MLP_NPARAM) {
 #pragma unroll
     for (int q = 1; q < kGradSegs; ++q) v += seg[q][lane];
-    if (k == MLP_NPARAM) *loss += v;
-    else grad[k] += v;
+    atomicAdd(k == MLP_NPARAM ? loss : grad + k, v);
   }
 }
 

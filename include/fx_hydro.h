@@ -253,7 +253,8 @@ int fx_fluxreg_conserve(const fx_tile* coarse, int nCoarse, const fx_fluxreg_fac
 enum { FX_MLP_NPARAM = 4673 };
 int fx_mlp_features(const double* states, long n, double gamma, float* x /* [n][6] */);
 int fx_mlp_forward(const float* params, const float* x, long n, float* y);
-/* grad += d/dparams of scale*sum_n (y_n - t_n)^2; *loss += the same sum */
+/* grad += d/dparams of scale*sum_n (y_n - t_n)^2; *loss += the same sum.  Calls
+ * on several streams may overlap and may add to the same grad and loss. */
 int fx_mlp_grad(const float* params, const float* x, const float* t, long n, float scale,
                 float* grad, float* loss);
 /* one Adam step (beta 0.9, 0.999, eps 1e-8) on FP32 master parameters */
