@@ -209,19 +209,37 @@ class UniformGrid:
             raise FxError("fx_grid_fill_guards_dt", st, rc)
         return dt.value
 
+    def _replaced(self) -> bool:
+        """Whether fill_guards or hydro.compute_dt is another than this
+        package's (a subclass's, or one set on the class or the object)."""
+        return (getattr(self.fill_guards, "__func__", None) is not _FILL_GUARDS or
+                getattr(self.hydro.compute_dt, "__func__", None) is not _COMPUTE_DT)
+
     def step(self, dt_max: float = math.inf) -> float:
         """Guard fill, CFL dt (capped by dt_max), unsplit update in place.
         With shock detection on: fill, flag, fill again, as Hydro.F90:94-123
         orders them; the detector writes SHOK_VAR only, so the second fill
         takes that variable alone (512 blocks of 16^3: 510 -> 30 us).  Under shockLowerCFL or
         hy_fallbackLowerCFL the dt takes the CFL that the previous step's
-        flags and fallbacks left (step_cfl)."""
+        flags and fallbacks left (step_cfl).  Fill and dt go out in one launch;
+        a fill_guards or hydro.compute_dt of the program's own is called
+        instead, as fill, flag, fill, dt."""
         cfl = self._cfl_next
-        dt = min(self._fill_guards_dt(cfl), dt_max)
+        own = self._replaced()
+        if own:
+            self.fill_guards()
+        else:
+            dt = self._fill_guards_dt(cfl)
         shock_cap = 0.0
         if self.detect:
             shock_cap = self.hydro.shock_detect_batch(self.U, self.deltas).min_cell_cfl
-            self.fill_guards(self.params.shokVar, wait=False)
+            if own:
+                self.fill_guards()
+            else:
+                self.fill_guards(self.params.shokVar, wait=False)
+        if own:
+            dt = self.hydro.compute_dt(self.U, self.deltas, cfl)
+        dt = min(dt, dt_max)
         st = self.hydro.advance_batch(self.U, dt, self.deltas)
         self._cfl_next = step_cfl(self.cfl, cfl, self.detect, shock_cap, st.fallback_cfl)
         self.t += dt
@@ -263,6 +281,10 @@ class UniformGrid:
             n += 1
         torch.cuda.synchronize()
         return RunStats(n, self.t, time.perf_counter() - t0, n * zones, fb)
+
+
+# this package's own, for UniformGrid._replaced
+_FILL_GUARDS, _COMPUTE_DT = UniformGrid.fill_guards, Hydro.compute_dt
 
 
 def sod(nblk: int = 16, nb: int = 8, tmax: float = 0.2, **kw):
