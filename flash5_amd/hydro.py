@@ -174,6 +174,10 @@ def load_library(path: str = LIB_PATH):
     if not os.path.exists(path):
         raise FileNotFoundError(
             f"{path} is missing: build it with `python -m flash5_amd.build` (hipcc, gfx950)")
+    # torch first: its HIP runtime then serves this library too, where a torch
+    # imported later would bring a second one into the process, and neither
+    # would know the other's streams and memory
+    import torch  # noqa: F401
     L = C.CDLL(path)
     for name, (args, res) in EXPORTS.items():
         fn = getattr(L, name)
