@@ -1071,6 +1071,7 @@ struct Lib {
   int itemsOrder = 0;                  // item order they were built in
   int persist = 0;                     // multi-class march: multiple of the resident workgroups (0 = 1)
   int tuneTX = 0;                      // autotuned column-tile width (0: built-in choice)
+  int tuneFusedTX = 0;                 // the same of batch steps with the update in the march
   int tuneOcc = 0;                     // autotuned waves-per-SIMD hint of the FP32 3-D march (0 or 4)
   int itemOrder = 0;                   // multi-class items: 0 longest first, 1 tile by tile
   unsigned long uploadGen = 0;         // counts tile-list uploads
@@ -1226,10 +1227,11 @@ DevParams make_dev_params(const fx_params& p) {
 
 // Column-tile shape of the fused kernel for this block shape, or false
 // when only the three-kernel path applies (1-D, or sizes not tileable).
-bool march_shape(const DevParams& P, int* TX, int* TY, int* NT) {
+// tuned: the autotuned width, 0 for the built-in one
+bool march_shape(const DevParams& P, int* TX, int* TY, int* NT, int tuned) {
   if (P.ndim < 2) return false;
   const int nx = P.nxb, ny = P.nyb;
-  if (nx % 16 == 0 && ny % 8 == 0 && g.tuneTX != 8) {
+  if (nx % 16 == 0 && ny % 8 == 0 && tuned != 8) {
     *TX = 16;
     *TY = 8;
   } else if (nx % 8 == 0 && ny % 8 == 0) {
@@ -1332,7 +1334,13 @@ bool free_pays(const DevParams& P, long n, int tx, int ty) {
 bool batch_fused(const DevParams& P, long n) {
   int tx, ty, NT;
   if (g.legacy || g.solveUpdOff || P.riemann == FX_EXACT || P.fP != 1.0) return false;
-  return march_shape(P, &tx, &ty, &NT) || (free_shape(P, &tx, &ty) && free_pays(P, n, tx, ty));
+  return march_shape(P, &tx, &ty, &NT, 0) || (free_shape(P, &tx, &ty) && free_pays(P, n, tx, ty));
+}
+
+// Column tile of a batch step of n blocks.  A step with the update inside is
+// another kernel than the flux stages and was tuned on its own.
+bool batch_shape(const DevParams& P, long n, int* TX, int* TY, int* NT) {
+  return march_shape(P, TX, TY, NT, batch_fused(P, n) ? g.tuneFusedTX : g.tuneTX);
 }
 
 // Where the update of n such blocks runs.  kFuseDirect gives a block's column
@@ -1934,7 +1942,10 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
       }
   }
   int TX = 0, TY = 8, NT = 0;
-  const bool march = g.multi ? multi_march_shape(&TX) : (!g.legacy && march_shape(P, &TX, &TY, &NT));
+  const bool batch = tilesUploaded && !tiles && !inPlace && !g.multi;
+  const bool march = g.multi ? multi_march_shape(&TX)
+                             : (!g.legacy && (batch ? batch_shape(P, nTiles, &TX, &TY, &NT)
+                                                    : march_shape(P, &TX, &TY, &NT, g.tuneTX)));
   if (P.learned && (!march || !g.seedReady)) {  // the seed needs the march path and a network
     if (st) st->code = 3;
     return 3;
@@ -1953,7 +1964,7 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     // batch steps with the exact solver: its face stage and the update run
     // as one kernel (k_solve_update) for 3-D blocks up to 16 x 16 across
     // (where the batch is large enough for that)
-    const bool solveUpdate = tilesUploaded && !tiles && !inPlace && !g.multi && !g.solveUpdOff &&
+    const bool solveUpdate = batch && !g.solveUpdOff &&
                              P.riemann == FX_EXACT && P.ndim == 3 &&
                              P.nxb * P.nyb <= kSolveMaxCols &&
                              P.nxb <= kSolveMaxSide && P.nyb <= kSolveMaxSide &&
@@ -1964,13 +1975,12 @@ int run_compute(const fx_tile* tiles, int nTiles, double dt, const unsigned char
     if (solveUpdate && P.learned && ensure_seed_patch(g.hfaceStart[nTiles], nTiles, st)) return 4;
     if (!g.capturing) hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
     if (record(0)) return 4;
-    const int fuse = tilesUploaded && !tiles && !inPlace && !g.multi
-                         ? batch_fuse_mode(P, TX, TY, nTiles) : kFuseNone;
+    const int fuse = batch ? batch_fuse_mode(P, TX, TY, nTiles) : kFuseNone;
     if (launch_flux_stages(nTiles, dt, TX, TY, solveUpdate, fuse)) return 4;
     if (fuse == kFuseScratch) launch_update_finish(P, g.dtiles, nTiles, g.upd);
     else if (fuse == kFuseNone && !solveUpdate && anyInPlace) launch_update(nTiles, dt, dIn);
     if (record(3)) return 4;
-  } else if (tilesUploaded && !tiles && !inPlace && !g.multi && batch_fused(P, nTiles)) {
+  } else if (batch && batch_fused(P, nTiles)) {
     if (!g.capturing) hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
     if (record(0)) return 4;
     if (launch_free(P, nTiles, dt)) return 4;
@@ -2205,11 +2215,62 @@ void launch_fill(double* U, long nBlocks, long blockStride, int onlyVar = -1,
 // ---------------------------------------------------------------------
 // autotuner: launch shapes of the flux stages timed on the caller's batch
 // ---------------------------------------------------------------------
+struct TuneCand {
+  int tx, persist, order, occ;
+};
+
+// The fastest of each candidate's reps runs, in ms (-1: setup refused it), and
+// the fastest candidate.  before(c) runs ahead of every run(c), not timed; the
+// first run of a candidate warms up.
+template <typename Setup, typename Before, typename Run>
+int time_candidates(const std::vector<TuneCand>& cands, int reps, Setup setup, Before before,
+                    Run run, std::vector<float>& ms, int* best, fx_status* st) {
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  HIPCALL(hipEventCreate(&e0), st);
+  HIPCALL(hipEventCreate(&e1), st);
+  const int savedTiming = g.timing;
+  g.timing = 0;
+  ms.assign(cands.size(), -1.f);
+  *best = -1;
+  int rc = 0;
+  for (size_t c = 0; c < cands.size() && !rc; ++c) {
+    bool skip = false;
+    rc = setup(cands[c], &skip);
+    if (rc || skip) continue;
+    for (int r = 0; r <= reps && !rc; ++r) {
+      float t = 0.f;
+      if (before() || hipEventRecord(e0, g.stream) != hipSuccess || run(cands[c]) ||
+          hipEventRecord(e1, g.stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+          hipEventElapsedTime(&t, e0, e1) != hipSuccess)
+        rc = 4;
+      else if (r > 0 && (ms[c] < 0.f || t < ms[c]))
+        ms[c] = t;
+    }
+    if (!rc && (*best < 0 || ms[c] < ms[*best])) *best = (int)c;
+  }
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
+  g.timing = savedTiming;
+  if (!rc && *best < 0) rc = 3;
+  if (rc && st) st->code = rc;
+  return rc;
+}
+
+void tune_report(const std::vector<TuneCand>& cands, const std::vector<float>& ms, int best,
+                 fx_tune_result* out, int cap, int* n) {
+  int k = 0;
+  for (size_t c = 0; c < cands.size(); ++c) {
+    if (ms[c] < 0.f) continue;
+    if (out && k < cap)
+      out[k] = fx_tune_result{cands[c].tx, cands[c].persist, cands[c].order, cands[c].occ,
+                              (int)c == best, ms[c]};
+    ++k;
+  }
+  if (n) *n = k;
+}
+
 int tune_flux_stages(int nTiles, double dt, int reps, fx_tune_result* out, int cap, int* n,
                      int* chosenTX, fx_status* st) {
-  struct Cand {
-    int tx, persist, order, occ;
-  };
   const DevParams& P = g.cur;
   bool can16 = true, any16 = false;
   if (g.multi) {
@@ -2220,7 +2281,7 @@ int tune_flux_stages(int nTiles, double dt, int reps, fx_tune_result* out, int c
   } else {
     can16 = P.nxb % 16 == 0 && P.nyb % 8 == 0;
   }
-  std::vector<Cand> cands;
+  std::vector<TuneCand> cands;
   // waves-per-SIMD hint 4 for the FP32 3-D march: at most 128 VGPRs (a few
   // spills), so that two 512-thread workgroups share a CU
   const bool occ4 = P.precision == FX_PREC_MIXED && P.ndim == 3;
@@ -2231,63 +2292,38 @@ int tune_flux_stages(int nTiles, double dt, int reps, fx_tune_result* out, int c
       if (tx == kPerClassTX && (!g.multi || can16 || !any16)) continue;
       if (g.multi) {
         for (int persist : {1, 2, 4})
-          for (int order : {0, 1}) cands.push_back(Cand{tx, persist, order, occ});
+          for (int order : {0, 1}) cands.push_back(TuneCand{tx, persist, order, occ});
       } else {
-        cands.push_back(Cand{tx, 0, 0, occ});
+        cands.push_back(TuneCand{tx, 0, 0, occ});
       }
     }
   }
   if (ensure_step_scratch(nTiles, st)) return 4;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  HIPCALL(hipEventCreate(&e0), st);
-  HIPCALL(hipEventCreate(&e1), st);
-  const int savedTiming = g.timing;
-  g.timing = 0;
-  int best = -1, rc = 0;
-  float bestMs = 0.f;
-  std::vector<float> ms(cands.size(), -1.f);
-  for (size_t c = 0; c < cands.size() && !rc; ++c) {
-    g.tuneTX = cands[c].tx;
-    g.persist = cands[c].persist;
-    g.itemOrder = cands[c].order;
-    g.tuneOcc = cands[c].occ;
-    int TX = 8, TY = 8, NT = 0;
-    const bool ok = g.multi ? multi_march_shape(&TX) : march_shape(P, &TX, &TY, &NT);
-    if (!ok) continue;
-    if (g.multi && build_march_items(nTiles, TX, st)) {
-      rc = 4;
-      break;
-    }
+  int TX = 8, TY = 8, NT = 0, best = -1;
+  std::vector<float> ms;
+  auto use = [&](const TuneCand& c) {
+    g.tuneTX = c.tx;
+    g.persist = c.persist;
+    g.itemOrder = c.order;
+    g.tuneOcc = c.occ;
+  };
+  auto setup = [&](const TuneCand& c, bool* skip) -> int {
+    use(c);
+    *skip = g.multi ? !multi_march_shape(&TX) : !march_shape(P, &TX, &TY, &NT, g.tuneTX);
+    if (*skip) return 0;
+    if (g.multi && build_march_items(nTiles, TX, st)) return 4;
     hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, g.stream, g.status);
-    if (launch_flux_stages(nTiles, dt, TX, TY)) rc = 4;  // warm-up
-    for (int r = 0; r < reps && !rc; ++r) {
-      float t = 0.f;
-      if (hipEventRecord(e0, g.stream) != hipSuccess || launch_flux_stages(nTiles, dt, TX, TY) ||
-          hipEventRecord(e1, g.stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-          hipEventElapsedTime(&t, e0, e1) != hipSuccess) {
-        rc = 4;
-        break;
-      }
-      if (ms[c] < 0.f || t < ms[c]) ms[c] = t;
-    }
-    if (!rc && ms[c] >= 0.f && (best < 0 || ms[c] < bestMs)) {
-      best = (int)c;
-      bestMs = ms[c];
-    }
+    return 0;
+  };
+  const int rc = time_candidates(
+      cands, reps, setup, [] { return 0; },
+      [&](const TuneCand&) { return launch_flux_stages(nTiles, dt, TX, TY); }, ms, &best, st);
+  if (rc) {
+    use(TuneCand{0, 0, 0, 0});
+    return rc;
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  g.timing = savedTiming;
-  if (rc || best < 0) {
-    g.tuneTX = g.persist = g.itemOrder = g.tuneOcc = 0;
-    if (st) st->code = rc ? rc : 3;
-    return rc ? rc : 3;
-  }
-  g.tuneTX = cands[best].tx;
-  g.persist = cands[best].persist;
-  g.itemOrder = cands[best].order;
-  g.tuneOcc = cands[best].occ;
-  int TX = 8;
+  use(cands[best]);
+  TX = 8;
   if (g.multi) {
     multi_march_shape(&TX);
     if (build_march_items(nTiles, TX, st)) return 4;
@@ -2295,15 +2331,56 @@ int tune_flux_stages(int nTiles, double dt, int reps, fx_tune_result* out, int c
     TX = cands[best].tx;
   }
   if (chosenTX) *chosenTX = TX;
-  int k = 0;
-  for (size_t c = 0; c < cands.size(); ++c) {
-    if (ms[c] < 0.f) continue;
-    if (out && k < cap)
-      out[k] = fx_tune_result{cands[c].tx, cands[c].persist, cands[c].order, cands[c].occ,
-                              (int)c == best, ms[c]};
-    ++k;
+  tune_report(cands, ms, best, out, cap, n);
+  return finish(st);
+}
+
+// Column-tile width of the batch step with the update in the march.  The step
+// writes its blocks, so it runs on a copy of them, renewed before each run; of
+// fewer blocks where memory does not hold one of all.
+int tune_fused_step(const double* U, long nBlocks, long blockStride, const double del[3], double dt,
+                    int reps, fx_tune_result* out, int cap, int* n, fx_status* st) {
+  const DevParams& P = g.dp;
+  std::vector<TuneCand> cands;
+  if (P.nxb % 16 == 0 && P.nyb % 8 == 0) cands.push_back(TuneCand{16, 0, 0, 0});
+  cands.push_back(TuneCand{8, 0, 0, 0});
+  double* copy = nullptr;
+  size_t bytes = 0;
+  for (;; nBlocks = (nBlocks + 1) / 2) {
+    bytes = sizeof(double) * ((size_t)(nBlocks - 1) * (size_t)blockStride +
+                              (size_t)P.ncell * (size_t)P.nunk);
+    if (hipMalloc((void**)&copy, bytes) == hipSuccess) break;
+    (void)hipGetLastError();
+    if (nBlocks == 1) {
+      if (st) st->code = 4;
+      return 4;
+    }
   }
-  if (n) *n = k;
+  int rc = batch_fused(P, nBlocks) ? prepare_batch(copy, nBlocks, blockStride, del, st) : 3;
+  const int savedAsync = g.async;
+  int best = -1;
+  std::vector<float> ms;
+  if (!rc) {
+    g.async = 1;
+    rc = time_candidates(
+        cands, reps,
+        [&](const TuneCand& c, bool*) {
+          g.tuneFusedTX = c.tx;
+          return 0;
+        },
+        [&] {
+          return hipMemcpyAsync(copy, U, bytes, hipMemcpyDeviceToDevice, g.stream) == hipSuccess
+                     ? 0 : 4;
+        },
+        [&](const TuneCand&) { return run_compute(nullptr, (int)nBlocks, dt, nullptr, nullptr, true); },
+        ms, &best, st);
+    g.async = savedAsync;
+  }
+  g.tuneFusedTX = rc ? 0 : cands[best].tx;
+  g.batchValid = false;  // the tile list names the copy
+  (void)hipFree(copy);
+  if (rc) return rc;
+  tune_report(cands, ms, best, out, cap, n);
   return finish(st);
 }
 
@@ -2554,7 +2631,7 @@ int fx_hydro_advance_batch_noalloc(double* U, long nBlocks, long blockStride,
   if (nBlocks == 0) return 0;
   const DevParams& P = g.dp;
   int TX = 0, TY = 0, NT = 0;
-  if (P.riemann == FX_EXACT || !march_shape(P, &TX, &TY, &NT)) {
+  if (P.riemann == FX_EXACT || !batch_shape(P, nBlocks, &TX, &TY, &NT)) {
     fprintf(stderr, "fx_hydro_advance_batch_noalloc: takes the HLLC, HLL and hybrid solvers on "
                     "2-D/3-D blocks with x and y extents multiples of 8\n");
     if (st) st->code = 3;
@@ -3142,7 +3219,7 @@ int fx_amr_setup(const fx_tile* tiles, const fx_amr_block* blocks, int nBlocks, 
     A.TY = 8;
   } else {
     int NT = 0;
-    if (!march_shape(g.cur, &A.TX, &A.TY, &NT)) return bad();
+    if (!march_shape(g.cur, &A.TX, &A.TY, &NT, g.tuneTX)) return bad();
   }
   if (g.multi && build_march_items(nBlocks, A.TX, st)) return 4;
   if (ensure_step_scratch(nBlocks, st)) return 4;
@@ -3360,10 +3437,26 @@ int fx_hydro_autotune(const fx_tile* tiles, int nTiles, double dt, int reps, fx_
   const int rc = upload_tiles(tiles, nTiles, true, &st);
   if (rc) return rc;
   int TX = 8, TY = 8, NT = 0;
-  if (g.multi ? !multi_march_shape(&TX) : (g.legacy || !march_shape(g.cur, &TX, &TY, &NT)))
+  if (g.multi ? !multi_march_shape(&TX) : (g.legacy || !march_shape(g.cur, &TX, &TY, &NT, 0)))
     return 3;  // the tuned stages are the column march's
   if (g.cur.learned && !g.seedReady) return 3;
   return tune_flux_stages(nTiles, dt, reps, out, cap, n, nullptr, &st);
+}
+
+int fx_hydro_autotune_batch(double* U, long nBlocks, long blockStride, const double del[3],
+                            double dt, int reps, fx_tune_result* out, int cap, int* n) {
+  fx_status st{};
+  if (n) *n = 0;
+  int TX = 8, TY = 8, NT = 0;
+  if (!g.init || !U || !del || nBlocks <= 0 || nBlocks > 0x7fffffffL || !(dt > 0.) || reps < 1 ||
+      blockStride < g.dp.ncell * g.dp.nunk || g.legacy || !march_shape(g.dp, &TX, &TY, &NT, 0) ||
+      (g.dp.learned && !g.seedReady))
+    return 3;
+  if (batch_fused(g.dp, nBlocks))
+    return tune_fused_step(U, nBlocks, blockStride, del, dt, reps, out, cap, n, &st);
+  const int rc = prepare_batch(U, nBlocks, blockStride, del, &st);
+  if (rc) return rc;
+  return tune_flux_stages((int)nBlocks, dt, reps, out, cap, n, nullptr, &st);
 }
 
 int fx_amr_autotune(double dt, int reps, fx_tune_result* out, int cap, int* n) {
@@ -3380,11 +3473,11 @@ int fx_amr_autotune(double dt, int reps, fx_tune_result* out, int cap, int* n) {
 }
 
 void fx_hydro_autotune_reset(void) {
-  g.tuneTX = g.persist = g.itemOrder = g.tuneOcc = 0;
+  g.tuneTX = g.tuneFusedTX = g.persist = g.itemOrder = g.tuneOcc = 0;
   g.nItems = 0;
   if (g.amr.ready) {  // back to the built-in tile of the grid
     int TX = 8, TY = 8, NT = 0;
-    if (g.multi ? multi_march_shape(&TX) : march_shape(g.cur, &TX, &TY, &NT)) g.amr.TX = TX;
+    if (g.multi ? multi_march_shape(&TX) : march_shape(g.cur, &TX, &TY, &NT, 0)) g.amr.TX = TX;
   }
 }
 

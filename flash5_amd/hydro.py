@@ -136,6 +136,8 @@ EXPORTS = {
     "fx_hydro_set_block_classes": ([C.POINTER(C.c_int), C.c_int], C.c_int),
     "fx_hydro_autotune": ([C.c_void_p, C.c_int, C.c_double, C.c_int, C.c_void_p, C.c_int,
                            C.POINTER(C.c_int)], C.c_int),
+    "fx_hydro_autotune_batch": ([_DP, C.c_long, C.c_long, C.c_double * 3, C.c_double, C.c_int,
+                                 C.c_void_p, C.c_int, C.POINTER(C.c_int)], C.c_int),
     "fx_amr_autotune": ([C.c_double, C.c_int, C.c_void_p, C.c_int, C.POINTER(C.c_int)], C.c_int),
     "fx_hydro_autotune_reset": ([], None),
     "fx_amr_setup": ([C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.POINTER(C.c_int),
@@ -371,9 +373,20 @@ class Hydro:
         return self._tune_list(buf, n.value)
 
     def autotune_batch(self, U, dt: float, deltas: Sequence[float], reps: int = 3):
-        """autotune on a batch tensor (nBlocks, nunk, nz, ny, nx) of blocks."""
-        tiles = [Tile(U=U[b], deltas=deltas) for b in range(U.shape[0])]
-        return self.autotune(tiles, dt, reps)
+        """autotune for advance_batch on a batch tensor (nBlocks, nunk, nz, ny,
+        nx): the whole step where it runs the update inside the march (timed on
+        a copy of the blocks), else the flux stages."""
+        self._reinit()
+        nb = U.shape[0]
+        stride = U.stride(0) if nb > 1 else (U[0].numel() if nb else 0)
+        buf = (FxTuneResult * 32)()
+        n = C.c_int(0)
+        rc = self.lib.fx_hydro_autotune_batch(_ptr(U[0]) if nb else None, nb, stride,
+                                              (C.c_double * 3)(*[float(x) for x in deltas]), dt,
+                                              reps, C.cast(buf, C.c_void_p), 32, C.byref(n))
+        if rc:
+            raise FxError("fx_hydro_autotune_batch", rc=rc)
+        return self._tune_list(buf, n.value)
 
     def amr_autotune(self, dt: float, reps: int = 3):
         buf = (FxTuneResult * 32)()

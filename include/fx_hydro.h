@@ -378,7 +378,15 @@ typedef struct {
 } fx_tune_result;
 int fx_hydro_autotune(const fx_tile* tiles, int nTiles, double dt, int reps, fx_tune_result* out,
                       int cap, int* n);
-/* The same on the multi-level grid of fx_amr_setup. */
+/* The same for fx_hydro_advance_batch (and its no-allocation form) on a batch
+ * of blocks.  Where that step runs the update inside the march (HLLC, HLL and
+ * the hybrid switch), the whole step is timed instead of the flux stages, on a
+ * copy of the blocks (of fewer of them where memory does not hold one), and the
+ * candidates are its column-tile widths; fx_hydro_autotune's choice does not
+ * apply to it. */
+int fx_hydro_autotune_batch(double* U, long nBlocks, long blockStride, const double del[3],
+                            double dt, int reps, fx_tune_result* out, int cap, int* n);
+/* fx_hydro_autotune on the multi-level grid of fx_amr_setup. */
 int fx_amr_autotune(double dt, int reps, fx_tune_result* out, int cap, int* n);
 /* Forget the tuned choice (back to the built-in one). */
 void fx_hydro_autotune_reset(void);
