@@ -103,8 +103,24 @@ def build_lib(verbose: bool = False, jobs: int = 0) -> str:
     return LIB
 
 
+def build_checks(verbose: bool = False) -> str:
+    """Compile tests/cdiv/device_div.hip, the device functions that the test of
+    the FP64 quotients calls by themselves (test infrastructure)."""
+    src = os.path.join(ROOT, "tests", "cdiv", "device_div.hip")
+    out = os.path.join(os.path.dirname(src), "libdevice_div.so")
+    res = subprocess.run([hipcc(), *HIP_FLAGS, "-shared", src, "-o", out + ".tmp"],
+                         capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed:\n{_filter(res.stderr)}")
+    if verbose and _filter(res.stderr).strip():
+        print(_filter(res.stderr), file=sys.stderr)
+    os.replace(out + ".tmp", out)
+    return out
+
+
 def main() -> None:
     print(build_lib(verbose=True))
+    print(build_checks(verbose=True))
 
 
 if __name__ == "__main__":
