@@ -680,10 +680,9 @@ __device__ __forceinline__ bool exact_window(double g, double rl, double pl, dou
   return lo >= 1. / W && hi <= W && fabs(du) <= W && g1 >= 0x1p-10 && g1 <= 0x1p+10;
 }
 
-// what the pressure function and the sampling take from gamma alone, and from
-// one side's state
+// what the pressure function takes from gamma alone, and from one side's state
 struct ExactGas {
-  double g, t1, e1, gr, gp1, rp1;   // 2/(g-1), (g-1)/(2g), (g-1)/(g+1), g+1 and its reciprocal
+  double g, t1, e1, gr, gp1;   // 2/(g-1), (g-1)/(2g), (g-1)/(g+1), g+1
 };
 struct ExactSide {
   double rho, p, c;
@@ -696,10 +695,9 @@ __device__ __forceinline__ ExactGas exact_gas(double g) {
   ExactGas G;
   G.g = g;
   G.gp1 = g + 1.;
-  G.rp1 = O::recip(G.gp1);
   G.t1 = O::div(2., g - 1.);
   G.e1 = O::div(g - 1., 2. * g);
-  G.gr = O::divr(g - 1., G.gp1, G.rp1);
+  G.gr = O::div(g - 1., G.gp1);
   return G;
 }
 template <bool FAST>
@@ -804,7 +802,13 @@ struct ExactStats {
 // tangential velocities and gammas.  The right side is sampled as the left one
 // of the mirrored problem (velocities negated, which is exact), so that
 // wavefronts with faces on either side of the contact run one copy.
-template <bool FAST>
+// FRESH: what a branch takes from gamma it forms again, from a copy that the
+// compiler cannot see through: kept from exact_gas through the iteration, those
+// values took the registers that k_face_solve's three waves per SIMD lack (14
+// spilled of 168 on tiles of several classes: the exact solver's step on a
+// three-level grid of 29.4M zones 27.8 ms instead of 24.7).  k_solve_update, at
+// two waves, has them (1024 x 16^3 2561 us a step, 2569 with FRESH).
+template <bool FAST, bool FRESH>
 __device__ __forceinline__ void exact_sample(const ExactGas& G, const ExactSide& L, double ul,
                                              const ExactSide& Q, double ur, double pm, double um, double& r, double& u,
                                              double& pp, bool& leftside) {
@@ -814,6 +818,8 @@ __device__ __forceinline__ void exact_sample(const ExactGas& G, const ExactSide&
   const double rk = left ? L.rho : Q.rho, pk = left ? L.p : Q.p, ck = left ? L.c : Q.c;
   const double v = left ? ul : -ur, w = left ? um : -um;
   const double pmk = O::div(pm, pk);
+  double g = G.g;
+  if constexpr (FRESH) asm("" : "+v"(g));
   if (left ? pm <= pk : !(pm > pk)) {
     if (0. <= v - ck) {
       r = rk; u = v; pp = pk;
@@ -822,23 +828,25 @@ __device__ __forceinline__ void exact_sample(const ExactGas& G, const ExactSide&
       const double st = w - cm;
       // isentropic: rho = gamma p / c^2 behind the rarefaction
       if (left ? 0. > st : 0. >= st) {
-        r = O::div(G.g * pm, cm * cm); u = w; pp = pm;
+        r = O::div(g * pm, cm * cm); u = w; pp = pm;
       } else {
-        const double c = O::divr(2., G.gp1, G.rp1) * (ck + (G.g - 1.) * 0.5 * v);
+        const double c = O::div(2., g + 1.) * (ck + (g - 1.) * 0.5 * v);
         u = left ? c : -(-c + 0.);   // a zero is +0 on either side
         // in the fan, (c/ck)^(2g/(g-1)) = (c/ck)^(2/(g-1)) (c/ck)^2
         const double x = O::div(c, ck);
-        const double q = pow_pos(x, G.t1), s2 = x * x;
+        const double q = pow_pos(x, O::div(2., g - 1.)), s2 = x * x;
         r = rk * q;
         pp = pk * (q * s2);
       }
     }
   } else {
-    const double sk = v - ck * O::root(O::div(G.gp1, 2. * G.g) * pmk + G.e1);
+    const double gp1 = g + 1.;
+    const double sk = v - ck * O::root(O::div(gp1, 2. * g) * pmk + G.e1);
     if (0. <= sk) {
       r = rk; u = v; pp = pk;
     } else {
-      r = O::div(rk * (pmk + G.gr), O::divr(pmk * (G.g - 1.), G.gp1, G.rp1) + 1.);
+      const double rp1 = O::recip(gp1);
+      r = O::div(rk * (pmk + O::divr(g - 1., gp1, rp1)), O::divr(pmk * (g - 1.), gp1, rp1) + 1.);
       u = w; pp = pm;
     }
   }
@@ -846,7 +854,7 @@ __device__ __forceinline__ void exact_sample(const ExactGas& G, const ExactSide&
 }
 
 // exact_riemann's problem once its states are known to be positive
-template <bool FAST, bool SEEDED>
+template <bool FAST, bool SEEDED, bool FRESH>
 __device__ __forceinline__ int exact_solve(const DevParams& P, double g, double rl, double ul, double pl, double rr, double ur,
                                            double pr, double guess, ExactStats& es, double& r, double& u, double& pp,
                                            bool& left) {
@@ -878,7 +886,7 @@ __device__ __forceinline__ int exact_solve(const DevParams& P, double g, double 
   exact_fk<FAST>(pm, G, L, fl, fld);
   exact_fk<FAST>(pm, G, Q, fr, frd);
   const double um = 0.5 * (ul + ur) + 0.5 * (fr - fl);
-  exact_sample<FAST>(G, L, ul, Q, ur, pm, um, r, u, pp, left);
+  exact_sample<FAST, FRESH>(G, L, ul, Q, ur, pm, um, r, u, pp, left);
   return 0;
 }
 
@@ -889,14 +897,14 @@ __device__ __forceinline__ int exact_solve(const DevParams& P, double g, double 
 // converge restarts from the two-shock guess (counted as fallback).  One
 // Newton loop serves both passes, which keeps a seeded kernel's register
 // budget that of the unseeded one.  SEEDED = false ignores guess.
-template <bool SEEDED>
+template <bool SEEDED, bool FRESH>
 __device__ __forceinline__ int exact_riemann(const DevParams& P, double g, double rl, double ul, double pl, double rr, double ur,
                                              double pr, double guess, ExactStats& es, double& r, double& u,
                                              double& pp, bool& left) {
   if (!(rl > 0. && rr > 0. && pl > 0. && pr > 0.)) return 1;
   if (__builtin_expect(__all(exact_window(g, rl, pl, rr, pr, ur - ul)), 1))
-    return exact_solve<true, SEEDED>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
-  return exact_solve<false, SEEDED>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+    return exact_solve<true, SEEDED, FRESH>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+  return exact_solve<false, SEEDED, FRESH>(P, g, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
 }
 
 // ---- the FP32 solver (mixed-precision mode): the pressure function, sampling
@@ -1092,8 +1100,8 @@ __device__ __forceinline__ void prim2flx_dir(int d, R r, R vx, R vy, R vz, R p, 
 // them with the run-time offset d keeps them out of private arrays, and one
 // copy of the solver serves all directions.  gamc is the left cell's, game
 // the cells' on either side.  The states and the solve are in R; F is FP64
-// for the update.  Returns exact_riemann's codes.
-template <bool SEEDED, typename R>
+// for the update.  FRESH as in exact_sample.  Returns exact_riemann's codes.
+template <bool SEEDED, typename R, bool FRESH = true>
 __device__ __forceinline__ int exact_face_flux(const DevParams& P, int d, const R* Lb,
                                                const R* Rb, long s, double gamc,
                                                double gameL, double gameR, double guess,
@@ -1104,7 +1112,7 @@ __device__ __forceinline__ int exact_face_flux(const DevParams& P, int d, const 
   bool left;
   int e;
   if constexpr (sizeof(R) == sizeof(double))
-    e = exact_riemann<SEEDED>(P, gamc, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
+    e = exact_riemann<SEEDED, FRESH>(P, gamc, rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
   else
     e = exact_riemann_f32<SEEDED>(P, float(gamc), rl, ul, pl, rr, ur, pr, guess, es, r, u, pp, left);
   if (e) return e;

@@ -373,8 +373,8 @@ __device__ __forceinline__ FaceRef face_ref(const DevParams& P, int t, long rt) 
 // the flux component that takes the pressure are picked at run time.  R is
 // the solver's arithmetic: double, or float in the mixed-precision mode
 // (FP64 Newton iterate and convergence test, FP64 fluxes out).
-// (3 waves per SIMD fit the FP64 solver's registers without spilling, 4 the
-// FP32 one's)
+// (3 waves per SIMD fit the FP64 solver's registers, 2 spilled on tiles of
+// several classes, 4 the FP32 one's)
 template <bool SEEDED, bool MULTI, typename R>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(sizeof(R) == sizeof(float) ? 4 : 3)))
@@ -585,9 +585,9 @@ k_solve_update(DevParams P, FaceLaunch F, double dt0, const double* dtp, const R
       const R* Lb = b + r;
       const R* Rb = b + 6 * nf + r;
       double Fo[8];
-      const int ierr = exact_face_flux<false, R>(P, d, Lb, Rb, nf, U[P.voff[FX_GAMC] + cL],
-                                                 U[P.voff[FX_GAME] + cL], U[P.voff[FX_GAME] + cR],
-                                                 -1.0, Fo, es);
+      const int ierr = exact_face_flux<false, R, false>(
+          P, d, Lb, Rb, nf, U[P.voff[FX_GAMC] + cL], U[P.voff[FX_GAME] + cL],
+          U[P.voff[FX_GAME] + cR], -1.0, Fo, es);
       if (ierr) report_error(F.status, 2, t, i, j, kf, d);
 #pragma unroll
       for (int q = 0; q < 8; ++q) flx[q * kSolveMaxFaces + slot] = ierr ? R(0.) : R(Fo[q]);
