@@ -26,10 +26,11 @@ void launch_march_f(const DevParams& P, const MarchLaunch& M, int TX, dim3 grid,
     }
   }
   constexpr int NT3 = sizeof(R) == 8 ? 768 : 512;  // FP64 3-D 16x8: 768 threads
-  // FP64 2-D 16x8: 448 threads, since stage A has seven wavefronts of items
-  // (4096 x 16^2 293 -> 270 us; two workgroups a CU either way).  FP32 runs
-  // four workgroups of 384 on a CU instead.
-  constexpr int NT2 = sizeof(R) == 8 ? 448 : 384;
+  // 2-D 16x8: 448 threads, since stage A has seven wavefronts of items and the
+  // state cells only six.  With 384 one wavefront took a second item: 4096 x
+  // 16^2 FP64 293 against 270 us; 16000 x 16^2 FP32 HLLC 617 against 556, to face
+  // states 563 against 520, 20000 tiles of two classes 915 against 815.
+  constexpr int NT2 = 448;
   if (P.ndim == 3 && TX == 16) hipLaunchKernelGGL((k_march<3, 16, 8, NT3, RS, R, OCC, FUSE>), grid, dim3(NT3), 0, H.stream, P, M);
   else if (P.ndim == 3) hipLaunchKernelGGL((k_march<3, 8, 8, 384, RS, R, OCC, FUSE>), grid, dim3(384), 0, H.stream, P, M);
   else if (TX == 16) hipLaunchKernelGGL((k_march<2, 16, 8, NT2, RS, R, OCC, FUSE>), grid, dim3(NT2), 0, H.stream, P, M);
@@ -124,7 +125,7 @@ void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHos
       }
     }
     if (ndim == 3) launch_march_mixw_k<3, 512, RS, R>(M, H);
-    else launch_march_mixw_k<2, 384, RS, R, OCC>(M, H);
+    else launch_march_mixw_k<2, 448, RS, R, OCC>(M, H);
     return;
   }
   if constexpr (sizeof(R) == 4) {  // FP32 3-D: the autotuner may ask for 4 waves per SIMD
@@ -142,7 +143,7 @@ void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHos
   }
   if (ndim == 3 && TX == 16) launch_march_multi_k<3, 16, 8, 512, RS, R>(M, H);
   else if (ndim == 3) launch_march_multi_k<3, 8, 8, 384, RS, R, OCC>(M, H);
-  else if (TX == 16) launch_march_multi_k<2, 16, 8, 384, RS, R, OCC>(M, H);
+  else if (TX == 16) launch_march_multi_k<2, 16, 8, 448, RS, R, OCC>(M, H);
   else launch_march_multi_k<2, 8, 8, 256, RS, R, OCC>(M, H);
 }
 
