@@ -1047,6 +1047,7 @@ struct Lib {
   std::vector<DevParams> hcls;
   DevParams* dcls = nullptr;
   size_t dclsCap = 0;
+  bool clsSent = false;                // dcls holds hcls
   // the uploaded tile list: one shape (cur) or several classes (multi)
   DevParams cur{};
   bool multi = false;
@@ -3064,12 +3065,15 @@ int fx_hydro_set_block_classes(const int* nb, int nClasses) {
   }
   // what is on the device already (every entry point sets its classes again)
   // stays there
-  if (nClasses > 0 && (cls.size() != g.hcls.size() ||
+  if (nClasses > 0 && (!g.clsSent || cls.size() != g.hcls.size() ||
                        memcmp(cls.data(), g.hcls.data(), sizeof(DevParams) * nClasses) != 0)) {
-    if (grow(&g.dcls, &g.dclsCap, (size_t)nClasses, nullptr)) return 4;
+    // room for the most there can be, so that no table that hcls names is freed
+    if (grow(&g.dcls, &g.dclsCap, FX_MAX_CLASSES, nullptr)) return 4;
+    g.clsSent = false;
     if (hipMemcpy(g.dcls, cls.data(), sizeof(DevParams) * nClasses, hipMemcpyHostToDevice) !=
         hipSuccess)
       return 4;
+    g.clsSent = true;
   }
   bool same = cls.size() == g.hcls.size();
   for (size_t c = 0; same && c < cls.size(); ++c)
