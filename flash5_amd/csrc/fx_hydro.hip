@@ -1416,8 +1416,6 @@ double fallback_cfl_cap(const fx_params& p) {
 // a CFL lowered by the step's flags or fallbacks
 bool cfl_varies(const fx_params& p) { return p.shockLowerCFL || fallback_cfl_cap(p) > 0.0; }
 
-// Synchronise and copy the device status record ds into st (nothing in
-// async mode, where the call returns before its kernels end).
 // The library's pinned buffer, of at least bytes.  A device-to-host copy into it
 // queues behind the kernels, so that a call waits once, for both.
 int pinned(size_t bytes, fx_status* st) {
@@ -1430,6 +1428,8 @@ int pinned(size_t bytes, fx_status* st) {
   return 0;
 }
 
+// Synchronise and copy the device status record ds into st (nothing in
+// async mode, where the call returns before its kernels end).
 int finish_from(const DevStatus* ds, fx_status* st) {
   if (g.async) return 0;
   if (pinned(sizeof(DevStatus), st)) return 4;
