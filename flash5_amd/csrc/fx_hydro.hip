@@ -1231,11 +1231,15 @@ DevParams make_dev_params(const fx_params& p) {
   return d;
 }
 
+// Whether the march can address a block's array: by 32-bit byte offsets within
+// one buffer resource (TileView), whose range ends at 2 GiB.
+bool march_addresses(const DevParams& P) { return P.ncell * P.nunk <= 0x7fffffffL / 8; }
+
 // Column-tile shape of the fused kernel for this block shape, or false
-// when only the three-kernel path applies (1-D, or sizes not tileable).
-// tuned: the autotuned width, 0 for the built-in one
+// when only the three-kernel path applies (1-D, sizes not tileable, or blocks
+// past march_addresses).  tuned: the autotuned width, 0 for the built-in one
 bool march_shape(const DevParams& P, int* TX, int* TY, int* NT, int tuned) {
-  if (P.ndim < 2) return false;
+  if (P.ndim < 2 || !march_addresses(P)) return false;
   const int nx = P.nxb, ny = P.nyb;
   if (nx % 16 == 0 && ny % 8 == 0 && tuned != 8) {
     *TX = 16;
@@ -1251,11 +1255,9 @@ bool march_shape(const DevParams& P, int* TX, int* TY, int* NT, int tuned) {
 }
 
 // Column tiles of a block that no fixed tile divides: the fewest equal ones
-// that fit the 16x8 layout, the last along an axis with what is left.  The
-// march addresses a block's array by 32-bit byte offsets, so larger blocks
-// keep the three-kernel path.
+// that fit the 16x8 layout, the last along an axis with what is left.
 bool free_shape(const DevParams& P, int* tx, int* ty) {
-  if (P.ndim < 2 || P.ncell * P.nunk > 0x7fffffffL / 8) return false;
+  if (P.ndim < 2 || !march_addresses(P)) return false;
   if (g.freeOf[0] != P.nxb || g.freeOf[1] != P.nyb) {
     int best = 1 << 30;
     for (int x = 1; x <= P.nxb && free_tile_fits<16, 8>(x, 1); ++x)
@@ -3062,6 +3064,7 @@ int fx_hydro_set_block_classes(const int* nb, int nClasses) {
     if (validate(&p)) return 3;
     if (p.ndim < 2 || p.nxb % 8 || p.nyb % 8) return 3;  // the column march's tiles
     cls.push_back(make_dev_params(p));
+    if (!march_addresses(cls.back())) return 3;
   }
   // what is on the device already (every entry point sets its classes again)
   // stays there

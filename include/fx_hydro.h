@@ -343,7 +343,8 @@ void fx_hydro_set_kernel_path(int path);
  * and the flux-register calls read each tile's shape from
  * fx_tile.block_class; tiles of several classes go through one persistent
  * launch per stage.  The shapes must admit the fused column-march kernel
- * (interior x and y extents multiples of 8, 2-D or 3-D).  nClasses = 0
+ * (interior x and y extents multiples of 8, 2-D or 3-D, a block's array below
+ * 2 GiB).  nClasses = 0
  * returns to the fx_hydro_init shape.  The batch entry points
  * (fx_hydro_advance_batch, fx_grid_*) keep the fx_hydro_init shape.
  * fx_hydro_init with different knobs clears the classes. 
