@@ -85,12 +85,19 @@ using Eig = EigT<double>;
 // residual correction q + (x - y q) r in two FMAs.  They hold while the
 // divisor, the quotient and the residual x - y q are normal: |x| at least
 // 2^-960 (below, the quotient may differ in its last place), |x| and |y| below
-// 2^1000 and y not 0 (there: NaN), and a zero quotient is +0.  Callers either
-// check their operands (in_window) and divide plainly outside, or discard the
-// result there.  tests/cdiv/fast_div_check.c runs the same steps against IEEE
-// division and root.  The march and the 2-D/3-D steps are bound by instruction
-// issue: 4096 x 16^3 FP64 HLLC step 6.02 -> 5.72 ms, 1024^2 in 64^2 blocks 492 ->
-// 475 us a step, 1024 x 16^3 exact 3.15 -> 2.96 ms, the same bits.
+// 2^1000 and y normal (else: NaN), and a zero quotient is +0.  The eigen
+// systems and the exact solver check their operands (window_pos,
+// exact_window) and divide plainly outside, HLLC its divisor; the van Leer
+// limiter and the flattening check nothing, and drop the result where the
+// divisor is zero.  So what differs from plain division is the last place of
+// slopes of differences, or of star-state momenta, below about 2^-480 and
+// 2^-960.  For a divisor of all-ones significand the hardware's estimate has
+// to lie above 1/y, and gfx950's does.  tests/test_gpu_fast_division.py runs
+// these functions against IEEE division and root,
+// tests/cdiv/fast_div_check.c their steps from other starts.  The march and the
+// 2-D/3-D steps are bound by instruction issue: 4096 x 16^3 FP64 HLLC step 6.02 ->
+// 5.72 ms, 1024^2 in 64^2 blocks 492 -> 475 us a step, 1024 x 16^3 exact 3.15 ->
+// 2.96 ms, the same bits.
 __device__ __forceinline__ double recip_fast(double y) {
   const double r0 = __builtin_amdgcn_rcp(y);
   const double e = fma(-y, r0, 1.0);
@@ -125,8 +132,9 @@ __device__ __forceinline__ unsigned window_pos(double x) {
 }
 
 // x / y as the compiler divides in FP32 at the accuracy the FP32 code is
-// built for (a reciprocal and a product, y scaled down where the reciprocal
-// would be flushed), spelled out: where code merges two branches' divisions
+// built for (LLVM's AMDGPU lowering of fdiv with 2.5 ulp allowed: a reciprocal
+// and a product, y scaled down by 2^-32 above 2^96, where the reciprocal would
+// be flushed), spelled out: where code merges two branches' divisions
 // into one, the compiler drops that accuracy setting and emits the correctly
 // rounded sequence, with other bits.
 __device__ __forceinline__ float quot(float x, float y) {

@@ -1303,10 +1303,10 @@ ZSplit z_split(const DevParams& P, long columnTiles, long slots) {
 // for solve and update.  That takes the time of a block's rounds one after the
 // other however few the blocks; the face solve and the update as kernels of
 // their own take a time in proportion to the faces, up to about 30000 of them
-// (16000 in FP32) in the time of a round.  One / separate, the whole step:
-// 16^3 FP64 1 block 383 / 88 us, 100 556 / 509, 128 576 / 602, 512 1341 / 1783;
-// mixed 64 308 / 288, 100 350 / 420; 8^3 FP64 128 184 / 169, 256 223 / 246;
-// mixed 64 101 / 97, 128 113 / 126; 16 x 16 x 32 FP64 128 1190 / 1143.
+// (16000 in FP32) in the time of a round.  One / separate, the step's kernels:
+// 16^3 FP64 1 block 364 / 75 us, 100 521 / 496, 128 554 / 590, 512 1336 / 1790;
+// mixed 64 282 / 276, 100 326 / 418; 8^3 FP64 128 160 / 151, 192 194 / 201;
+// mixed 64 89 / 81, 128 98 / 109; 16 x 16 x 32 FP64 128 1130 / 1123.
 bool solve_update_pays(const DevParams& P, long n) {
   const long faces = n * (P.nface[0] + P.nface[1] + P.nface[2]);
   return faces > (P.precision == FX_PREC_MIXED ? 16000L : 30000L) *
@@ -1352,15 +1352,16 @@ bool batch_shape(const DevParams& P, long n, int* TX, int* TY, int* NT) {
 }
 
 // Where the update of n such blocks runs.  kFuseDirect gives a block's column
-// tiles to one workgroup in turn and saves k_update_finish: 6.10 against
-// 5.81 + 1.09 ms on 4096 x 16^3 (FP64), 2.08 against 1.85 + 0.51 on 2048 x
-// 16^3 (mixed), 6.58 against 6.32 + 0.58 on 16384 x 8^3.  It takes blocks one
+// tiles to one workgroup in turn and saves k_update_finish: 5.73 against
+// 5.57 + 1.09 ms on 4096 x 16^3 (FP64), 2.02 against 1.83 + 0.51 on 2048 x
+// 16^3 (mixed), 5.77 against 5.58 + 0.59 on 16384 x 8^3.  It takes blocks one
 // column tile wide, no contact steepening (which reads planes that the update
 // has written by then), and a batch that fills the workgroups resident at a
 // time: whole blocks come in fewer, longer rounds than column tiles do, and
 // k_update_finish costs about an eighth of the march.  In 2-D the tiles are
-// short, and taking two in turn costs more than k_update_finish (4096 x 16^2
-// mixed: 190 against 152 + 25 us): blocks of one tile only.
+// short, and taking two in turn costs as much as k_update_finish or more (4096 x
+// 16^2 FP64 251 against 228 + 28 us, mixed 185 against 141 + 28): blocks of one
+// tile only.
 int batch_fuse_mode(const DevParams& P, int TX, int TY, long n) {
   if (!batch_fused(P, n)) return kFuseNone;
   const long tiles = P.nyb / TY;

@@ -686,11 +686,10 @@ __global__ void k_zero_count(unsigned* c) { c[threadIdx.x] = 0u; }
 // The learned seed's gate over every face of the launch, from the face
 // states the march stored: a face at or above the gate (seed_gate_pass, in
 // FP64 from the stored values) joins the strong list (one atomic per
-// wavefront, ranks by ballot) for k_face_seed.  With y, every face's seed
-// slot also becomes "no seed" first (k_face_seed then fills the listed
-// ones), which the face stage that reads a seed per face needs.  The batch
-// step's list-driven solve does not: there the march lists the strong faces
-// itself (list_strong_face), since this pass over the states took 251 us of
+// wavefront, ranks by ballot) for k_face_seed, and every face's seed slot in
+// y becomes "no seed" (k_face_seed then fills the listed ones) for the face
+// stage, which reads a seed per face.  The batch step's list-driven solve has
+// no such slots: there the march lists the strong faces itself (list_strong_face), since this pass over the states took 251 us of
 // 3117 on 2048 x 16^3 mixed, and the list adds 69 us to the march (the step
 // 3117 -> 3040 us).
 template <bool MULTI, typename S>
@@ -712,7 +711,7 @@ __global__ void __launch_bounds__(kThreads) k_face_gate(DevParams P0, FaceLaunch
     const long nf = P.nface[d];
     const double rl = b[r], ul = b[(1 + d) * nf + r], pl = b[4 * nf + r];
     const double rr = b[6 * nf + r], ur = b[(7 + d) * nf + r], pr = b[10 * nf + r];
-    if (y) y[gid] = kNoSeed;
+    y[gid] = kNoSeed;
     return rl > 0. && rr > 0. && pl > 0. && pr > 0. &&
            seed_gate_pass(G, P.gamma, rl, ul, pl, rr, ur, pr);
   };

@@ -322,11 +322,10 @@ __device__ __forceinline__ T ld_at(const __attribute__((address_space(1))) T* ba
 
 // The tile's primitives are read as one buffer (a scalar resource) with the
 // variable's byte offset in a scalar operand and the cell's in a vector
-// one, so no 64-bit address is formed per lane.  With 64-bit addresses the
-// compiler kept several per stencil point live across the item loops: the
-// FP32 march at 4 waves per SIMD spilled 36 registers instead of 21, and
-// the 8-wide march tiles ran at 7.6 instead of 10.1 ms (FP32) and 11.6
-// instead of 20.1 ms (FP64) on 4096 x 16^3.
+// one, so no 64-bit address is formed per lane.  With 64-bit addresses several
+// per stencil point stay live across the item loops: the FP32 march takes 161
+// registers instead of 114, which leaves one workgroup on a CU for two (4096 x
+// 16^3 mixed 5.83 against 4.05 ms a step), the FP64 one 5.97 against 5.80 ms.
 struct TileView {
   __amdgpu_buffer_rsrc_t rs;  // the tile's guard-inclusive array
   unsigned ob[8];             // byte offsets of the primitive slots P_DENS .. P_EINT
@@ -373,9 +372,11 @@ __device__ __forceinline__ void tv_st(const TileView& tv, unsigned ob, unsigned 
 // A stage's item number.  With OPAQUE it passes through an empty asm
 // statement, which the compiler cannot see through: the index arithmetic of
 // each stage's items (item kind, column, cell offsets) is then redone per
-// plane instead of being hoisted out of the plane loop and kept live.  With
-// the hoisted form the FP32 16x8 march took 160 registers instead of 104 and
-// the FP64 multi-class kernels 256 with 51 spilled instead of 195.
+// plane instead of being hoisted out of the plane loop and kept live.  Hoisted,
+// the FP64 16x8 march spills 106 registers instead of 10 (4096 x 16^3 7.70
+// against 5.80 ms a step) and the FP32 one takes 167 instead of 114 (5.57
+// against 4.05); the FP64 march over several classes spills 55 instead of none
+// (29.4M zones 12.5 against 11.5 ms).
 template <bool OPAQUE>
 __device__ __forceinline__ int item_index(int w) {
   if constexpr (OPAQUE) asm volatile("" : "+v"(w));
@@ -441,10 +442,20 @@ __device__ __forceinline__ void write_flux_b(const DevParams& P, gdouble* Fo, un
   for (int q = 0; q < FX_NFLUX; ++q) st_at(Fo + q * nf, rb, F[q]);
 }
 
-// The march's barrier: a workgroup's threads exchange data through LDS alone
-// (the block's cells are only read, its outputs only written), so the LDS
-// accesses are waited for and the global ones stay in flight.  The plain
-// barrier also waits for every store to reach the cache, once per stage.
+// The march's barrier: a workgroup's threads exchange data through LDS alone,
+// so the LDS accesses are waited for and the global ones stay in flight.  The
+// plain barrier also waits for every store to reach the cache, once per stage.
+// What makes that safe where the update runs inside the march (stage D):
+// - kFuseDirect stores a block's cells while other wavefronts load from it.
+//   Beside stage B of plane k it stores plane k - 2 (in 2-D the one plane, after
+//   the last stage), and no load still to come or in flight is below plane
+//   k - 1: stage B and the z slopes of k + 1 reach down to k - 1, stage C(k) to
+//   k - 1.  Contact steepening reads two planes down and takes kFuseScratch.
+// - The neighbouring column tile's rows within a stencil's reach (kSeamRows) are
+//   kept back until that tile is done (march_block).
+// - Scratch that is read back during the march (FP32's carried cells) is read by
+//   the thread that stored it; the seam rows, read by others, lie behind the full
+//   barrier that ends a column tile.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
@@ -1164,10 +1175,11 @@ __device__ __forceinline__ MarchPlace march_place(const DevParams& P, const Marc
 // segment forms the states and sigmas of the planes next to it anew: three
 // planes' work).  OCC > 0
 // asks the compiler for OCC waves per SIMD (fewer registers, maybe spills);
-// the autotuner decides whether that pays.  The FP64 16x8 tile runs 768
-// threads: its LDS allows one workgroup per CU, stage A has 12 wavefronts of
-// items, and 3 waves per SIMD leave 168 registers (at 512 threads the march
-// took 8.83 instead of 8.41 ms on 4096 x 16^3).
+// without the update the autotuner decides whether that pays in FP32.  The FP64
+// 16x8 tile runs 768 threads: its LDS allows one workgroup per CU, stage A has
+// 12 wavefronts of items, and 3 waves per SIMD leave 168 registers, of which
+// the form with the update in place spills 10 (at 512 threads and 176 registers
+// the step of 4096 x 16^3 takes 6.40 instead of 5.80 ms).
 template <int NDIM, int TX, int TY, int NT, int RS, typename R, int OCC = 0, int FUSE = kFuseNone>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 k_march(DevParams P, MarchLaunch L) {

@@ -118,8 +118,8 @@ void launch_march_multi_r(int ndim, int TX, const MarchLaunch& M, const MarchHos
         return;
       }
     }
-    if constexpr (sizeof(R) == 8) {  // FP64: 768 threads, as k_march (quadrant grid
-      if (ndim == 3) {               // march 15.4 -> 14.8 ms, though 26 registers spill)
+    if constexpr (sizeof(R) == 8) {  // FP64: 768 threads, as k_march (29.4M zones of three
+      if (ndim == 3) {               // classes 11.5 ms, 11.9 at 512)
         launch_march_mixw_k<3, 768, RS, R, 3>(M, H);
         return;
       }

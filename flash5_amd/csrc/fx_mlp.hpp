@@ -31,7 +31,6 @@ constexpr int OFF_B3 = OFF_W3 + MLP_H;             // b3
 constexpr int MLP_NPARAM = OFF_B3 + 1;             // 4673
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) unsigned short u16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 // round to nearest even (v_cvt_pk_bf16_f32)

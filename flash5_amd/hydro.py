@@ -453,9 +453,9 @@ class Hydro:
         return t.value
 
     def set_kernel_path(self, path: int) -> None:
-        """0 = fused column-march kernel (default; exact-solver batch steps of
-        3-D blocks up to 16 x 16 across solve and update in one kernel),
-        1 = three-kernel path, 2 = as 0 with the update always separate."""
+        """0 = column march (default; batch steps update inside it, or with
+        the exact solver solve and update in one kernel), 1 = three-kernel
+        path, 2 = as 0 with the update always a kernel of its own."""
         self.lib.fx_hydro_set_kernel_path(int(path))
 
     def set_timing(self, on: bool) -> None:

@@ -324,14 +324,19 @@ void fx_hydro_set_stream(void* stream);
 void fx_hydro_set_async(int async_);
 /* Per-stage timing: when on, each compute call records HIP events on the
  * library's stream around its kernels; fx_hydro_stage_times copies the last
- * call's durations in ms (states, fluxes, update) and returns the count. */
+ * call's durations in ms (states, fluxes, update) and returns the count.  The
+ * column march counts as states, with the fluxes of all solvers but the exact
+ * one, and with the update where it runs inside the march. */
 void fx_hydro_set_timing(int on);
 int fx_hydro_stage_times(float* ms, int n);
-/* Kernel path: 0 = fused column-march kernel where the block shape allows
- * (default; batch steps of 3-D blocks up to 16 x 16 across with the exact
- * solver also run its face solve and the conservative update as one
- * kernel), 1 = three-kernel path (states, fluxes, update), 2 = as 0 but the
- * exact solver's batch steps keep the update as a kernel of its own. */
+/* Kernel path: 0 = column march where the block shape allows (default).  Batch
+ * steps (fx_hydro_advance_batch, fx_grid_run_graph) with HLLC, HLL or the hybrid
+ * switch run the update inside it, on blocks whose x and y extents are no
+ * multiples of 8 in FP64; large batches of 3-D blocks up to 16 x 16 across with
+ * the exact solver run its face solve and the update as one kernel.
+ * 1 = three-kernel path (states, fluxes, update).  2 = as 0 with the update
+ * always a kernel of its own, and the three kernels for extents that are no
+ * multiples of 8. */
 void fx_hydro_set_kernel_path(int path);
 
 /* Block classes: tiles of several interior shapes in one call, e.g. levels
